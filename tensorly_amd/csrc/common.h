@@ -150,6 +150,10 @@ int mttkrp_launch(int x_dtype, const void* X, int ndim, const int64_t* shape, co
                   const void* weights, int rank, int kb, int ke, int precision, void* out, void* ws, size_t ws_bytes,
                   const InvJob* job, bool* job_taken, hipStream_t st);
 
+// Scratch below which tla_mttkrp refuses the call (its
+// tla_mttkrp_workspace_size, or 0 where it runs without as well).
+size_t mttkrp_min_workspace(int x_dtype, int ndim, const int64_t* shape, int rank, int mode, int precision);
+
 struct ModeShape {
   int ndim;
   int64_t shape[kMaxOrder];

@@ -21,7 +21,11 @@
 //    per wave), and MFMA number t uses column k0 + 4c + t -- a permutation
 //    of the output columns undone when the tile is written.
 //
-//  * mttkrp_generic  plain vector-ALU fallback for any shape / rank / dtype.
+//  * mttkrp_any_*    (mttkrp_any.hip) shapes that are not aligned, ranks above
+//    64 and float64, on the FP32 / FP64 matrix instructions.
+//
+//  * mttkrp_generic  plain vector ALU: precision "valu", sizes past the index
+//    ranges of mttkrp_any, and callers that bring no scratch.
 //
 // Precisions: FP32 (v_mfma_f32_16x16x4_f32), BF16 (v_mfma_f32_16x16x32_bf16:
 // the tensor RNE-rounded to bf16, or a bf16 copy of it, times the factor
@@ -38,6 +42,7 @@
 
 #include "common.h"
 #include "inverse.h"
+#include "mttkrp_any.h"
 
 namespace tla {
 
@@ -1295,11 +1300,12 @@ __global__ void build_gm_kernel(GmArgs args, float* __restrict__ gm) {
 // ---------------------------------------------------------------------------
 // Host planning
 // ---------------------------------------------------------------------------
-enum class Path { Generic, Inner, Tiles, Last, Stream, LastStream };
+enum class Path { Generic, Any, Inner, Tiles, Last, Stream, LastStream };
 
 struct Plan {
   Path path;
   int RT;
+  AnyPlan any;
   // stream
   StreamArgs st;
   int sepi;
@@ -1360,6 +1366,21 @@ static int make_plan(int x_dtype, int ndim, const int64_t* shape, int R, int kb,
     return TLA_OK;
   };
   const bool mfma = prec_ok(x_dtype, precision) && R <= 64;
+  // Shapes the aligned kernels below do not take, ranks above 64 and
+  // float64: the matrix-core kernels for any shape (float32 arithmetic in
+  // float32, whatever the precision asks for).  The vector kernel is left
+  // for precision "valu" and for sizes past those kernels' index ranges.
+  auto unaligned = [&]() -> int {
+    p->path = Path::Generic;
+    p->ws_bytes = 0;
+    if ((x_dtype == TLA_F64 || prec_ok(x_dtype, precision)) &&
+        any_plan(x_dtype == TLA_F64, ndim, shape, R, kb, true, &p->any)) {
+      p->path = Path::Any;
+      p->out_rows = shape[kb];
+      p->ws_bytes = p->any.ws_bytes;
+    }
+    return TLA_OK;
+  };
   const int RT = (R + 15) / 16;
   p->RT = RT;
   const int64_t K = shape[ndim - 1];
@@ -1375,9 +1396,7 @@ static int make_plan(int x_dtype, int ndim, const int64_t* shape, int R, int kb,
     if (!(mfma && K % 32 == 0)) {
       TLA_REQUIRE(standard, "partial contraction needs an MFMA-eligible shape");
       TLA_REQUIRE(x_dtype != TLA_BF16, "bf16 tensor copy needs K %% 32 == 0 and R <= 64");
-      p->path = Path::Generic;
-      p->ws_bytes = 0;
-      return TLA_OK;
+      return unaligned();
     }
     // Row-tile kernel when mode N-2 is contracted (rows reduce into the
     // output) or when every non-contiguous mode is kept (rows are the output).
@@ -1541,9 +1560,7 @@ static int make_plan(int x_dtype, int ndim, const int64_t* shape, int R, int kb,
   if (!(mfma && shape_ok)) {
     TLA_REQUIRE(standard, "partial contraction needs an MFMA-eligible shape");
     TLA_REQUIRE(x_dtype != TLA_BF16, "bf16 tensor copy needs an MFMA-eligible shape");
-    p->path = Path::Generic;
-    p->ws_bytes = 0;
-    return TLA_OK;
+    return unaligned();
   }
   GmArgs& gm = p->gm;
   gm.n = kb - 1;
@@ -1783,7 +1800,12 @@ static int run_plan(const Plan& p0, int x_dtype, const void* X, int ndim, const 
     p.grid.x += 1;
     if (job_taken) *job_taken = true;
   }
-  if (p.path == Path::Generic) {
+  if (p.path == Path::Any && ws_bytes >= p.ws_bytes && (ws || p.ws_bytes == 0)) {
+    any_plan(x_dtype == TLA_F64, ndim, shape, R, kb, weights != nullptr, &p.any);
+    return any_launch(x_dtype == TLA_F64, p.any, X, ndim, shape, factors, weights, R, kb, out, ws, st);
+  }
+  // (a caller with less scratch than the plan's gets the vector kernel, which needs none)
+  if (p.path == Path::Generic || p.path == Path::Any) {
     if (x_dtype == TLA_F64)
       return launch_generic<double, double>((const double*)X, ndim, shape, factors, weights, R, kb,
                                             (double*)out, st);
@@ -1938,7 +1960,8 @@ int tla::mttkrp_launch(int x_dtype, const void* X, int ndim, const int64_t* shap
   Plan p;
   int rc = make_plan(x_dtype, ndim, shape, rank, kb, ke, precision, &p, job != nullptr && job->R > 0);
   if (rc != TLA_OK) return rc;
-  TLA_REQUIRE(ke == kb + 1 || p.path != Path::Generic, "partial MTTKRP needs an MFMA-eligible shape");
+  TLA_REQUIRE(ke == kb + 1 || (p.path != Path::Generic && p.path != Path::Any),
+              "partial MTTKRP needs an MFMA-eligible shape");
   if (job) TLA_REQUIRE(job->R >= 0 && job->R <= kMaxRank && job->grams && job->vi && job->vist, "bad side job");
   return run_plan(p, x_dtype, X, ndim, shape, factors, weights, rank, kb, ke, precision, out, ws, ws_bytes, st, job,
                   job_taken);
@@ -1950,6 +1973,13 @@ extern "C" size_t tla_mttkrp_workspace_size(int x_dtype, int ndim, const int64_t
   Plan p;
   if (make_plan(x_dtype, ndim, shape, rank, mode, mode + 1, precision, &p) != TLA_OK) return 0;
   return p.ws_bytes;
+}
+
+size_t tla::mttkrp_min_workspace(int x_dtype, int ndim, const int64_t* shape, int rank, int mode, int precision) {
+  if (mode < 0 || mode >= ndim) return 0;
+  Plan p;
+  if (make_plan(x_dtype, ndim, shape, rank, mode, mode + 1, precision, &p) != TLA_OK) return 0;
+  return p.path == Path::Any ? 0 : p.ws_bytes;
 }
 
 extern "C" int tla_mttkrp(int x_dtype, const void* X, int ndim, const int64_t* shape,
@@ -1972,7 +2002,7 @@ extern "C" size_t tla_mttkrp_partial_workspace_size(int x_dtype, int ndim, const
                                                     int precision) {
   Plan p;
   if (make_plan(x_dtype, ndim, shape, rank, keep_begin, keep_end, precision, &p) != TLA_OK) return 0;
-  return p.ws_bytes;
+  return p.path == Path::Any ? 0 : p.ws_bytes;
 }
 
 extern "C" int tla_mttkrp_partial(int x_dtype, const void* X, int ndim, const int64_t* shape,
@@ -1986,7 +2016,7 @@ extern "C" int tla_mttkrp_partial(int x_dtype, const void* X, int ndim, const in
   Plan p;
   int rc = make_plan(x_dtype, ndim, shape, rank, keep_begin, keep_end, precision, &p);
   if (rc != TLA_OK) return rc;
-  TLA_REQUIRE(p.path != Path::Generic, "partial MTTKRP needs an MFMA-eligible shape");
+  TLA_REQUIRE(p.path != Path::Generic && p.path != Path::Any, "partial MTTKRP needs an MFMA-eligible shape");
   return run_plan(p, x_dtype, X, ndim, shape, factors, weights, rank, keep_begin, keep_end,
                   precision, out, workspace, workspace_bytes, (hipStream_t)stream);
 }
@@ -1996,5 +2026,5 @@ extern "C" int tla_mttkrp_partial_supported(int x_dtype, int ndim, const int64_t
   if (!(keep_begin == 0 || keep_end == ndim) || (keep_begin == 0 && keep_end == ndim)) return 0;
   Plan p;
   if (make_plan(x_dtype, ndim, shape, rank, keep_begin, keep_end, precision, &p) != TLA_OK) return 0;
-  return p.path != Path::Generic ? 1 : 0;
+  return p.path != Path::Generic && p.path != Path::Any ? 1 : 0;
 }

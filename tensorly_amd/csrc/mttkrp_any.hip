@@ -1,0 +1,574 @@
+// MTTKRP of any mode sizes on the matrix cores, float32 and float64.
+//
+// The tensor is viewed as X[a, i, q] (i = output mode) and the output is
+// out[i, r] = sum_{a, q} X[a, i, q] B[(a, q), r], where B holds the rows of
+// the Khatri-Rao product of the other modes.  B is never stored: every wave
+// forms the part it needs in the registers that the matrix instructions read.
+//
+//  * any_rows_kernel (output mode is not the contiguous one): a wave takes
+//    chunks of 128 contiguous bytes of q for TN tiles of 16 rows i.  Lane
+//    (c, g) reads 32 consecutive bytes of row c of each tile, as they lie
+//    (dword aligned 16-byte loads), and forms B[(a, q), r] = G[(a, b), r]
+//    F_k[k, r] for its own q = (b, k) once for all TN tiles; G is the product
+//    of the weights and the factors of every mode but the output and the
+//    contiguous one.
+//  * any_last_kernel (output mode contiguous): a wave takes blocks of rows p
+//    (all the other modes, flattened) for TN tiles of 256 contiguous bytes of
+//    columns; the matrix instruction contracts over p.
+//
+// Bound: memory for ranks up to 32, the FP32 matrix rate above.  One set of
+// B rows serves all TN tiles of a wave; two sets of loaded values take turns,
+// so that a chunk is in flight while the one before is multiplied; a wave's
+// loads are all independent, so 16 waves per compute unit keep 100 KB in
+// flight.  Before, these shapes ran one block per output row on the vector
+// ALU, which read the tensor once per 16 rank columns with a 64-bit division
+// per element.  Measured, call by call with the reduction, mode 0 / 1 / 2:
+//   257 x 301 x 203, R = 20, float32: 1333 (mean) -> 27 / 29 / 28 us (2.3 TB/s)
+//   761 x 380 x 283, R = 16, float32: 77 / 98 / 73 us (4.3 / 3.3 / 4.5 TB/s)
+//   201 x 179 x 160, R = 16, float64: 621 (mean) -> 18 / 17 / 16 us (2.7 TB/s)
+//   149 x 120 x 90,  R = 10, float32: 172 (mean) -> 8 / 8 / 11 us
+#include <algorithm>
+
+#include "mttkrp_any.h"
+
+namespace tla {
+
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// Vector types of the tensor's loads: 16 bytes, aligned to one element.
+template <typename T> struct AnyT;
+template <> struct AnyT<float> {
+  typedef float vec __attribute__((ext_vector_type(4), aligned(4)));
+  typedef floatx4 acc;
+  static constexpr int V = 4;
+  // row of element e of a lane's accumulator (lane group g)
+  static __device__ __forceinline__ int row(int g, int e) { return 4 * g + e; }
+  static __device__ __forceinline__ acc mma(float a, float b, acc c) { return mfma_f32_16x16x4(a, b, c); }
+};
+template <> struct AnyT<double> {
+  typedef double vec __attribute__((ext_vector_type(2), aligned(8)));
+  typedef doublex4 acc;
+  static constexpr int V = 2;
+  static __device__ __forceinline__ int row(int g, int e) { return g + 4 * e; }
+  static __device__ __forceinline__ acc mma(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+};
+
+constexpr int kAnyWaves = 4;
+
+// *(p + off bytes): a wave-uniform base with a 32-bit lane offset
+template <typename U, typename T>
+__device__ __forceinline__ U at(const T* p, uint32_t off) {
+  return *(const U*)((const char*)p + off);
+}
+
+// rows per lane of one visit of any_last_kernel
+__host__ __device__ constexpr int any_last_rows(int TN, int RT) { return TN > 1 || RT > 1 ? 4 : 8; }
+// Waves per SIMD that a kernel's registers are cut for: two sets of loaded
+// values, the factor rows, the accumulators and some 40 for addresses.
+__host__ __device__ constexpr int any_occ(int TN, int RT, bool last, bool f64) {
+  const int d = f64 ? 2 : 1;
+  const int nr = any_last_rows(TN, RT);
+  const int regs = last ? 8 * TN * nr + 16 * TN * RT + d * RT * (nr + 2) + (RT == 4 ? 56 : 40)
+                        : 16 * TN + 4 * d * TN * RT + (8 + 2 * d) * RT + (f64 ? 54 : 40);
+  return regs <= 128 ? 4 : regs <= 168 ? 3 : 2;
+}
+
+template <typename T>
+struct AnyRowsArgs {
+  const T* X;
+  int64_t In, Q;
+  int K, Pb;
+  int R, ldr;       // columns of this slab, row stride of the factors
+  const T* G;       // (A Pb) x ldr, nullable
+  const T* Fk;      // K x ldr
+  T* partial;       // [nblk][In][R]
+  int nqc;
+  int64_t nchunks, nblk;
+};
+
+// Sum the waves' accumulators in wave order through LDS.
+template <typename T, int N>
+__device__ __forceinline__ void any_block_sum(typename AnyT<T>::acc (&acc)[N], T* red, int wave, int lane) {
+  for (int w = 0; w < kAnyWaves; ++w) {
+    if (wave == w) {
+#pragma unroll
+      for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          T* p = red + (n * 4 + e) * 64 + lane;
+          *p = w == 0 ? acc[n][e] : *p + acc[n][e];
+        }
+    }
+    __syncthreads();
+  }
+}
+
+template <typename T, int TN, int RT>
+__global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) == 8)) void any_rows_kernel(AnyRowsArgs<T> a) {
+  using V = typename AnyT<T>::vec;
+  using Acc = typename AnyT<T>::acc;
+  constexpr int VL = AnyT<T>::V, NV = 2 * VL, CH = 4 * NV;
+  __shared__ T red[TN * RT * 256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int64_t grp = blockIdx.x / a.nblk, blk = blockIdx.x - grp * a.nblk;
+  const int K = a.K, R = a.R, ldr = a.ldr;
+  const int64_t Q = a.Q, In = a.In, i0 = grp * (16 * TN);
+  // rows past the mode's end read its last row; their results are dropped
+  uint32_t roff[TN];  // bytes
+#pragma unroll
+  for (int t = 0; t < TN; ++t) 
+    roff[t] = (uint32_t)((min((int64_t)(16 * t + c), In - 1 - i0) * Q + NV * g) * sizeof(T));
+  uint32_t rr[RT];  // rank columns, in bytes; those past the slab read its last one
+#pragma unroll
+  for (int n = 0; n < RT; ++n) rr[n] = min(n * 16 + c, R - 1) * sizeof(T);
+  const uint32_t ldb = ldr * sizeof(T);
+  Acc acc[TN * RT];
+#pragma unroll
+  for (int n = 0; n < TN * RT; ++n) acc[n] = Acc{0, 0, 0, 0};
+
+  const int64_t step = a.nblk * kAnyWaves;
+  auto load = [&](int64_t ch, T (&x)[TN][NV]) {
+    const int64_t ia = ch / a.nqc;
+    const int q0 = (int)(ch - ia * a.nqc) * CH;
+    const T* xb = a.X + (ia * In + i0) * Q + q0;
+    if (q0 + CH <= (int)Q) {
+#pragma unroll
+      for (int t = 0; t < TN; ++t) {
+        const V v0 = at<V>(xb, roff[t]), v1 = at<V>(xb + VL, roff[t]);
+#pragma unroll
+        for (int v = 0; v < VL; ++v) { x[t][v] = v0[v]; x[t][VL + v] = v1[v]; }
+      }
+    } else {
+      const int left = (int)Q - (q0 + NV * g);  // values of this lane inside the row
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) x[t][v] = v < left ? at<T>(xb + v, roff[t]) : (T)0;
+    }
+  };
+  // Multiplies the chunk in x while the next one is loaded into xn (loads
+  // return in order, so the chunk's own factor rows are requested first).
+  auto visit = [&](int64_t ch, T (&x)[TN][NV], T (&xn)[TN][NV]) {
+    const int64_t ia = ch / a.nqc;
+    const int q0 = (int)(ch - ia * a.nqc) * CH;
+    const int left = (int)Q - (q0 + NV * g);
+    // this lane's rows of B: q = b K + k, and the next NV - 1 values of q
+    // may run into b + 1 (K >= NV), or are divided one by one
+    T f[RT][NV], g0[RT], g1[RT];
+    const int q = left > 0 ? q0 + NV * g : (int)Q - 1;
+    const int b0 = q / K;
+    int k0 = q - b0 * K;
+    const T* Gb = a.G ? a.G + ia * a.Pb * ldr : nullptr;
+    if (K >= NV) {
+      const int b1 = min(b0 + 1, a.Pb - 1);
+#pragma unroll
+      for (int n = 0; n < RT; ++n) {
+        g0[n] = Gb ? at<T>(Gb, b0 * ldb + rr[n]) : (T)1;
+        g1[n] = Gb ? at<T>(Gb, b1 * ldb + rr[n]) : (T)1;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) f[n][v] = at<T>(a.Fk, (k0 + v - (k0 + v >= K ? K : 0)) * ldb + rr[n]);
+      }
+    } else {
+#pragma unroll
+      for (int n = 0; n < RT; ++n) {
+        g0[n] = g1[n] = (T)1;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int qv = min(q + v, (int)Q - 1), b = qv / K;
+          f[n][v] = at<T>(a.Fk, (qv - b * K) * ldb + rr[n]) * (Gb ? at<T>(Gb, b * ldb + rr[n]) : (T)1);
+        }
+      }
+      k0 = -NV;  // the products are complete
+    }
+    if (ch + step < a.nchunks) load(ch + step, xn);
+#pragma unroll
+    for (int n = 0; n < RT; ++n)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        f[n][v] *= k0 + v >= K ? g1[n] : g0[n];
+        f[n][v] = v < left ? f[n][v] : (T)0;  // past the row's end both sides are zero
+      }
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int n = 0; n < RT; ++n) acc[t * RT + n] = AnyT<T>::mma(x[t][v], f[n][v], acc[t * RT + n]);
+  };
+  int64_t ch = blk * kAnyWaves + wave;
+  T x0[TN][NV], x1[TN][NV];
+  if (ch < a.nchunks) load(ch, x0);
+  while (ch < a.nchunks) {
+    visit(ch, x0, x1);
+    ch += step;
+    if (ch >= a.nchunks) break;
+    visit(ch, x1, x0);
+    ch += step;
+  }
+  any_block_sum<T, TN * RT>(acc, red, wave, lane);
+  // red[(t RT + n) 4 + e][lane] = out[i0 + 16 t + row(g, e)][16 n + c]
+  T* dst = a.partial + blk * In * R;
+  for (int idx = tid; idx < TN * RT * 256; idx += 64 * kAnyWaves) {
+    const int col = idx % (16 * RT), row = idx / (16 * RT);
+    const int t = row >> 4, ri = row & 15, n = col >> 4, cc = col & 15;
+    const int gg = sizeof(T) == 4 ? ri >> 2 : ri & 3, e = sizeof(T) == 4 ? ri & 3 : ri >> 2;
+    const int64_t i = i0 + row;
+    if (i < In && col < R) dst[i * R + col] = red[((t * RT + n) * 4 + e) * 64 + gg * 16 + cc];
+  }
+}
+
+template <typename T>
+struct AnyLastArgs {
+  const T* X;
+  int64_t P, K;
+  int J, nG;    // P = nG J
+  int R, ldr;
+  const T* G;   // (P / J) x ldr, nullable
+  const T* Fj;  // J x ldr
+  T* partial;   // [nblk][K][R]
+  int64_t nvisits, nblk;
+};
+
+template <typename T, int TN, int RT>
+__global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 8)) void any_last_kernel(AnyLastArgs<T> a) {
+  using V = typename AnyT<T>::vec;
+  using Acc = typename AnyT<T>::acc;
+  constexpr int VL = AnyT<T>::V;
+  constexpr int NR = any_last_rows(TN, RT);
+  constexpr int RV = 4 * NR;
+  __shared__ T red[TN * VL * RT * 256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int64_t grp = blockIdx.x / a.nblk, blk = blockIdx.x - grp * a.nblk;
+  const int R = a.R, ldr = a.ldr, J = a.J;
+  const int64_t K = a.K, k0 = grp * (16 * VL * TN);
+  // lanes that would read past the row's end read its last 16 bytes (and
+  // write those columns, with the same values as the lane they belong to)
+  uint32_t col[TN];  // bytes, with the lane's first row
+#pragma unroll
+  for (int t = 0; t < TN; ++t) {
+    const int64_t k = k0 + (16 * t + c) * VL;
+    col[t] = (uint32_t)((NR * g * K + min(k, K - VL)) * sizeof(T));
+  }
+  uint32_t rr[RT];  // rank columns, in bytes; those past the slab read its last one
+#pragma unroll
+  for (int n = 0; n < RT; ++n) rr[n] = min(n * 16 + c, R - 1) * sizeof(T);
+  const uint32_t ldb = ldr * sizeof(T);
+  Acc acc[TN * VL * RT];
+#pragma unroll
+  for (int n = 0; n < TN * VL * RT; ++n) acc[n] = Acc{0, 0, 0, 0};
+
+  const int step = (int)a.nblk * kAnyWaves, nv = (int)a.nvisits, P = (int)a.P;
+  auto load = [&](int v, V (&x)[NR][TN]) {
+    const T* xb = a.X + (int64_t)v * RV * K;
+    const int left = P - (v * RV + NR * g);
+    if (v * RV + RV <= P) {
+#pragma unroll
+      for (int u = 0; u < NR; ++u)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) x[u][t] = at<V>(xb + u * K, col[t]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < NR; ++u)
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+          x[u][t] = V{};
+          if (u < left) x[u][t] = at<V>(xb + u * K, col[t]);
+        }
+    }
+  };
+  // Multiplies the visit in x while the next one is loaded into xn.
+  auto visit = [&](int v, V (&x)[NR][TN], V (&xn)[NR][TN]) {
+    const int p0 = v * RV + NR * g;
+    const int left = P - p0;
+    // rows p0 + u of the Khatri-Rao product of the other modes
+    T f[RT][NR], g0[RT], g1[RT];
+    const uint32_t p = left > 0 ? p0 : P - 1;
+    const int a0 = (int)(p / (uint32_t)J);
+    int j0 = (int)(p - (uint32_t)a0 * J);
+    if (J >= NR) {
+      const int a1 = min(a0 + 1, a.nG - 1);
+#pragma unroll
+      for (int n = 0; n < RT; ++n) {
+        g0[n] = a.G ? at<T>(a.G, a0 * ldb + rr[n]) : (T)1;
+        g1[n] = a.G ? at<T>(a.G, a1 * ldb + rr[n]) : (T)1;
+#pragma unroll
+        for (int u = 0; u < NR; ++u) f[n][u] = at<T>(a.Fj, (j0 + u - (j0 + u >= J ? J : 0)) * ldb + rr[n]);
+      }
+    } else {
+#pragma unroll
+      for (int n = 0; n < RT; ++n) {
+        g0[n] = g1[n] = (T)1;
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+          const uint32_t pu = min(p + u, (uint32_t)P - 1), au = pu / (uint32_t)J;
+          f[n][u] = at<T>(a.Fj, (pu - au * J) * ldb + rr[n]) * (a.G ? at<T>(a.G, au * ldb + rr[n]) : (T)1);
+        }
+      }
+      j0 = -NR;  // the products are complete
+    }
+    if (v + step < nv) load(v + step, xn);
+#pragma unroll
+    for (int n = 0; n < RT; ++n)
+#pragma unroll
+      for (int u = 0; u < NR; ++u) {
+        f[n][u] *= j0 + u >= J ? g1[n] : g0[n];
+        f[n][u] = u < left ? f[n][u] : (T)0;
+      }
+#pragma unroll
+    for (int u = 0; u < NR; ++u)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int e = 0; e < VL; ++e)
+#pragma unroll
+          for (int n = 0; n < RT; ++n) {
+            Acc& d = acc[(t * VL + e) * RT + n];
+            d = AnyT<T>::mma(f[n][u], x[u][t][e], d);
+          }
+  };
+  int v = (int)blk * kAnyWaves + wave;
+  V x0[NR][TN], x1[NR][TN];
+  if (v < nv) load(v, x0);
+  while (v < nv) {
+    visit(v, x0, x1);
+    v += step;
+    if (v >= nv) break;
+    visit(v, x1, x0);
+    v += step;
+  }
+  any_block_sum<T, TN * VL * RT>(acc, red, wave, lane);
+  // red[((t VL + s) RT + n) 4 + e][lane] = out[col[t] + s][16 n + row(g, e)]
+  T* dst = a.partial + blk * K * R;
+  for (int idx = tid; idx < TN * VL * RT * 256; idx += 64 * kAnyWaves) {
+    const int r = idx % (16 * RT), kc = idx / (16 * RT);  // kc: column within the group
+    const int t = kc / (16 * VL), cc = (kc / VL) % 16, s = kc % VL;
+    const int n = r >> 4, ri = r & 15;
+    const int gg = sizeof(T) == 4 ? ri >> 2 : ri & 3, e = sizeof(T) == 4 ? ri & 3 : ri >> 2;
+    const int64_t k = k0 + (16 * t + cc) * VL;
+    if (k < K && r < R) dst[(min(k, K - VL) + s) * R + r] = red[(((t * VL + s) * RT + n) * 4 + e) * 64 + gg * 16 + cc];
+  }
+}
+
+// out[i ldo + r] = sum_{b < nblk} partial[b][i][r] in a fixed order: 32
+// elements x 8 lanes of b per block.
+template <typename T>
+__global__ __launch_bounds__(256) void any_reduce_kernel(const T* __restrict__ partial, int64_t n, int64_t nblk, int R,
+                                                         int64_t ldo, T* __restrict__ out) {
+  __shared__ T red[8][32];
+  const int el = threadIdx.x & 31, bl = threadIdx.x >> 5;
+  const int64_t e = (int64_t)blockIdx.x * 32 + el;
+  T s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+  if (e < n) {
+    const T* p = partial + e;
+    int64_t b = bl;
+    for (; b + 24 < nblk; b += 32) {
+      s0 += p[b * n];
+      s1 += p[(b + 8) * n];
+      s2 += p[(b + 16) * n];
+      s3 += p[(b + 24) * n];
+    }
+    for (; b < nblk; b += 8) s0 += p[b * n];
+  }
+  red[bl][el] = (s0 + s1) + (s2 + s3);
+  __syncthreads();
+  if (bl == 0 && e < n) {
+    T s = red[0][el];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) s += red[k][el];
+    out[(e / R) * ldo + e % R] = s;
+  }
+}
+
+// G[q, r] = w[r] * product over the listed modes' factor rows (q row-major
+// over those modes).
+template <typename T>
+struct AnyGArgs {
+  int n, R;
+  int64_t sz[kMaxOrder];
+  const T* fac[kMaxOrder];
+  const T* weights;
+  int64_t rows;
+};
+template <typename T>
+__global__ void any_g_kernel(AnyGArgs<T> a, T* __restrict__ out) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= a.rows * a.R) return;
+  const int r = (int)(e % a.R);
+  int64_t q = e / a.R;
+  T v = a.weights ? a.weights[r] : (T)1;
+#pragma unroll
+  for (int m = kMaxOrder - 1; m >= 0; --m)
+    if (m < a.n) {
+      const int64_t i = q % a.sz[m];
+      q /= a.sz[m];
+      v *= a.fac[m][i * a.R + r];
+    }
+  out[e] = v;
+}
+
+static size_t any_align(size_t b) { return (b + 255) & ~size_t(255); }
+
+bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, bool weights, AnyPlan* p) {
+  *p = AnyPlan{};
+  const int V = f64 ? 2 : 4, sz = f64 ? 8 : 4;
+  const int Rs = std::min(R, 64);
+  p->RT = (Rs + 15) / 16;
+  p->last = mode == ndim - 1;
+  p->K = shape[ndim - 1];
+  p->In = shape[mode];
+  p->A = 1;
+  p->Q = 1;
+  for (int m = 0; m < mode; ++m) p->A *= shape[m];
+  for (int m = mode + 1; m < ndim; ++m) p->Q *= shape[m];
+  // the kernels' 32-bit indices: q or p, an element of a factor or of the
+  // scale rows of one a, a byte within the rows of a wave's tiles
+  constexpr int64_t kBig = 0x7fffff00;
+  for (int m = 0; m < ndim; ++m)
+    if (shape[m] > kBig / (R * sz)) return false;
+  int64_t tiles;
+  int most;  // tiles per wave that the registers hold
+  if (p->last) {
+    if (p->K < V) return false;
+    p->J = shape[ndim - 2];
+    p->g_rows = p->A / p->J;
+    if (p->A > kBig || p->g_rows > kBig / (R * sz) || p->K > kBig / (32 * sz)) return false;
+    tiles = (p->K + 16 * V - 1) / (16 * V);
+    most = p->RT == 1 ? 3 : p->RT == 2 ? 2 : 1;
+  } else {
+    p->Pb = p->Q / p->K;
+    if (p->Q > kBig / (32 * sz) || p->Pb > kBig / (R * sz)) return false;
+    p->g_rows = p->A * p->Pb;
+    p->nqc = (int)((p->Q + 8 * V - 1) / (8 * V));
+    tiles = (p->In + 15) / 16;
+    most = !f64 || p->RT <= 2 ? 4 : p->RT == 3 ? 3 : 2;
+  }
+  // Tiles per wave: every wave forms its part of B once for all its tiles
+  // (about the cost of one more tile), and the chunks are dealt to the waves
+  // that fit the GPU at once in equal numbers: the least sum over a wave's
+  // chunks wins.
+  int64_t best = -1;
+  for (int tn = most; tn >= 1; --tn) {
+    const int64_t groups = (tiles + tn - 1) / tn;
+    const int TN = (int)((tiles + groups - 1) / groups);
+    const int RV = 4 * any_last_rows(TN, p->RT);
+    const int64_t chunks = p->last ? (p->A + RV - 1) / RV : p->A * p->nqc;
+    const int64_t waves = std::max<int64_t>(1, 256 * 4 * any_occ(TN, p->RT, p->last, f64) / groups);
+    const int64_t per = (chunks + waves - 1) / waves;
+    const int64_t cost = per * (TN + 1) * (p->last ? RV : 16);
+    if (best >= 0 && cost >= best) continue;
+    best = cost;
+    p->TN = TN;
+    p->groups = groups;
+    p->nchunks = chunks;
+    p->nblk = (chunks + kAnyWaves * per - 1) / (kAnyWaves * per);
+  }
+  if (ndim == 2) p->g_rows = 0;
+  // the table is a factor as it is when it covers one mode and no weights
+  p->build_g = p->g_rows > 0 && !(ndim == 3 && !weights);
+  // bounded scratch: at most 32 MiB of partial sums (one set: written to the output)
+  const int64_t set = p->In * Rs * sz;
+  p->nblk = std::max<int64_t>(1, std::min<int64_t>(p->nblk, (int64_t(32) << 20) / set));
+  if (p->groups * p->nblk > kBig) return false;
+  p->ws_bytes = (p->build_g ? any_align(size_t(p->g_rows) * R * sz) : 0) +
+                (p->nblk > 1 || R > 64 ? any_align(size_t(p->nblk) * set) : 0);
+  return true;
+}
+
+template <typename T, int RT>
+static void any_run_rows(int TN, unsigned grid, const AnyRowsArgs<T>& a, hipStream_t st) {
+  if (TN == 1) any_rows_kernel<T, 1, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  if (TN == 2) any_rows_kernel<T, 2, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  if constexpr (RT <= 3 || sizeof(T) == 4)
+    if (TN == 3) any_rows_kernel<T, 3, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  if constexpr (RT <= 2 || sizeof(T) == 4)
+    if (TN == 4) any_rows_kernel<T, 4, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+}
+
+template <typename T, int RT>
+static void any_run_last(int TN, unsigned grid, const AnyLastArgs<T>& a, hipStream_t st) {
+  // (a slab of ranks past 64 may have fewer rank tiles than the plan's)
+  if constexpr (RT == 1)
+    if (TN == 3) any_last_kernel<T, 3, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  if constexpr (RT <= 2)
+    if (TN == 2) any_last_kernel<T, 2, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  if (TN == 1) any_last_kernel<T, 1, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+}
+
+template <typename T>
+static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* shape, const void* const* factors,
+                        const T* weights, int R, int mode, T* out, void* ws, hipStream_t st) {
+  for (int m = 0; m < ndim; ++m) TLA_REQUIRE(m == mode || factors[m] != nullptr, "factor %d is NULL", m);
+  // modes of the table: all but the output mode and the one the kernel reads itself
+  const int own = p.last ? ndim - 2 : ndim - 1;
+  const T* G = nullptr;
+  char* w = (char*)ws;
+  if (p.g_rows > 0) {
+    AnyGArgs<T> ga{};
+    ga.R = R;
+    ga.weights = weights;
+    ga.rows = p.g_rows;
+    for (int m = 0; m < ndim; ++m)
+      if (m != mode && m != own) {
+        ga.sz[ga.n] = shape[m];
+        ga.fac[ga.n++] = (const T*)factors[m];
+      }
+    if (p.build_g) {
+      const int64_t ne = p.g_rows * R;
+      TLA_REQUIRE(ne <= int64_t(0x7fffffff) * 256, "scale table too large");
+      any_g_kernel<T><<<(unsigned)((ne + 255) / 256), 256, 0, st>>>(ga, (T*)w);
+      TLA_LAUNCH_CHECK();
+      G = (const T*)w;
+      w += any_align(size_t(ne) * sizeof(T));
+    } else {
+      G = ga.fac[0];
+    }
+  }
+  const unsigned grid = (unsigned)(p.groups * p.nblk);
+  for (int r0 = 0; r0 < R; r0 += 64) {
+    const int Rs = std::min(64, R - r0), RT = (Rs + 15) / 16;
+    const bool direct = p.nblk == 1 && Rs == R;
+    T* part = direct ? out : (T*)w;
+    const T* Gs = G ? G + r0 : nullptr;
+    if (p.last) {
+      const int RV = 4 * any_last_rows(p.TN, RT);
+      AnyLastArgs<T> a{X,    p.A, p.K, (int)p.J, (int)(p.A / p.J), Rs, R, Gs, (const T*)factors[own] + r0,
+                       part, (p.A + RV - 1) / RV, p.nblk};
+      switch (RT) {
+        case 1: any_run_last<T, 1>(p.TN, grid, a, st); break;
+        case 2: any_run_last<T, 2>(p.TN, grid, a, st); break;
+        case 3: any_run_last<T, 3>(p.TN, grid, a, st); break;
+        default: any_run_last<T, 4>(p.TN, grid, a, st); break;
+      }
+    } else {
+      AnyRowsArgs<T> a{X, p.In, p.Q, (int)p.K, (int)p.Pb, Rs, R, Gs, (const T*)factors[own] + r0, part, p.nqc,
+                       p.nchunks, p.nblk};
+      switch (RT) {
+        case 1: any_run_rows<T, 1>(p.TN, grid, a, st); break;
+        case 2: any_run_rows<T, 2>(p.TN, grid, a, st); break;
+        case 3: any_run_rows<T, 3>(p.TN, grid, a, st); break;
+        default: any_run_rows<T, 4>(p.TN, grid, a, st); break;
+      }
+    }
+    TLA_LAUNCH_CHECK();
+    if (!direct) {
+      const int64_t n = p.In * Rs;
+      any_reduce_kernel<T><<<(unsigned)((n + 31) / 32), 256, 0, st>>>(part, n, p.nblk, Rs, R, out + r0);
+      TLA_LAUNCH_CHECK();
+    }
+  }
+  return TLA_OK;
+}
+
+int any_launch(bool f64, const AnyPlan& p, const void* X, int ndim, const int64_t* shape, const void* const* factors,
+               const void* weights, int R, int mode, void* out, void* ws, hipStream_t st) {
+  return f64 ? any_launch_t<double>(p, (const double*)X, ndim, shape, factors, (const double*)weights, R, mode,
+                                    (double*)out, ws, st)
+             : any_launch_t<float>(p, (const float*)X, ndim, shape, factors, (const float*)weights, R, mode,
+                                   (float*)out, ws, st);
+}
+
+}  // namespace tla

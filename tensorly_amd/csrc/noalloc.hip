@@ -52,7 +52,7 @@ extern "C" int tla_mttkrp_noalloc(int x_dtype, const void* X, int ndim, const in
                                   void* out, void* stream) {
   TLA_REQUIRE(ndim >= 1 && ndim <= kMaxOrder && shape, "mttkrp_noalloc: bad order %d", ndim);
   const int prec = x_dtype == TLA_F64 ? TLA_PREC_VALU : precision;
-  const size_t need = tla_mttkrp_workspace_size(x_dtype, ndim, shape, rank, mode, prec);
+  const size_t need = mttkrp_min_workspace(x_dtype, ndim, shape, rank, mode, prec);
   TLA_REQUIRE(need <= kNoAllocScratchBytes,
               "mttkrp_noalloc: this MTTKRP needs %zu bytes of scratch; the allocation-free entry point holds "
               "%zu (use tla_mttkrp with a workspace)",

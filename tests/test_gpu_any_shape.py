@@ -1,0 +1,87 @@
+"""MTTKRP of unaligned shapes, ranks above 64 and float64 on the matrix cores,
+at the edges of its tiles: 16 rows, 64 / 32 columns, 32 / 16 contiguous
+values, rank tiles of 16 and slabs of 64.  Reference: FP64 torch on the same
+inputs.
+
+Tolerances (relative, Frobenius): each term is a product of up to five
+rounded values, and the partial sums of q terms of random sign are about
+sqrt(q) terms large, so their roundings add up to about sqrt(q) eps of the
+result in one chain.  The chains here have at most 4,900 terms: 70 eps, halved
+because the partial sums grow to that size only at the end: 32 eps, 2e-6 for
+float32 and 4e-15 for float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.float32: 2e-6, torch.float64: 4e-15}
+
+
+def reference(X, w, F, mode):
+    k = None
+    for i, f in enumerate(F):
+        if i != mode:
+            f = f.double()
+            k = f if k is None else (k[:, None, :] * f[None, :, :]).reshape(-1, f.shape[1])
+    if w is not None and len(F) > 2:  # khatri_rao of one matrix ignores the weights
+        k = k * w.double()
+    return torch.movedim(X.double(), mode, 0).reshape(X.shape[mode], -1) @ k
+
+
+def problem(cuda, shape, rank, dtype, seed):
+    g = torch.Generator(device=cuda).manual_seed(seed)
+    X = torch.randn(shape, generator=g, device=cuda, dtype=dtype)
+    F = [torch.randn((s, rank), generator=g, device=cuda, dtype=dtype) for s in shape]
+    w = torch.rand(rank, generator=g, device=cuda, dtype=dtype) + 0.5
+    return X, F, w
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rank", [1, 16, 17, 33, 64, 65, 130])
+@pytest.mark.parametrize("shape", [(7, 9), (33, 4), (17, 3), (15, 16, 17), (16, 5, 33), (300, 7, 9), (65, 66, 67),
+                                   (3, 2, 130), (130, 3, 4), (5, 6, 7, 8), (12, 10, 8, 31), (4, 3, 2, 3, 5)])
+def test_mttkrp_any_shape(cuda, shape, rank, dtype):
+    import tensorly_amd as tla
+    X, F, w = problem(cuda, shape, rank, dtype, sum(shape) + rank)
+    for mode in range(len(shape)):
+        for weights in (None, w):
+            out = tla.unfolding_dot_khatri_rao(X, (weights, F), mode)
+            ref = reference(X, weights, F, mode)
+            assert out.dtype == dtype and out.shape == ref.shape
+            err = float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref))
+            assert err < TOL[dtype], (mode, err)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(19, 21, 35), (6, 5, 11, 37)])
+def test_mttkrp_any_shape_infinities_stay_in_their_rows(cuda, shape, dtype):
+    """Padded rows, columns and rank columns must not carry an infinity or a
+    NaN into an output that does not depend on it."""
+    import tensorly_amd as tla
+    X, F, w = problem(cuda, shape, 5, dtype, 3)
+    F = [f.abs() + 0.1 for f in F]
+    for where, value in ((tuple(s - 1 for s in shape), float("inf")), (tuple(0 for _ in shape), float("nan")),
+                         (tuple(s // 2 for s in shape), float("-inf"))):
+        Y = X.clone()
+        Y[where] = value
+        for mode in range(len(shape)):
+            out = tla.unfolding_dot_khatri_rao(Y, (w, F), mode)
+            hit = torch.zeros(shape[mode], dtype=torch.bool, device=cuda)
+            hit[where[mode]] = True
+            assert bool(torch.isfinite(out[~hit]).all()), (where, mode)
+            bad = out[hit]
+            assert bool(torch.isnan(bad).all() if value != value else (bad == value).all()), (where, mode)
+
+
+def test_mttkrp_any_shape_without_scratch(cuda):
+    """A caller that brings no scratch gets the same result (to rounding)."""
+    from tensorly_amd import _lib
+    X, F, w = problem(cuda, (37, 41, 43), 9, torch.float32, 11)
+    sh, _k = _lib.shape_array(X.shape)
+    pp, _kf = _lib.ptr_array(F)
+    for mode in range(3):
+        out = torch.empty((X.shape[mode], 9), device=cuda)
+        _lib.check(_lib.lib().tla_mttkrp(_lib.F32, _lib.ptr(X), 3, sh, pp, _lib.ptr(w), 9, mode, _lib.PREC_FP32,
+                                         _lib.ptr(out), None, 0, _lib.stream(cuda)))
+        ref = reference(X, w, F, mode)
+        assert float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref)) < TOL[torch.float32]
