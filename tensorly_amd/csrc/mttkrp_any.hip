@@ -29,39 +29,12 @@
 //   149 x 120 x 90,  R = 10, float32: 172 (mean) -> 8 / 8 / 11 us
 #include <algorithm>
 
+#include "mma_any.h"
 #include "mttkrp_any.h"
 
 namespace tla {
 
-typedef double doublex4 __attribute__((ext_vector_type(4)));
-
-// Vector types of the tensor's loads: 16 bytes, aligned to one element.
-template <typename T> struct AnyT;
-template <> struct AnyT<float> {
-  typedef float vec __attribute__((ext_vector_type(4), aligned(4)));
-  typedef floatx4 acc;
-  static constexpr int V = 4;
-  // row of element e of a lane's accumulator (lane group g)
-  static __device__ __forceinline__ int row(int g, int e) { return 4 * g + e; }
-  static __device__ __forceinline__ acc mma(float a, float b, acc c) { return mfma_f32_16x16x4(a, b, c); }
-};
-template <> struct AnyT<double> {
-  typedef double vec __attribute__((ext_vector_type(2), aligned(8)));
-  typedef doublex4 acc;
-  static constexpr int V = 2;
-  static __device__ __forceinline__ int row(int g, int e) { return g + 4 * e; }
-  static __device__ __forceinline__ acc mma(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-};
-
 constexpr int kAnyWaves = 4;
-
-// *(p + off bytes): a wave-uniform base with a 32-bit lane offset
-template <typename U, typename T>
-__device__ __forceinline__ U at(const T* p, uint32_t off) {
-  return *(const U*)((const char*)p + off);
-}
 
 // rows per lane of one visit of any_last_kernel
 __host__ __device__ constexpr int any_last_rows(int TN, int RT) { return TN > 1 || RT > 1 ? 4 : 8; }
@@ -87,23 +60,6 @@ struct AnyRowsArgs {
   int nqc;
   int64_t nchunks, nblk;
 };
-
-// Sum the waves' accumulators in wave order through LDS.
-template <typename T, int N>
-__device__ __forceinline__ void any_block_sum(typename AnyT<T>::acc (&acc)[N], T* red, int wave, int lane) {
-  for (int w = 0; w < kAnyWaves; ++w) {
-    if (wave == w) {
-#pragma unroll
-      for (int n = 0; n < N; ++n)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          T* p = red + (n * 4 + e) * 64 + lane;
-          *p = w == 0 ? acc[n][e] : *p + acc[n][e];
-        }
-    }
-    __syncthreads();
-  }
-}
 
 template <typename T, int TN, int RT>
 __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) == 8)) void any_rows_kernel(AnyRowsArgs<T> a) {
@@ -208,7 +164,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
     visit(ch, x1, x0);
     ch += step;
   }
-  any_block_sum<T, TN * RT>(acc, red, wave, lane);
+  any_block_sum<T, TN * RT, kAnyWaves>(acc, red, wave, lane);
   // red[(t RT + n) 4 + e][lane] = out[i0 + 16 t + row(g, e)][16 n + c]
   T* dst = a.partial + blk * In * R;
   for (int idx = tid; idx < TN * RT * 256; idx += 64 * kAnyWaves) {
@@ -340,7 +296,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
     visit(v, x1, x0);
     v += step;
   }
-  any_block_sum<T, TN * VL * RT>(acc, red, wave, lane);
+  any_block_sum<T, TN * VL * RT, kAnyWaves>(acc, red, wave, lane);
   // red[((t VL + s) RT + n) 4 + e][lane] = out[col[t] + s][16 n + row(g, e)]
   T* dst = a.partial + blk * K * R;
   for (int idx = tid; idx < TN * VL * RT * 256; idx += 64 * kAnyWaves) {

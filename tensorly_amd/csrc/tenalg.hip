@@ -1,8 +1,7 @@
 // Khatri-Rao product, n-mode product (TTM / TTV) and the rank-diagonal
 // contraction used by the dimension-tree MTTKRP.
 //
-// mode_dot has two MFMA kernels for the Tucker chain (FP32 MFMA, BF16 or
-// split BF16x3, FP32 accumulation):
+// mode_dot has two MFMA kernels for BF16 and split BF16x3 (FP32 accumulation):
 //  * ttm_rows   -- contracting the contiguous (last) mode:
 //                  out[p, j] = sum_k X[p, k] U'[j, k], 16 rows per wave, the
 //                  U' panel staged transposed in LDS;
@@ -11,11 +10,12 @@
 //                  (16-byte loads of 4 consecutive b per lane, 256 bytes per
 //                  row per wave) and the m-range split over the 4 waves of a
 //                  block, reduced in LDS in a fixed order.
-// and a vector-ALU kernel for everything else (vectors, f64, J > 64, odd
-// sizes).
+// ttm_any.hip holds the float32 and float64 kernels (any sizes); a vector-ALU
+// kernel is left for precision "valu".
 #include <algorithm>
 
 #include "common.h"
+#include "ttm_any.h"
 
 namespace tla {
 
@@ -96,8 +96,7 @@ __global__ __launch_bounds__(256) void ttm_rows_kernel(TtmRowsArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, g = lane >> 4;
-  const int LDF = a.panel + 4, LDB = a.panel + 8;
-  float* Ct = (float*)smem;
+  const int LDB = a.panel + 8;
   __bf16* Ch = (__bf16*)smem;
   __bf16* Cl = Ch + RP * LDB;
   const int64_t p = ((int64_t)blockIdx.x * 4 + wave) * 16 + c;
@@ -112,13 +111,9 @@ __global__ __launch_bounds__(256) void ttm_rows_kernel(TtmRowsArgs a) {
     for (int idx = tid; idx < RP * klen; idx += 256) {
       const int n = idx % RP, kk = idx / RP;
       const float v = (n < a.J) ? a.U[n * a.ldj + (kb + kk) * a.ldk] : 0.0f;
-      if constexpr (PREC == TLA_PREC_FP32) {
-        Ct[n * LDF + kk] = v;
-      } else {
-        const __bf16 h = (__bf16)v;
-        Ch[n * LDB + kk] = h;
-        Cl[n * LDB + kk] = (__bf16)(v - (float)h);
-      }
+      const __bf16 h = (__bf16)v;
+      Ch[n * LDB + kk] = h;
+      Cl[n * LDB + kk] = (__bf16)(v - (float)h);
     }
     __syncthreads();
     for (int kk = 0; kk < klen; kk += 32) {
@@ -127,30 +122,17 @@ __global__ __launch_bounds__(256) void ttm_rows_kernel(TtmRowsArgs a) {
       floatx8 av;
       av[0] = x0[0]; av[1] = x0[1]; av[2] = x0[2]; av[3] = x0[3];
       av[4] = x1[0]; av[5] = x1[1]; av[6] = x1[2]; av[7] = x1[3];
-      if constexpr (PREC == TLA_PREC_FP32) {
+      bf16x8 ah, al;
+      if constexpr (PREC == TLA_PREC_BF16X3) split_bf16(av, ah, al);
+      else ah = __builtin_convertvector(av, bf16x8);
 #pragma unroll
-        for (int nb = 0; nb < RT; ++nb) {
-          const float* bp = Ct + (nb * 16 + c) * LDF + kk + 8 * g;
-          const floatx4 b0 = *(const floatx4*)bp;
-          const floatx4 b1 = *(const floatx4*)(bp + 4);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) d[nb] = mfma_f32_16x16x4(av[v], b0[v], d[nb]);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) d[nb] = mfma_f32_16x16x4(av[4 + v], b1[v], d[nb]);
-        }
-      } else {
-        bf16x8 ah, al;
-        if constexpr (PREC == TLA_PREC_BF16X3) split_bf16(av, ah, al);
-        else ah = __builtin_convertvector(av, bf16x8);
-#pragma unroll
-        for (int nb = 0; nb < RT; ++nb) {
-          const int off = (nb * 16 + c) * LDB + kk + 8 * g;
-          const bf16x8 bh = *(const bf16x8*)(Ch + off);
-          const bf16x8 bl = *(const bf16x8*)(Cl + off);
-          d[nb] = mfma_bf16_16x16x32(ah, bh, d[nb]);
-          d[nb] = mfma_bf16_16x16x32(ah, bl, d[nb]);
-          if constexpr (PREC == TLA_PREC_BF16X3) d[nb] = mfma_bf16_16x16x32(al, bh, d[nb]);
-        }
+      for (int nb = 0; nb < RT; ++nb) {
+        const int off = (nb * 16 + c) * LDB + kk + 8 * g;
+        const bf16x8 bh = *(const bf16x8*)(Ch + off);
+        const bf16x8 bl = *(const bf16x8*)(Cl + off);
+        d[nb] = mfma_bf16_16x16x32(ah, bh, d[nb]);
+        d[nb] = mfma_bf16_16x16x32(ah, bl, d[nb]);
+        if constexpr (PREC == TLA_PREC_BF16X3) d[nb] = mfma_bf16_16x16x32(al, bh, d[nb]);
       }
     }
   }
@@ -183,7 +165,7 @@ struct TtmColsArgs {
 template <int PREC, int RT>
 __global__ __launch_bounds__(256) void ttm_cols_kernel(TtmColsArgs a) {
   constexpr int RP = RT * 16;
-  constexpr int STEP = (PREC == TLA_PREC_FP32) ? 4 : 32;
+  constexpr int STEP = 32;
   __shared__ float red[64 * RP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, g = lane >> 4;
@@ -201,55 +183,38 @@ __global__ __launch_bounds__(256) void ttm_cols_kernel(TtmColsArgs a) {
 #pragma unroll
     for (int mb = 0; mb < RT; ++mb) acc[t][mb] = floatx4{0.f, 0.f, 0.f, 0.f};
   for (int64_t m0 = mb0; m0 < me; m0 += STEP) {
-    if constexpr (PREC == TLA_PREC_FP32) {
-      const int64_t m = m0 + g;
-      const bool ok = m < me;
-      floatx4 xv = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (ok && colok) xv = *(const floatx4*)(Xa + m * a.Pb + col);
-      float uv[RT];
+    floatx4 xv[8];
 #pragma unroll
-      for (int mb = 0; mb < RT; ++mb) {
-        const int j = mb * 16 + c;
-        uv[mb] = (ok && j < a.J) ? a.U[j * a.ldj + m * a.ldm] : 0.0f;
-      }
+    for (int v = 0; v < 8; ++v) {
+      const int64_t m = m0 + 8 * g + v;
+      xv[v] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (m < me && colok) xv[v] = *(const floatx4*)(Xa + m * a.Pb + col);
+    }
+    bf16x8 uh[RT], ul[RT];
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int mb = 0; mb < RT; ++mb) acc[t][mb] = mfma_f32_16x16x4(uv[mb], xv[t], acc[t][mb]);
-    } else {
-      floatx4 xv[8];
+    for (int mb = 0; mb < RT; ++mb) {
+      const int j = mb * 16 + c;
+      floatx8 u8;
 #pragma unroll
       for (int v = 0; v < 8; ++v) {
         const int64_t m = m0 + 8 * g + v;
-        xv[v] = floatx4{0.f, 0.f, 0.f, 0.f};
-        if (m < me && colok) xv[v] = *(const floatx4*)(Xa + m * a.Pb + col);
+        u8[v] = (m < me && j < a.J) ? a.U[j * a.ldj + m * a.ldm] : 0.0f;
       }
-      bf16x8 uh[RT], ul[RT];
+      split_bf16(u8, uh[mb], ul[mb]);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      floatx8 x8;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) x8[v] = xv[v][t];
+      bf16x8 xh, xl;
+      if constexpr (PREC == TLA_PREC_BF16X3) split_bf16(x8, xh, xl);
+      else xh = __builtin_convertvector(x8, bf16x8);
 #pragma unroll
       for (int mb = 0; mb < RT; ++mb) {
-        const int j = mb * 16 + c;
-        floatx8 u8;
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-          const int64_t m = m0 + 8 * g + v;
-          u8[v] = (m < me && j < a.J) ? a.U[j * a.ldj + m * a.ldm] : 0.0f;
-        }
-        split_bf16(u8, uh[mb], ul[mb]);
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        floatx8 x8;
-#pragma unroll
-        for (int v = 0; v < 8; ++v) x8[v] = xv[v][t];
-        bf16x8 xh, xl;
-        if constexpr (PREC == TLA_PREC_BF16X3) split_bf16(x8, xh, xl);
-        else xh = __builtin_convertvector(x8, bf16x8);
-#pragma unroll
-        for (int mb = 0; mb < RT; ++mb) {
-          acc[t][mb] = mfma_bf16_16x16x32(uh[mb], xh, acc[t][mb]);
-          acc[t][mb] = mfma_bf16_16x16x32(ul[mb], xh, acc[t][mb]);
-          if constexpr (PREC == TLA_PREC_BF16X3) acc[t][mb] = mfma_bf16_16x16x32(uh[mb], xl, acc[t][mb]);
-        }
+        acc[t][mb] = mfma_bf16_16x16x32(uh[mb], xh, acc[t][mb]);
+        acc[t][mb] = mfma_bf16_16x16x32(ul[mb], xh, acc[t][mb]);
+        if constexpr (PREC == TLA_PREC_BF16X3) acc[t][mb] = mfma_bf16_16x16x32(uh[mb], xl, acc[t][mb]);
       }
     }
   }
@@ -449,8 +414,7 @@ static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 template <int PREC>
 static int launch_ttm_rows(const TtmRowsArgs& a, hipStream_t st) {
   const int RT = (a.J + 15) / 16;
-  const size_t smem = (PREC == TLA_PREC_FP32) ? size_t(RT * 16) * (a.panel + 4) * 4
-                                              : size_t(2) * RT * 16 * (a.panel + 8) * 2;
+  const size_t smem = size_t(2) * RT * 16 * (a.panel + 8) * 2;
   const dim3 grid((unsigned)ceil_div(a.P, 64));
   switch (RT) {
     case 1: ttm_rows_kernel<PREC, 1><<<grid, 256, smem, st>>>(a); break;
@@ -597,21 +561,24 @@ extern "C" int tla_mode_dot(int dtype, const void* X, int ndim, const int64_t* s
   hipStream_t st = (hipStream_t)stream;
   const int64_t ne = Pa * J * Pb;
   if (ne == 0) return TLA_OK;
-  const bool mfma = dtype == TLA_F32 && !is_vector && J <= 64 &&
-                    (precision == TLA_PREC_FP32 || precision == TLA_PREC_BF16 || precision == TLA_PREC_BF16X3);
-  if (mfma && Pb == 1 && Im % 32 == 0) {
+  // BF16 and BF16x3 where the shape allows their aligned loads
+  const bool bf16 = dtype == TLA_F32 && !is_vector && J <= 64 &&
+                    (precision == TLA_PREC_BF16 || precision == TLA_PREC_BF16X3);
+  if (bf16 && Pb == 1 && Im % 32 == 0) {
     TtmRowsArgs a{(const float*)X, Pa, Im, (const float*)U, ldj, ldm, (int)J, (float*)out,
                   (int)std::min<int64_t>(Im, 128)};
-    if (precision == TLA_PREC_FP32) return launch_ttm_rows<TLA_PREC_FP32>(a, st);
     if (precision == TLA_PREC_BF16) return launch_ttm_rows<TLA_PREC_BF16>(a, st);
     return launch_ttm_rows<TLA_PREC_BF16X3>(a, st);
   }
-  if (mfma && Pb > 1 && Pb % 4 == 0 && Pa <= 65535) {
+  if (bf16 && Pb > 1 && Pb % 4 == 0 && Pa <= 65535) {
     TtmColsArgs a{(const float*)X, Pa, Im, Pb, (const float*)U, ldj, ldm, (int)J, (float*)out};
-    if (precision == TLA_PREC_FP32) return launch_ttm_cols<TLA_PREC_FP32>(a, st);
     if (precision == TLA_PREC_BF16) return launch_ttm_cols<TLA_PREC_BF16>(a, st);
     return launch_ttm_cols<TLA_PREC_BF16X3>(a, st);
   }
+  // everything else in the tensor's own arithmetic; precision "valu" and the
+  // sizes that the matrix kernels do not index stay on the vector ALU
+  if ((dtype == TLA_F64 || precision != TLA_PREC_VALU) && ttm_any_ok(dtype == TLA_F64, Pa, Im, Pb, J))
+    return ttm_any_launch(dtype == TLA_F64, X, Pa, Im, Pb, U, ldj, ldm, J, out, st);
   if (dtype == TLA_F32)
     ttm_generic_kernel<float><<<ceil_div(ne, 256), 256, 0, st>>>((const float*)X, Pa, Im, Pb, (const float*)U, J,
                                                                  ldj, ldm, (float*)out);

@@ -85,3 +85,40 @@ def test_mttkrp_any_shape_without_scratch(cuda):
                                          _lib.ptr(out), None, 0, _lib.stream(cuda)))
         ref = reference(X, w, F, mode)
         assert float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref)) < TOL[torch.float32]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("J", [1, 16, 17, 64, 65, 200])
+@pytest.mark.parametrize("shape", [(9,), (33, 4), (17, 19, 23), (3, 2, 130), (65, 66, 67), (300, 5, 9), (4, 3, 2),
+                                   (2, 70, 129), (4, 3, 2, 5)])
+def test_mode_dot_any_shape(cuda, shape, J, dtype):
+    """The tiles of the n-mode product: 16 or 64 rows, 64 / 32 columns, 16 rows
+    of the matrix per tile and 64 per block; sums of at most 300 terms, so the
+    tolerance above holds with room."""
+    import tensorly_amd as tla
+    g = torch.Generator(device=cuda).manual_seed(sum(shape) + J)
+    X = torch.randn(shape, generator=g, device=cuda, dtype=dtype)
+    for mode in range(len(shape)):
+        for transpose in (False, True):
+            U = torch.randn((shape[mode], J) if transpose else (J, shape[mode]), generator=g, device=cuda, dtype=dtype)
+            out = tla.mode_dot(X, U, mode, transpose=transpose)
+            A = (U.T if transpose else U).double()
+            ref = torch.movedim(torch.tensordot(A, X.double(), dims=([1], [mode])), 0, mode)
+            assert out.dtype == dtype and out.shape == ref.shape
+            err = float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref))
+            assert err < TOL[dtype], (mode, transpose, err)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_mode_dot_any_shape_infinities_stay_in_their_fibres(cuda, mode):
+    import tensorly_amd as tla
+    g = torch.Generator(device=cuda).manual_seed(5)
+    shape = (19, 21, 35)
+    X = torch.randn(shape, generator=g, device=cuda)
+    where = tuple(s - 1 for s in shape)
+    X[where] = float("inf")
+    U = torch.rand((shape[mode], 18), generator=g, device=cuda) + 0.1
+    out = torch.movedim(tla.mode_dot(X, U, mode, transpose=True), mode, -1)
+    hit = torch.zeros(out.shape[:2], dtype=torch.bool, device=cuda)
+    hit[tuple(s - 1 for s in out.shape[:2])] = True
+    assert bool(torch.isfinite(out[~hit]).all()) and bool((out[hit] == float("inf")).all())
