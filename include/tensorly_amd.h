@@ -249,9 +249,9 @@ int tla_cp_lstsq_grad_mode(int dtype, const void* factor, const void* mttkrp, vo
  * V, as the reference does (tensorly/solvers/nnls.py:147).  factor (rows x rank, dtype) is
  * updated in place, in FP64 arithmetic; iters_out (device int, nullable)
  * receives the iterations run.  With a workspace (nullable) and
- * n_iter_max <= 1000 each iteration is one launch over the whole GPU (a
- * device-side flag ends the remaining launches early); otherwise one
- * workgroup runs the loop.  Arguments otherwise as tla_nn_mu_update.
+ * n_iter_max <= 1000 the rows run up to 128 iterations per launch over the
+ * whole GPU (float32 factors are rounded at the end, not in between);
+ * otherwise one workgroup runs the loop.  Arguments otherwise as tla_nn_mu_update.
  * ------------------------------------------------------------------- */
 size_t tla_hals_nnls_workspace_size(int64_t rows, int rank);
 int tla_hals_nnls(int dtype, void* factor, const void* mttkrp, int64_t rows, int rank,

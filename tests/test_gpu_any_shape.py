@@ -122,3 +122,32 @@ def test_mode_dot_any_shape_infinities_stay_in_their_fibres(cuda, mode):
     hit = torch.zeros(out.shape[:2], dtype=torch.bool, device=cuda)
     hit[tuple(s - 1 for s in out.shape[:2])] = True
     assert bool(torch.isfinite(out[~hit]).all()) and bool((out[hit] == float("inf")).all())
+
+
+@pytest.mark.parametrize("rows,rank,n_iter", [(37, 1, 100), (16, 4, 127), (17, 5, 128), (33, 8, 129), (50, 20, 300),
+                                              (9, 1, 300)])
+def test_hals_chunks_and_stopping_rule(cuda, rows, rank, n_iter):
+    """The chunk lengths (128 iterations), workgroups of 16 rows, and the rule:
+    at rank 1 the second iteration changes nothing, so it fires there.  FP64
+    against the oracle: 300 iterations of a convergent descent, rounding
+    about 1e-13 relative to the largest entry."""
+    import numpy as np
+    from oracle import tensorly_np as T
+    from tensorly_amd import _lib
+    from tensorly_amd.cp_tensor import grams64
+    g = torch.Generator(device=cuda).manual_seed(rows + rank)
+    F = [torch.rand((s, rank), generator=g, device=cuda, dtype=torch.float64) for s in (rows, 12, 10)]
+    M = torch.randn((rows, rank), generator=g, device=cuda, dtype=torch.float64) * 3 + 1
+    A0, L = F[0].cpu().numpy(), _lib.lib()
+    grams = grams64(F)
+    gp, _k = _lib.ptr_array(grams)
+    iters = torch.zeros(1, dtype=torch.int32, device=cuda)
+    nb = L.tla_hals_nnls_workspace_size(rows, rank)
+    ws = _lib.workspace(nb, F[0].device)
+    _lib.check(L.tla_hals_nnls(_lib.F64, _lib.ptr(F[0]), _lib.ptr(M), rows, rank, gp, 3, 0, None, _lib.F64, 0.0, 0,
+                               n_iter, 1e-8, _lib.ptr(iters), _lib.ptr(ws), nb, _lib.stream(F[0].device)), "hals")
+    Fn = [f.cpu().numpy() for f in F]
+    utu = (Fn[1].T @ Fn[1]) * (Fn[2].T @ Fn[2])
+    ref = T.hals_nnls(M.cpu().numpy().T, utu, A0.T, n_iter_max=n_iter, tol=1e-8).T
+    np.testing.assert_allclose(Fn[0], ref, rtol=1e-9, atol=1e-12 * np.abs(ref).max())
+    assert int(iters) == (2 if rank == 1 else n_iter)
