@@ -126,12 +126,17 @@ int tla_rankdiag_contract(const float* Y, int64_t I, int64_t J, int rank, const 
  *   segments each row's nonzeros cut into n_seg pieces of at most seg_len:
  *            seg_row[j] / seg_start[j] (device int64, n_seg) give piece j's
  *            row and first position in perm; seg_row_ptr (shape[mode] + 1)
- *            delimits each row's pieces;
+ *            delimits each row's pieces.  With seg_row and seg_start NULL the
+ *            pieces are those of seg_row_ptr, all but a row's last of
+ *            seg_len, and n_seg is an upper bound of their number;
  *   factors  host array of ndim device pointers (entry `mode` unused), dtype;
  *   weights  R values (dtype) or NULL (ignored when ndim == 2, as for
  *            tla_mttkrp).  rank <= 64.
  *   workspace  tla_mttkrp_coo_workspace_size(dtype, n_seg, rank) bytes.
  * ------------------------------------------------------------------- */
+/* *bad (device int) = 1 when a coordinate (device int64 [ndim][nnz]) lies
+ * outside [0, shape[m]) of its mode, else 0. */
+int tla_coo_check(const int64_t* coords, int64_t nnz, int ndim, const int64_t* shape, int* bad, void* stream);
 size_t tla_mttkrp_coo_workspace_size(int dtype, int64_t n_seg, int rank);
 int tla_mttkrp_coo(int dtype, int64_t nnz, int ndim, const int64_t* shape, const int64_t* coords,
                    const void* values, const int64_t* perm, const int64_t* row_ptr, int64_t n_seg,

@@ -157,7 +157,7 @@ def unfolding_dot_khatri_rao(tensor, cp_tensor, mode):
     return out
 
 
-_COO_SEG = 1024  # nonzeros per piece of a row in the COO MTTKRP
+_COO_SEG = 256  # nonzeros per piece of a row in the COO MTTKRP
 
 
 def unfolding_dot_khatri_rao_coo(coords, values, shape, cp_tensor, mode):
@@ -187,33 +187,36 @@ def unfolding_dot_khatri_rao_coo(coords, values, shape, cp_tensor, mode):
                 raise ValueError(f"factor {m} has shape {tuple(factors[m].shape)}, expected ({int(s)}, {rank})")
     if weights is not None:
         _lib.require_on_device(weights, values.device, "weights")
-    if nnz and (int(coords.min()) < 0 or any(int(coords[m].max()) >= int(s) for m, s in enumerate(shape))):
-        raise ValueError("coordinates out of the tensor's shape")
     dev = values.device
     rows = int(shape[mode])
-    idx = coords[mode]
-    perm = torch.argsort(idx, stable=True) if nnz else torch.zeros(0, dtype=torch.int64, device=dev)
-    counts = torch.bincount(idx, minlength=rows) if nnz else torch.zeros(rows, dtype=torch.int64, device=dev)
-    row_ptr = torch.zeros(rows + 1, dtype=torch.int64, device=dev)
-    row_ptr[1:] = torch.cumsum(counts, 0)
+    sh, _keep_sh = shape_array(shape)
+    if nnz:
+        bad = torch.empty(1, dtype=torch.int32, device=dev)
+        check(lib().tla_coo_check(ptr(coords), nnz, len(shape), sh, ptr(bad), stream(dev)), "coo_check")
+        if bad.item():
+            raise ValueError("coordinates out of the tensor's shape")
+        # the narrowest key type: the sort makes a pass per eight bits
+        key = next(t for t in (torch.int16, torch.int32, torch.int64) if rows < torch.iinfo(t).max)
+        idx, perm = torch.sort(coords[mode].to(key), stable=True)
+        row_ptr = torch.searchsorted(idx, torch.arange(rows + 1, device=dev, dtype=key))
+    else:
+        perm = torch.zeros(0, dtype=torch.int64, device=dev)
+        row_ptr = torch.zeros(rows + 1, dtype=torch.int64, device=dev)
     # each row's nonzeros in pieces of at most _COO_SEG, so that modes with
-    # few rows still spread over many waves
-    nseg = (counts + (_COO_SEG - 1)) // _COO_SEG
+    # few rows still spread over many waves; at most one piece of a row is
+    # shorter, which bounds their number without reading it back
     seg_row_ptr = torch.zeros(rows + 1, dtype=torch.int64, device=dev)
-    seg_row_ptr[1:] = torch.cumsum(nseg, 0)
-    n_seg = int(seg_row_ptr[-1])
-    seg_row = torch.repeat_interleave(torch.arange(rows, device=dev), nseg)
-    seg_start = row_ptr[seg_row] + (torch.arange(n_seg, device=dev) - seg_row_ptr[seg_row]) * _COO_SEG
+    torch.cumsum((torch.diff(row_ptr) + (_COO_SEG - 1)) // _COO_SEG, 0, out=seg_row_ptr[1:])
+    n_seg = nnz // _COO_SEG + min(rows, nnz)
     facs = [None if m == mode else factors[m].to(dt).contiguous() for m in range(len(shape))]
     w = None if weights is None else weights.to(dt).contiguous()
     out = torch.empty((rows, rank), dtype=dt, device=dev)
     code = _lib.dtype_code(values)
     nb = lib().tla_mttkrp_coo_workspace_size(code, n_seg, rank)
     ws = workspace(nb, dev)
-    sh, _keep_sh = shape_array(shape)
     pp, _keep_f = ptr_array(facs)
     check(lib().tla_mttkrp_coo(code, nnz, len(shape), sh, ptr(coords), ptr(values.contiguous()), ptr(perm),
-                               ptr(row_ptr), n_seg, ptr(seg_row), ptr(seg_start), ptr(seg_row_ptr), _COO_SEG, pp,
+                               ptr(row_ptr), n_seg, None, None, ptr(seg_row_ptr), _COO_SEG, pp,
                                ptr(w), rank, mode, ptr(out), ptr(ws), nb, stream(dev)),
           "mttkrp_coo")
     return out

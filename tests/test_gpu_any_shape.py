@@ -151,3 +151,32 @@ def test_hals_chunks_and_stopping_rule(cuda, rows, rank, n_iter):
     ref = T.hals_nnls(M.cpu().numpy().T, utu, A0.T, n_iter_max=n_iter, tol=1e-8).T
     np.testing.assert_allclose(Fn[0], ref, rtol=1e-9, atol=1e-12 * np.abs(ref).max())
     assert int(iters) == (2 if rank == 1 else n_iter)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rank", [1, 4, 5, 16, 33, 64])
+@pytest.mark.parametrize("shape,nnz", [((3, 40), 700), ((1, 9, 7), 257), ((40, 3, 5), 64), ((6, 5, 4, 3), 1000),
+                                       ((2, 3, 4, 5, 6), 300), ((70, 2, 2), 1)])
+def test_mttkrp_coo_tiles(cuda, shape, nnz, rank, dtype):
+    """Lane groups of the padded rank, pieces of 256 nonzeros and their ends,
+    rows without nonzeros.  Sums of at most 1,000 terms: tolerance as above."""
+    from tensorly_amd.tenalg import unfolding_dot_khatri_rao_coo
+    g = torch.Generator(device=cuda).manual_seed(nnz + rank)
+    coords = torch.stack([torch.randint(0, s, (nnz,), generator=g, device=cuda) for s in shape])
+    values = torch.randn(nnz, generator=g, device=cuda, dtype=dtype)
+    F = [torch.randn((s, rank), generator=g, device=cuda, dtype=dtype) for s in shape]
+    w = torch.rand(rank, generator=g, device=cuda, dtype=dtype) + 0.5
+    for mode in range(len(shape)):
+        out = unfolding_dot_khatri_rao_coo(coords, values, shape, (w, F), mode)
+        t = values.double()[:, None].expand(nnz, rank)
+        for m in range(len(shape)):
+            if m != mode:
+                t = t * F[m].double()[coords[m]]
+        ref = torch.zeros((shape[mode], rank), dtype=torch.float64, device=cuda).index_add_(0, coords[mode], t)
+        if len(shape) > 2:
+            ref = ref * w.double()
+        assert out.dtype == dtype and out.shape == ref.shape
+        err = float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref))
+        assert err < TOL[dtype], (mode, err)
+    assert torch.equal(unfolding_dot_khatri_rao_coo(coords, values, shape, (w, F), 0),
+                       unfolding_dot_khatri_rao_coo(coords, values, shape, (w, F), 0))
