@@ -180,3 +180,44 @@ def test_mttkrp_coo_tiles(cuda, shape, nnz, rank, dtype):
         assert err < TOL[dtype], (mode, err)
     assert torch.equal(unfolding_dot_khatri_rao_coo(coords, values, shape, (w, F), 0),
                        unfolding_dot_khatri_rao_coo(coords, values, shape, (w, F), 0))
+
+
+def _spd(kind, n, rng):
+    import numpy as np
+    q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+    lam = {"spread": 10.0 ** -np.linspace(0, 6, n), "noise": np.sort(rng.random(n))[::-1] + 1.0,
+           "clusters": np.repeat(np.arange(n // 4 + 1, 0, -1.0), 4)[:n],
+           "low rank": np.where(np.arange(n) < max(1, n // 3), n - np.arange(n), 0.0),
+           "identity": np.ones(n)}[kind]
+    a = (q * lam) @ q.T
+    return (a + a.T) / 2, np.sort(lam)[::-1]
+
+
+@pytest.mark.parametrize("kind", ["spread", "noise", "clusters", "low rank", "identity"])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 16, 17, 48, 63, 64, 65, 90, 127, 128])
+def test_sym_eig_small(cuda, kind, n):
+    """The direct solver (separated eigenvalues) and the Jacobi sweeps it
+    leaves clusters to: eigenvalues, residuals and orthonormality to 1e-13 n
+    of the norm (backward stable steps of n rotations or reflections each)."""
+    import numpy as np
+    from tensorly_amd.svd import gram_eigh
+    a, lam = _spd(kind, n, np.random.default_rng(n))
+    G = torch.tensor(a, device=cuda)
+    for k in sorted({1, max(1, n // 3), n}):
+        w, v = (t.cpu().numpy() for t in gram_eigh(G, k))
+        tol = 1e-13 * max(n, 4) * lam[0]
+        assert np.max(np.abs(w - lam[:k])) < tol
+        assert np.max(np.abs(a @ v - v * w)) < tol
+        assert np.max(np.abs(v.T @ v - np.eye(k))) < 1e-13 * max(n, 4)
+
+
+@pytest.mark.parametrize("a", [[[0.0, 0.0], [0.0, 0.0]], [[2.0, 0.0, 0.0], [0.0, 3.0, 0.0], [0.0, 0.0, 1.0]],
+                               [[1e-30, 1e-31], [1e-31, 3e-30]], [[1e30, 1e29], [1e29, 3e30]]])
+def test_sym_eig_scales_and_diagonals(cuda, a):
+    import numpy as np
+    from tensorly_amd.svd import gram_eigh
+    a = np.array(a)
+    w, v = (t.cpu().numpy() for t in gram_eigh(torch.tensor(a, device=cuda), len(a)))
+    ref = np.linalg.eigvalsh(a)[::-1]
+    np.testing.assert_allclose(w, ref, rtol=1e-13, atol=0)
+    np.testing.assert_allclose(v.T @ v, np.eye(len(a)), atol=1e-13)
