@@ -172,23 +172,29 @@ def dtype_code(t):
 
 
 def ptr(t):
-    return c_p(t.data_ptr()) if t is not None else c_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def ptr_array(ts):
-    arr = (c_p * len(ts))()
-    for i, t in enumerate(ts):
-        arr[i] = t.data_ptr() if t is not None else 0
-    return ctypes.cast(arr, PP), arr
+    """``(pointers, keep)``: a C array of the tensors' device pointers (NULL
+    for None); ``keep`` has to outlive the call."""
+    arr = (c_p * len(ts))(*[t.data_ptr() if t is not None else None for t in ts])
+    return arr, arr
 
 
 def shape_array(shape):
     arr = (ctypes.c_int64 * len(shape))(*[int(s) for s in shape])
-    return ctypes.cast(arr, P_i64), arr
+    return arr, arr
 
 
 def stream(device=None):
-    return c_p(torch.cuda.current_stream(device).cuda_stream)
+    index = device.index if device is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+def ready(t, dtype):
+    """``t`` contiguous in ``dtype`` (itself where it already is)."""
+    return t if t.dtype is dtype and t.is_contiguous() else t.to(dtype).contiguous()
 
 
 def workspace(nbytes, device):

@@ -16,6 +16,7 @@ struct AnyPlan {
   int64_t nchunks;    // chunks (rows) / row visits (last)
   int64_t g_rows;     // rows of the precomputed scale table (0: none)
   bool build_g;       // the table has to be built (else it is a factor itself, or absent)
+  bool direct_g;      // ... but its rows are formed in the kernel
   size_t ws_bytes;
 };
 

@@ -48,6 +48,32 @@ __host__ __device__ constexpr int any_occ(int TN, int RT, bool last, bool f64) {
   return regs <= 128 ? 4 : regs <= 168 ? 3 : 2;
 }
 
+// G[q, r] = w[r] * product over the listed modes' factor rows (q row-major
+// over those modes).
+template <typename T>
+struct AnyGArgs {
+  int n, R;
+  int64_t sz[kMaxOrder];
+  const T* fac[kMaxOrder];
+  const T* weights;
+  int64_t rows;
+};
+
+// The entry of row q and byte column rb of the table G, formed from the
+// factors.
+template <typename T>
+__device__ __forceinline__ T g_entry(const AnyGArgs<T>& a, uint32_t q, uint32_t rb, uint32_t ldb) {
+  T v = a.weights ? at<T>(a.weights, rb) : (T)1;
+#pragma unroll
+  for (int m = kMaxOrder - 1; m >= 0; --m)
+    if (m < a.n) {
+      const uint32_t sz = (uint32_t)a.sz[m], i = q % sz;
+      q /= sz;
+      v *= at<T>(a.fac[m], i * ldb + rb);
+    }
+  return v;
+}
+
 template <typename T>
 struct AnyRowsArgs {
   const T* X;
@@ -55,13 +81,16 @@ struct AnyRowsArgs {
   int K, Pb;
   int R, ldr;       // columns of this slab, row stride of the factors
   const T* G;       // (A Pb) x ldr, nullable
+  AnyGArgs<T> ga;   // GD: the factors of G instead
   const T* Fk;      // K x ldr
   T* partial;       // [nblk][In][R]
   int nqc;
   int64_t nchunks, nblk;
 };
 
-template <typename T, int TN, int RT>
+// GD: every wave forms its scale rows from the factors (small problems, where
+// a launch for the table G costs more).
+template <typename T, int TN, int RT, bool GD = false>
 __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) == 8)) void any_rows_kernel(AnyRowsArgs<T> a) {
   using V = typename AnyT<T>::vec;
   using Acc = typename AnyT<T>::acc;
@@ -117,13 +146,17 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
     const int q = left > 0 ? q0 + NV * g : (int)Q - 1;
     const int b0 = q / K;
     int k0 = q - b0 * K;
-    const T* Gb = a.G ? a.G + ia * a.Pb * ldr : nullptr;
+    const T* Gb = !GD && a.G ? a.G + ia * a.Pb * ldr : nullptr;
+    auto scale = [&](int b, uint32_t rb) -> T {
+      if constexpr (GD) return g_entry(a.ga, (uint32_t)ia * a.Pb + b, rb, ldb);
+      else return Gb ? at<T>(Gb, b * ldb + rb) : (T)1;
+    };
     if (K >= NV) {
       const int b1 = min(b0 + 1, a.Pb - 1);
 #pragma unroll
       for (int n = 0; n < RT; ++n) {
-        g0[n] = Gb ? at<T>(Gb, b0 * ldb + rr[n]) : (T)1;
-        g1[n] = Gb ? at<T>(Gb, b1 * ldb + rr[n]) : (T)1;
+        g0[n] = scale(b0, rr[n]);
+        g1[n] = scale(b1, rr[n]);
 #pragma unroll
         for (int v = 0; v < NV; ++v) f[n][v] = at<T>(a.Fk, (k0 + v - (k0 + v >= K ? K : 0)) * ldb + rr[n]);
       }
@@ -134,7 +167,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
           const int qv = min(q + v, (int)Q - 1), b = qv / K;
-          f[n][v] = at<T>(a.Fk, (qv - b * K) * ldb + rr[n]) * (Gb ? at<T>(Gb, b * ldb + rr[n]) : (T)1);
+          f[n][v] = at<T>(a.Fk, (qv - b * K) * ldb + rr[n]) * scale(b, rr[n]);
         }
       }
       k0 = -NV;  // the products are complete
@@ -183,12 +216,13 @@ struct AnyLastArgs {
   int J, nG;    // P = nG J
   int R, ldr;
   const T* G;   // (P / J) x ldr, nullable
+  AnyGArgs<T> ga;  // GD: the factors of G instead
   const T* Fj;  // J x ldr
   T* partial;   // [nblk][K][R]
   int64_t nvisits, nblk;
 };
 
-template <typename T, int TN, int RT>
+template <typename T, int TN, int RT, bool GD = false>
 __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 8)) void any_last_kernel(AnyLastArgs<T> a) {
   using V = typename AnyT<T>::vec;
   using Acc = typename AnyT<T>::acc;
@@ -245,12 +279,16 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
     const uint32_t p = left > 0 ? p0 : P - 1;
     const int a0 = (int)(p / (uint32_t)J);
     int j0 = (int)(p - (uint32_t)a0 * J);
+    auto scale = [&](int i, uint32_t rb) -> T {
+      if constexpr (GD) return g_entry(a.ga, (uint32_t)i, rb, ldb);
+      else return a.G ? at<T>(a.G, i * ldb + rb) : (T)1;
+    };
     if (J >= NR) {
       const int a1 = min(a0 + 1, a.nG - 1);
 #pragma unroll
       for (int n = 0; n < RT; ++n) {
-        g0[n] = a.G ? at<T>(a.G, a0 * ldb + rr[n]) : (T)1;
-        g1[n] = a.G ? at<T>(a.G, a1 * ldb + rr[n]) : (T)1;
+        g0[n] = scale(a0, rr[n]);
+        g1[n] = scale(a1, rr[n]);
 #pragma unroll
         for (int u = 0; u < NR; ++u) f[n][u] = at<T>(a.Fj, (j0 + u - (j0 + u >= J ? J : 0)) * ldb + rr[n]);
       }
@@ -261,7 +299,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
           const uint32_t pu = min(p + u, (uint32_t)P - 1), au = pu / (uint32_t)J;
-          f[n][u] = at<T>(a.Fj, (pu - au * J) * ldb + rr[n]) * (a.G ? at<T>(a.G, au * ldb + rr[n]) : (T)1);
+          f[n][u] = at<T>(a.Fj, (pu - au * J) * ldb + rr[n]) * scale(au, rr[n]);
         }
       }
       j0 = -NR;  // the products are complete
@@ -339,16 +377,6 @@ __global__ __launch_bounds__(256) void any_reduce_kernel(const T* __restrict__ p
   }
 }
 
-// G[q, r] = w[r] * product over the listed modes' factor rows (q row-major
-// over those modes).
-template <typename T>
-struct AnyGArgs {
-  int n, R;
-  int64_t sz[kMaxOrder];
-  const T* fac[kMaxOrder];
-  const T* weights;
-  int64_t rows;
-};
 template <typename T>
 __global__ void any_g_kernel(AnyGArgs<T> a, T* __restrict__ out) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -425,18 +453,26 @@ bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, bool we
   if (ndim == 2) p->g_rows = 0;
   // the table is a factor as it is when it covers one mode and no weights
   p->build_g = p->g_rows > 0 && !(ndim == 3 && !weights);
+  // Small problems are short of launches, not of work: up to 24 chunks, a few
+  // per wave, one workgroup per group writes the output itself (5 us, where
+  // the sum of partials is another launch of 3 us on the host and 2.5 us on
+  // the GPU); up to 1024 chunks, a fraction of the GPU's waves, the scale
+  // rows are formed in place of a table (one launch of 3 us).
+  p->direct_g = p->build_g && p->TN == 1 && p->nchunks * p->groups <= 1024 && p->g_rows <= kBig;
+  if (p->nchunks <= 24) p->nblk = 1;
   // bounded scratch: at most 32 MiB of partial sums (one set: written to the output)
   const int64_t set = p->In * Rs * sz;
   p->nblk = std::max<int64_t>(1, std::min<int64_t>(p->nblk, (int64_t(32) << 20) / set));
   if (p->groups * p->nblk > kBig) return false;
-  p->ws_bytes = (p->build_g ? any_align(size_t(p->g_rows) * R * sz) : 0) +
+  p->ws_bytes = (p->build_g && !p->direct_g ? any_align(size_t(p->g_rows) * R * sz) : 0) +
                 (p->nblk > 1 || R > 64 ? any_align(size_t(p->nblk) * set) : 0);
   return true;
 }
 
 template <typename T, int RT>
 static void any_run_rows(int TN, unsigned grid, const AnyRowsArgs<T>& a, hipStream_t st) {
-  if (TN == 1) any_rows_kernel<T, 1, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  if (TN == 1 && a.ga.R) any_rows_kernel<T, 1, RT, true><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  else if (TN == 1) any_rows_kernel<T, 1, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
   if (TN == 2) any_rows_kernel<T, 2, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
   if constexpr (RT <= 3 || sizeof(T) == 4)
     if (TN == 3) any_rows_kernel<T, 3, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
@@ -451,7 +487,8 @@ static void any_run_last(int TN, unsigned grid, const AnyLastArgs<T>& a, hipStre
     if (TN == 3) any_last_kernel<T, 3, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
   if constexpr (RT <= 2)
     if (TN == 2) any_last_kernel<T, 2, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
-  if (TN == 1) any_last_kernel<T, 1, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  if (TN == 1 && a.ga.R) any_last_kernel<T, 1, RT, true><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  else if (TN == 1) any_last_kernel<T, 1, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
 }
 
 template <typename T>
@@ -461,9 +498,9 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
   // modes of the table: all but the output mode and the one the kernel reads itself
   const int own = p.last ? ndim - 2 : ndim - 1;
   const T* G = nullptr;
+  AnyGArgs<T> ga{};
   char* w = (char*)ws;
   if (p.g_rows > 0) {
-    AnyGArgs<T> ga{};
     ga.R = R;
     ga.weights = weights;
     ga.rows = p.g_rows;
@@ -472,7 +509,9 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
         ga.sz[ga.n] = shape[m];
         ga.fac[ga.n++] = (const T*)factors[m];
       }
-    if (p.build_g) {
+    if (p.direct_g) {
+      // (the kernels take it from ga)
+    } else if (p.build_g) {
       const int64_t ne = p.g_rows * R;
       TLA_REQUIRE(ne <= int64_t(0x7fffffff) * 256, "scale table too large");
       any_g_kernel<T><<<(unsigned)((ne + 255) / 256), 256, 0, st>>>(ga, (T*)w);
@@ -489,9 +528,15 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
     const bool direct = p.nblk == 1 && Rs == R;
     T* part = direct ? out : (T*)w;
     const T* Gs = G ? G + r0 : nullptr;
+    AnyGArgs<T> gs{};  // of this slab's columns; R = 0: not used
+    if (p.direct_g) {
+      gs = ga;
+      if (gs.weights) gs.weights += r0;
+      for (int m = 0; m < gs.n; ++m) gs.fac[m] += r0;
+    }
     if (p.last) {
       const int RV = 4 * any_last_rows(p.TN, RT);
-      AnyLastArgs<T> a{X,    p.A, p.K, (int)p.J, (int)(p.A / p.J), Rs, R, Gs, (const T*)factors[own] + r0,
+      AnyLastArgs<T> a{X,    p.A, p.K, (int)p.J, (int)(p.A / p.J), Rs, R, Gs, gs, (const T*)factors[own] + r0,
                        part, (p.A + RV - 1) / RV, p.nblk};
       switch (RT) {
         case 1: any_run_last<T, 1>(p.TN, grid, a, st); break;
@@ -500,7 +545,7 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
         default: any_run_last<T, 4>(p.TN, grid, a, st); break;
       }
     } else {
-      AnyRowsArgs<T> a{X, p.In, p.Q, (int)p.K, (int)p.Pb, Rs, R, Gs, (const T*)factors[own] + r0, part, p.nqc,
+      AnyRowsArgs<T> a{X, p.In, p.Q, (int)p.K, (int)p.Pb, Rs, R, Gs, gs, (const T*)factors[own] + r0, part, p.nqc,
                        p.nchunks, p.nblk};
       switch (RT) {
         case 1: any_run_rows<T, 1>(p.TN, grid, a, st); break;

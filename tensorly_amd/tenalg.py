@@ -133,27 +133,36 @@ def unfolding_dot_khatri_rao(tensor, cp_tensor, mode):
     if len(factors) != nd:
         raise ValueError(f"got {len(factors)} factors for a tensor of order {nd}")
     rank = factors[0].shape[1] if _ndim(factors[0]) == 2 else 1
-    for i, f in enumerate(factors):
-        _lib.require_on_device(f, tensor.device, f"factors[{i}]")
-        if i != mode and (f.shape[0] != tensor.shape[i] or (f.shape[1] if f.dim() == 2 else 1) != rank):
-            raise ValueError(f"factor {i} has shape {tuple(f.shape)}, expected "
-                             f"({tensor.shape[i]}, {rank})")
-    if weights is not None:
-        _lib.require_on_device(weights, tensor.device, "weights")
+    shape, dev = tensor.shape, tensor.device
     fdt = _mttkrp_dtype(tensor, factors)
+    facs = []
+    for i, f in enumerate(factors):
+        # (a factor that is as the kernels take it needs no further look)
+        if type(f) is torch.Tensor and f.dtype is fdt and f.device == dev and f.shape == (shape[i], rank):
+            facs.append(None if i == mode else f if f.is_contiguous() else f.contiguous())
+            continue
+        _lib.require_on_device(f, dev, f"factors[{i}]")
+        if i == mode:
+            facs.append(None)
+            continue
+        if f.shape[0] != shape[i] or (f.shape[1] if f.dim() == 2 else 1) != rank:
+            raise ValueError(f"factor {i} has shape {tuple(f.shape)}, expected ({shape[i]}, {rank})")
+        facs.append(_lib.ready(f.reshape(f.shape[0], rank), fdt))
+    w = None
+    if weights is not None:
+        _lib.require_on_device(weights, dev, "weights")
+        w = _lib.ready(weights, fdt)
     x = tensor.contiguous()
-    facs = [None if i == mode else f.reshape(f.shape[0], rank).to(fdt).contiguous()
-            for i, f in enumerate(factors)]
-    w = weights.to(fdt).contiguous() if weights is not None else None
-    out = torch.empty((tensor.shape[mode], rank), dtype=fdt, device=tensor.device)
+    out = torch.empty((shape[mode], rank), dtype=fdt, device=dev)
     xcode = _lib.dtype_code(x)
     prec = _lib.PREC_BF16 if xcode == _lib.BF16 else (_lib.PREC_VALU if xcode == _lib.F64 else _prec_code())
-    sh, _ks = shape_array(x.shape)
-    nbytes = lib().tla_mttkrp_workspace_size(xcode, nd, sh, rank, mode, prec)
-    ws = workspace(nbytes, x.device)
+    sh, _ks = shape_array(shape)
+    L = lib()
+    nbytes = L.tla_mttkrp_workspace_size(xcode, nd, sh, rank, mode, prec)
+    ws = workspace(nbytes, dev)
     pp, _keep = ptr_array(facs)
-    check(lib().tla_mttkrp(xcode, ptr(x), nd, sh, pp, ptr(w), rank, mode, prec, ptr(out), ptr(ws),
-                           nbytes, stream(x.device)), "unfolding_dot_khatri_rao")
+    check(L.tla_mttkrp(xcode, ptr(x), nd, sh, pp, ptr(w), rank, mode, prec, ptr(out), ptr(ws), nbytes, stream(dev)),
+          "unfolding_dot_khatri_rao")
     return out
 
 
