@@ -570,15 +570,20 @@ __device__ int lds_jacobi(double* A, double* W, int m, int max_sweeps, double2* 
   return sweep;
 }
 
-// order[r] = index of the r-th largest diagonal entry of A (ties by index)
+// order[r] = index of the r-th largest diagonal entry of A (ties by index,
+// NaN last: order is a permutation whatever A holds, as it indexes memory)
 template <int LDA>
 __device__ void sort_desc(const double* A, int m, int* order) {
   const int tid = threadIdx.x;
   if (tid < m) {
-    const double v = A[tid * LDA + tid];
+    auto key = [=](int i) {
+      const double v = A[i * LDA + i];
+      return v == v ? v : -INFINITY;
+    };
+    const double v = key(tid);
     int rank = 0;
     for (int j = 0; j < m; ++j) {
-      const double u = A[j * LDA + j];
+      const double u = key(j);
       if (u > v || (u == v && j < tid)) ++rank;
     }
     order[rank] = tid;
@@ -1180,7 +1185,13 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_small_kernel(EigBatch bat
 // (the same span; columns of very different lengths no longer spoil the
 // conditioning), and report whether one pass suffices: true when every
 // pivot of the equilibrated S is >= 1e-3 (cond(S) ~ 1e3 at most, so the
-// columns come out orthonormal to ~1e-13).  Without equil it returns true.
+// columns come out orthonormal to ~1e-13).
+//
+// A column whose pivot is lost to rounding (below 1e-15 of its own diagonal
+// entry: M has fewer than b independent columns) has no direction of its own;
+// eliminating with such a pivot overflows after a few of them.  It is left
+// out and comes out zero, with dpiv = infinity.  Without equil the return
+// value says whether there was none.
 template <int B>
 __device__ bool block_orth(const double* M, double* Out, int np, double* Sbuf, double* Tbuf, int ldt, bool shift,
                            double* pbuf, double* dpiv, double* scratch, double* stage, bool equil = false,
@@ -1204,6 +1215,7 @@ __device__ bool block_orth(const double* M, double* Out, int np, double* Sbuf, d
     double mx = 0.0;
     for (int i = 0; i < B; ++i) mx = fmax(mx, Sbuf[i * LDS_S + i]);
     scratch[40] = mx;
+    scratch[42] = 1.0;
   }
   __syncthreads();
   const double mx = scratch[40];
@@ -1229,8 +1241,13 @@ __device__ bool block_orth(const double* M, double* Out, int np, double* Sbuf, d
       }
       if (live && seg == kb) col[i] = x[kk];
       __syncthreads();
-      const double p = fmax(col[k], floor);
-      if (i == k && seg == 0) dpiv[k] = p;
+      const double q = col[k];
+      const bool lost = !(q > fmax(floor, 1e-15 * Sbuf[k * LDS_S + k]));
+      const double p = lost ? INFINITY : q;
+      if (i == k && seg == 0) {
+        dpiv[k] = p;
+        if (lost) scratch[42] = 0.0;
+      }
       if (live && i > k) {
         const double f = col[i] / p;
 #pragma unroll
@@ -1252,11 +1269,34 @@ __device__ bool block_orth(const double* M, double* Out, int np, double* Sbuf, d
     const int c = c0 + j;
     if (live && c >= B) Tbuf[(c - B) * ldt + i] = x[j] * ds * (equil ? dsc[c - B] : 1.0);
   }
-  const bool well = !equil || scratch[41] != 0.0;
+  const bool well = scratch[42] != 0.0 && (!equil || scratch[41] != 0.0);
   __syncthreads();
   if constexpr (B == 48) block_gemm_f64_panel<B>(M, Tbuf, ldt, Out, CAP, np, B, stage);
   else block_gemm_f64<false>(M, CAP, Tbuf, ldt, Out, CAP, np, B, B);
   return well;
+}
+
+// Out <- orth(M): one equilibrated Cholesky-QR pass when that leaves S well
+// conditioned, else two passes, shifted and plain, through `spare` (M itself
+// is kept).  Columns that the plain pass left out are filled with
+// pseudo-random ones and two more passes make the whole block orthonormal, so
+// that a matrix of rank below b keeps a whole block.
+template <int B>
+__device__ void orth_step(const double* M, double* spare, double* Out, int n, int np, double* H, double* T, int ldt,
+                          double* pbuf, double* dpiv, double* scratch, double* stage, double* resid) {
+#pragma unroll 1
+  for (int pass = 0; pass < 5; ++pass) {
+    const double* from = pass < 2 ? M : pass == 3 ? Out : spare;
+    double* to = pass == 1 || pass == 3 ? spare : Out;
+    const bool whole =
+        block_orth<B>(from, to, np, H, T, ldt, pass == 1, pbuf, dpiv, scratch, stage, pass == 0, resid);
+    if (whole && (pass == 0 || pass == 2)) return;
+    if (pass == 2) {
+      for (int e = threadIdx.x; e < n * B; e += blockDim.x)
+        if (isinf(dpiv[e % B])) Out[e] = hash_unit(e / B, B + e % B);
+      __syncthreads();
+    }
+  }
 }
 
 // Z = G V of the warm-block path spread over the GPU: one wave per 16 x 16
@@ -1332,10 +1372,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
   // Gp (zero-padded symmetric G) and the starting block Y come from
   // eig_prep_kernel, launched just before on the same stream
   if (phase == 1) {
-    if (!block_orth<B>(Z, V, np, H, T, ldt, false, pbuf, dpiv, scratch, stage, true, resid)) {
-      block_orth<B>(Z, U, np, H, T, ldt, true, pbuf, dpiv, scratch, stage);
-      block_orth<B>(U, V, np, H, T, ldt, false, pbuf, dpiv, scratch, stage);
-    }
+    orth_step<B>(Z, U, V, n, np, H, T, ldt, pbuf, dpiv, scratch, stage, resid);
     return;
   }
   const double jfloor = fmax(1e-30, 1e-2 * a.tol * a.tol);
@@ -1374,10 +1411,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
     else block_gemm_f64<true>(a.Gp, np, V, CAP, Z, CAP, np, B, np);
     // G V's columns are close to multiples of the warm columns: once
     // equilibrated, one unshifted Cholesky-QR pass usually suffices
-    if (!block_orth<B>(Z, V, np, H, T, ldt, false, pbuf, dpiv, scratch, stage, true, resid)) {
-      block_orth<B>(Z, U, np, H, T, ldt, true, pbuf, dpiv, scratch, stage);
-      block_orth<B>(U, V, np, H, T, ldt, false, pbuf, dpiv, scratch, stage);
-    }
+    orth_step<B>(Z, U, V, n, np, H, T, ldt, pbuf, dpiv, scratch, stage, resid);
     jthr = jfloor;
     it = 1;
   } else if (phase == 0 && !(a.Q0 && a.k0 > 0)) {
@@ -1387,10 +1421,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
     for (int p = 0; p < 2 && it + 2 < a.max_iter; ++p, ++it) {
       if constexpr (B == 48) gv_product<B, 128>(a.Gp, np, V, Z, stage);
       else block_gemm_f64<true>(a.Gp, np, V, CAP, Z, CAP, np, B, np);
-      if (!block_orth<B>(Z, V, np, H, T, ldt, false, pbuf, dpiv, scratch, stage, true, resid)) {
-        block_orth<B>(Z, U, np, H, T, ldt, true, pbuf, dpiv, scratch, stage);
-        block_orth<B>(U, V, np, H, T, ldt, false, pbuf, dpiv, scratch, stage);
-      }
+      orth_step<B>(Z, U, V, n, np, H, T, ldt, pbuf, dpiv, scratch, stage, resid);
     }
   }
   for (; it < a.max_iter; ++it) {
@@ -1495,10 +1526,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
     // V <- orth(U): the columns of U = G Y scale with the Ritz values, so
     // equilibrated first, one pass when that leaves S well conditioned,
     // else two Cholesky-QR passes (shifted, then plain)
-    if (!block_orth<B>(U, V, np, H, T, ldt, false, pbuf, dpiv, scratch, stage, true, resid)) {
-      block_orth<B>(U, Z, np, H, T, ldt, true, pbuf, dpiv, scratch, stage);
-      block_orth<B>(Z, V, np, H, T, ldt, false, pbuf, dpiv, scratch, stage);
-    }
+    orth_step<B>(U, Z, V, n, np, H, T, ldt, pbuf, dpiv, scratch, stage, resid);
   }
   eig_emit(a, Y, CAP, nullptr, theta, resid, B);
   if (tid == 0 && a.iters) *a.iters = it + 1;

@@ -221,3 +221,34 @@ def test_sym_eig_scales_and_diagonals(cuda, a):
     ref = np.linalg.eigvalsh(a)[::-1]
     np.testing.assert_allclose(w, ref, rtol=1e-13, atol=0)
     np.testing.assert_allclose(v.T @ v, np.eye(len(a)), atol=1e-13)
+
+
+@pytest.mark.parametrize("n,rank,k", [(144, 28, 28), (181, 28, 4), (200, 12, 30), (150, 1, 2), (130, 40, 44),
+                                      (256, 3, 60), (300, 90, 100), (160, 0, 5)])
+@pytest.mark.parametrize("warm", [False, True])
+def test_sym_eig_rank_below_the_block(cuda, n, rank, k, warm):
+    """Fewer independent directions than the block iteration keeps (48, 64 or
+    128), and than it is asked for: eigenvalues, residuals and orthonormality
+    as for a matrix of full rank.  2e-11: the solver stops at residuals of
+    1e-11 of the largest eigenvalue."""
+    import numpy as np
+    from tensorly_amd.svd import gram_eigh
+    x = np.random.default_rng(n).random((n, rank))
+    a = x @ x.T
+    q0 = torch.tensor(np.linalg.eigh(a)[1][:, ::-1][:, :k].copy(), device=cuda) if warm else None
+    w, v = (t.cpu().numpy() for t in gram_eigh(torch.tensor(a, device=cuda), k, q0))
+    lam = np.linalg.eigvalsh(a)[::-1]
+    tol = 2e-11 * lam[0]
+    assert np.max(np.abs(w - lam[:k])) <= tol
+    assert np.max(np.abs(a @ v - v * w)) <= tol
+    assert np.max(np.abs(v.T @ v - np.eye(k))) < 1e-12 * n
+
+
+@pytest.mark.parametrize("n", [40, 100, 150, 300])
+def test_sym_eig_nan(cuda, n):
+    """NaN in, NaN out, and the next solve is right."""
+    from tensorly_amd.svd import gram_eigh
+    w, v = gram_eigh(torch.full((n, n), float("nan"), device=cuda, dtype=torch.float64), 5)
+    assert torch.isnan(w).all()
+    w, v = gram_eigh(torch.eye(n, device=cuda, dtype=torch.float64), 5)
+    assert (w - 1).abs().max() < 1e-12
