@@ -1517,16 +1517,27 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
       scratch[63] = (worst <= a.tol * t1) ? 1.0 : 0.0;
       const double rr = worst / t1;
       scratch[62] = fmin(1e-10, fmax(jfloor, 1e-2 * rr * rr));
+      // A subspace step takes the residuals down by about the ratio of the
+      // block's last Ritz value to the k-th.  The steps that are still needed
+      // but the last are plain ones, V <- orth(G V), without the Ritz
+      // problem, which is most of a step's cost (n = 256: 67 us of 200).
+      const double rate = fabs(theta[B - 1]) / fmax(fabs(theta[k - 1]), 1e-300);
+      const double need = rate < 0.98 ? log(a.tol / rr) / log(rate) : 8.0;
+      scratch[61] = fmin(fmax(ceil(need) - 1.0, 0.0), 8.0);
     }
     __syncthreads();
     const bool done = scratch[63] != 0.0;
     jthr = scratch[62];
+    int plain = scratch[61] >= 1.0 ? (int)scratch[61] : 0;  // (0 for NaN)
     __syncthreads();
     if (done || it + 1 == a.max_iter) break;
-    // V <- orth(U): the columns of U = G Y scale with the Ritz values, so
-    // equilibrated first, one pass when that leaves S well conditioned,
-    // else two Cholesky-QR passes (shifted, then plain)
+    // V <- orth(U): the columns of U = G Y scale with the Ritz values
     orth_step<B>(U, Z, V, n, np, H, T, ldt, pbuf, dpiv, scratch, stage, resid);
+    for (; plain > 0 && it + 2 < a.max_iter; --plain, ++it) {
+      if constexpr (B == 48) gv_product<B, 128>(a.Gp, np, V, Z, stage);
+      else block_gemm_f64<true>(a.Gp, np, V, CAP, Z, CAP, np, B, np);
+      orth_step<B>(Z, U, V, n, np, H, T, ldt, pbuf, dpiv, scratch, stage, resid);
+    }
   }
   eig_emit(a, Y, CAP, nullptr, theta, resid, B);
   if (tid == 0 && a.iters) *a.iters = it + 1;
