@@ -367,74 +367,96 @@ __device__ bool lead_block_separated(const double* A, int m, int lead, double re
   return ok;
 }
 
-// Eigenvectors of the leading ma x ma block of a symmetric A that is nearly
-// diagonal, A = D + E (D its diagonal), by second-order perturbation theory
-// instead of Jacobi sweeps: with M[k][i] = E[k][i] / (d_i - d_k) (k != i),
-//   v_i = e_i + M e_i + sum_k e_k (E M)[k][i] / (d_i - d_k) - e_i sum_k M[k][i]^2 / 2,
-//   lambda_i = d_i + sum_k E[k][i] M[k][i],
-// correct to third order in max |M|.  Taken only when max |M| <= 1e-5 (no
-// close eigenvalues relative to the coupling): the neglected terms, sums of
-// up to ma^2 products of three entries of M, stay ~1e-12 of the vectors;
-// else false and nothing is written.  On success W[0:ma, 0:ma] = the vectors
-// (W is the identity on entry) and A's leading diagonal = the eigenvalues
-// (its off-diagonal entries are left as they were).  Mbuf, Pbuf: ma x ma
-// LDS scratch (stride ma).
+// The leading ma eigenvectors of a symmetric m x m A that is nearly diagonal
+// but for its trailing block, A = D + E (D its diagonal), by second-order
+// perturbation theory: with M[l][i] = E[l][i] / (d_i - d_l) (l != i < ma),
+//   v_i = e_i + M e_i + sum_l e_l (E M)[l][i] / (d_i - d_l) - e_i sum_l M[l][i]^2 / 2,
+//   lambda_i = d_i + sum_l E[l][i] M[l][i].
+// With mu = max |M|, g the same over the trailing rows l >= ma, and rho the
+// largest ratio of a trailing row's absolute sum within the trailing block to
+// its distance from the leading diagonal entries, the neglected terms are sums
+// of up to ma^2 products of three entries of M, and rho^2 g: taken when the
+// trailing diagonal lies below the leading one, mu <= mu_max, rho <= 0.05 and
+// rho^2 g <= 1e-13.  Returns 2 when mu <= 1e-5 (vectors good to ~1e-12), 1
+// otherwise (~1e-7: enough to go on with the iteration, not to end it), 0,
+// with nothing but scratch written, when not taken.  Writes columns < ma of W
+// (the identity on entry) and A's leading diagonal = the eigenvalues (its
+// other entries are left as they were).  Mbuf, Pbuf: m x ma LDS scratch
+// (stride ma).  Replaces the direct solver in a converging warm solve (n = 256,
+// k = 32, block 48): 125 -> 18 us.
 template <int LDA, int LDW>
-__device__ bool perturb_eigvecs(double* A, double* W, int ma, double* Mbuf, double* Pbuf, double* scratch) {
+__device__ int perturb_eigvecs(double* A, double* W, int m, int ma, double* Mbuf, double* Pbuf, double* scratch,
+                               double mu_max) {
   const int tid = threadIdx.x, nt = blockDim.x;
-  double mmax = 0.0;
-  for (int e = tid; e < ma * ma; e += nt) {
-    const int k = e / ma, i = e % ma;
+  double mu = 0.0, g = 0.0;
+  for (int e = tid; e < m * ma; e += nt) {
+    const int l = e / ma, i = e - l * ma;
     double mv = 0.0;
-    if (k != i) mv = A[k * LDA + i] / (A[i * LDA + i] - A[k * LDA + k]);
+    if (l != i) mv = A[l * LDA + i] / (A[i * LDA + i] - A[l * LDA + l]);
     Mbuf[e] = mv;
-    mmax = fmax(mmax, isfinite(mv) ? fabs(mv) : INFINITY);
+    const double mag = isfinite(mv) ? fabs(mv) : INFINITY;
+    mu = fmax(mu, mag);
+    if (l >= ma) g = fmax(g, mag);
   }
-  for (int off = 32; off > 0; off >>= 1) mmax = fmax(mmax, __shfl_xor(mmax, off, 64));
-  if ((tid & 63) == 0) scratch[tid >> 6] = mmax;
+  // trailing row tid: its sum, and its distance from the leading entries
+  double rho = 0.0;
+  if (tid >= ma && tid < m) {
+    double rad = 0.0, lo = INFINITY;
+#pragma unroll 4
+    for (int j = ma; j < m; ++j) rad += j == tid ? 0.0 : fabs(A[tid * LDA + j]);
+#pragma unroll 4
+    for (int i = 0; i < ma; ++i) lo = fmin(lo, A[i * LDA + i]);
+    const double gap = lo - A[tid * LDA + tid];
+    rho = gap > 0.0 && isfinite(rad) ? rad / gap : INFINITY;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    mu = fmax(mu, __shfl_xor(mu, off, 64));
+    g = fmax(g, __shfl_xor(g, off, 64));
+    rho = fmax(rho, __shfl_xor(rho, off, 64));
+  }
+  if ((tid & 63) == 0) {
+    const int w = tid >> 6;
+    scratch[w] = mu; scratch[8 + w] = g; scratch[16 + w] = rho;
+  }
   __syncthreads();
-  if (tid == 0) {
-    double mx = 0.0;
-    for (int w = 0; w < nt / 64 && w < 8; ++w) mx = fmax(mx, scratch[w]);
-    scratch[35] = (mx <= 1e-5) ? 1.0 : 0.0;
+  for (int w = 0; w < nt / 64; ++w) {
+    mu = fmax(mu, scratch[w]); g = fmax(g, scratch[8 + w]); rho = fmax(rho, scratch[16 + w]);
   }
   __syncthreads();
-  if (scratch[35] == 0.0) {
-    __syncthreads();
-    return false;
-  }
+  if (!(mu <= mu_max && rho <= 0.05 && rho * rho * g <= 1e-13)) return 0;
   // P = E M (E: A without its diagonal)
-  for (int e = tid; e < ma * ma; e += nt) {
-    const int k = e / ma, i = e % ma;
+  for (int e = tid; e < m * ma; e += nt) {
+    const int l = e / ma, i = e - l * ma;
     double pv = 0.0;
-    for (int l = 0; l < ma; ++l)
-      if (l != k) pv = fma(A[k * LDA + l], Mbuf[l * ma + i], pv);
+#pragma unroll 8
+    for (int q = 0; q < m; ++q) pv = fma(q == l ? 0.0 : A[l * LDA + q], Mbuf[q * ma + i], pv);
     Pbuf[e] = pv;
   }
   __syncthreads();
-  for (int e = tid; e < ma * ma; e += nt) {
-    const int k = e / ma, i = e % ma;
+  for (int e = tid; e < m * ma; e += nt) {
+    const int l = e / ma, i = e - l * ma;
     double wv;
-    if (k != i) {
-      wv = Mbuf[e] + Pbuf[e] / (A[i * LDA + i] - A[k * LDA + k]);
+    if (l != i) {
+      wv = Mbuf[e] + Pbuf[e] / (A[i * LDA + i] - A[l * LDA + l]);
     } else {
       double n2 = 0.0;
-      for (int l = 0; l < ma; ++l) n2 = fma(Mbuf[l * ma + i], Mbuf[l * ma + i], n2);
+#pragma unroll 4
+      for (int q = 0; q < m; ++q) n2 = fma(Mbuf[q * ma + i], Mbuf[q * ma + i], n2);
       wv = 1.0 - 0.5 * n2;
     }
-    W[k * LDW + i] = wv;
+    W[l * LDW + i] = wv;
   }
   // eigenvalues after every thread has read the diagonal above
   double lam = 0.0;
   if (tid < ma) {
     lam = A[tid * LDA + tid];
-    for (int k = 0; k < ma; ++k)
-      if (k != tid) lam = fma(A[k * LDA + tid], Mbuf[k * ma + tid], lam);
+#pragma unroll 4
+    for (int l = 0; l < m; ++l) lam = fma(l == tid ? 0.0 : A[l * LDA + tid], Mbuf[l * ma + tid], lam);
   }
   __syncthreads();
   if (tid < ma) A[tid * LDA + tid] = lam;
   __syncthreads();
-  return true;
+  return mu <= 1e-5 ? 2 : 1;
 }
 
 // One sweep is me - 1 rounds of me / 2 disjoint rotations.  Per round: wave 0
@@ -1380,6 +1402,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
   int it = 0;
   bool have_z = false;  // phase 2: Z = G V is there already
   bool direct = false;  // the Ritz matrix went through the direct solver
+  int pert = 0;         // or through perturb_eigvecs (its return value)
   if (phase == 2) {
     jthr = jfloor;
     it = 1;
@@ -1444,20 +1467,18 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
     // off-diagonal mass down to (residual / t_1)^2 / 100 of the total,
     // tightening to tol^2 / 100 as the residuals fall
     {
-      // a nearly diagonal leading block (a converging warm start): second-
-      // order perturbation instead of Jacobi sweeps when it is safe (block
-      // 48: its two k x k scratch matrices use the panel staging area)
-      const bool sep = k < B && lead_block_separated<LDH>(H, B, k, jthr, scratch);
-      bool pert = false;
+      // a nearly diagonal leading part (a converging warm start): second-
+      // order perturbation (block 48: its two B x k scratch matrices use the
+      // panel staging area); else the direct solver (block 48, its scratch in
+      // the staging area too); else Jacobi sweeps
       direct = false;
-      if constexpr (B == 48) {
-        if (sep) pert = perturb_eigvecs<LDH, LDW>(H, W, k, stage, stage + k * k, scratch);
-      }
-      // else the direct solver (block 48, its scratch in the staging area),
-      // else Jacobi sweeps
+      // (not twice in a row with what cannot end the iteration)
+      if constexpr (B == 48)
+        pert = perturb_eigvecs<LDH, LDW>(H, W, B, k, stage, stage + B * k, scratch, pert == 1 ? 1e-5 : 1e-3);
+      const bool sep = pert == 0 && k < B && lead_block_separated<LDH>(H, B, k, jthr, scratch);
       if constexpr (B == 48) {
         // (a separated leading block of few columns sweeps in less)
-        if (!pert && (!sep || k >= 24)) {
+        if (pert == 0 && (!sep || k >= 24)) {
           direct = direct_eig<1>([=](int i, int c) { return H[i * LDH + c]; }, B, B, stage, stage + B * 64, B, W, LDW,
                                  theta, dl);
           if (!direct) {
@@ -1467,7 +1488,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
           }
         }
       }
-      if (!pert && !direct) lds_jacobi<LDH, LDW>(H, W, B, 30, cs, pr, scratch, jthr, k, sep ? 1 : 0);
+      if (pert == 0 && !direct) lds_jacobi<LDH, LDW>(H, W, B, 30, cs, pr, scratch, jthr, k, sep ? 1 : 0);
     }
     if (direct) {
       if (tid < B) order[tid] = tid;
@@ -1514,13 +1535,13 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
       double worst = 0.0;
       for (int r = 0; r < k; ++r) worst = fmax(worst, resid[r]);
       const double t1 = fmax(fabs(theta[0]), 1e-300);
-      scratch[63] = (worst <= a.tol * t1) ? 1.0 : 0.0;
+      scratch[63] = (worst <= a.tol * t1 && pert != 1) ? 1.0 : 0.0;
       const double rr = worst / t1;
       scratch[62] = fmin(1e-10, fmax(jfloor, 1e-2 * rr * rr));
       // A subspace step takes the residuals down by about the ratio of the
       // block's last Ritz value to the k-th.  The steps that are still needed
       // but the last are plain ones, V <- orth(G V), without the Ritz
-      // problem, which is most of a step's cost (n = 256: 67 us of 200).
+      // problem (n = 256, block 48: 125 us of a step's 220).
       const double rate = fabs(theta[B - 1]) / fmax(fabs(theta[k - 1]), 1e-300);
       const double need = rate < 0.98 ? log(a.tol / rr) / log(rate) : 8.0;
       scratch[61] = fmin(fmax(ceil(need) - 1.0, 0.0), 8.0);

@@ -252,3 +252,27 @@ def test_sym_eig_nan(cuda, n):
     assert torch.isnan(w).all()
     w, v = gram_eigh(torch.eye(n, device=cuda, dtype=torch.float64), 5)
     assert (w - 1).abs().max() < 1e-12
+
+
+@pytest.mark.parametrize("n,k", [(130, 1), (200, 5), (256, 24), (256, 32), (300, 47), (256, 48)])
+@pytest.mark.parametrize("move", [1e-3, 1e-5, 1e-7, 1e-9, 1e-12])
+def test_sym_eig_warm_block_of_a_moved_matrix(cuda, n, k, move):
+    """Ritz problems from far to almost diagonal, over both sides of the
+    perturbation branch's limits, with a tail too flat to converge.  Residuals:
+    the solver's 1e-11, doubled; columns orthonormal to 1e-11 (third-order
+    terms: k^2 products of three ratios of at most 1e-5, ~1e-12)."""
+    import numpy as np
+    from tensorly_amd.svd import gram_left_singular
+    rng = np.random.default_rng(n + k)
+    lam = np.concatenate([np.linspace(10.0, 2.0, k), rng.uniform(0.3, 0.5, n - k)])
+    q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+    a = (q * lam) @ q.T
+    d = rng.standard_normal((n, n))
+    b = a + move * (d + d.T) / np.sqrt(n)
+    _, _, blk = gram_left_singular(torch.tensor((a + a.T) / 2, device=cuda), k, torch.float64, want_block=True)
+    for _ in range(2):
+        u, s, blk = gram_left_singular(torch.tensor(b, device=cuda), k, torch.float64, warm=blk, want_block=True)
+        u, w = u.cpu().numpy(), s.cpu().numpy() ** 2
+        assert np.max(np.abs(w - np.linalg.eigvalsh(b)[::-1][:k])) < 2e-10
+        assert np.max(np.abs(b @ u - u * w)) < 2e-10
+        assert np.max(np.abs(u.T @ u - np.eye(k))) < 1e-11
