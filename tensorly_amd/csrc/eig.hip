@@ -1564,130 +1564,11 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
   if (tid == 0 && a.iters) *a.iters = it + 1;
 }
 
-// ---------------------------------------------------------------------------
-// Mode Gram: G[i, j] = sum_{a,b} X[a, i, b] X[a, j, b], FP64 accumulation.
-// Block (ti, tj) computes a 32 x 32 tile for one chunk of the (a, b) pairs
-// (256 threads: four waves, one 16 x 16 FP64 MFMA tile each); partial tiles
-// are summed in chunk order.
-// ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256) void mode_gram_kernel(const T* __restrict__ X, int64_t Pa, int64_t In, int64_t Pb,
-                                                        int64_t chunk, double* __restrict__ partial) {
-  __shared__ double Ti[32][65];
-  __shared__ double Tj[32][65];
-  const int ti = blockIdx.x, tj = blockIdx.y;
-  if (tj < ti) return;
-  const int tid = threadIdx.x;
-  const int64_t q0 = (int64_t)blockIdx.z * chunk;
-  const int64_t Q = Pa * Pb;
-  const int64_t q1 = min(Q, q0 + chunk);
-  const int wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
-  const int mi = (wave >> 1) * 16, nj = (wave & 1) * 16;
-  doublex4 acc = doublex4{0.0, 0.0, 0.0, 0.0};
-  // thread: column qq of the 64-wide chunk, rows r0, r0 + 4, ..., r0 + 28 of
-  // both 32-row blocks; the chunk after the current one is loaded into
-  // registers while the current one is multiplied
-  const int qq = tid & 63, r0 = tid >> 6;
-  T ci[8], cj[8];
-  auto fetch = [&](int64_t qb) {
-    const int64_t q = qb + qq;
-    int64_t base = -1;
-    if (q < q1) {
-      const int64_t aa = q / Pb;
-      base = aa * In * Pb + (q - aa * Pb);
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int64_t gi = (int64_t)ti * 32 + r0 + 4 * u, gj = (int64_t)tj * 32 + r0 + 4 * u;
-      ci[u] = (base >= 0 && gi < In) ? X[base + gi * Pb] : (T)0;
-      cj[u] = (base >= 0 && gj < In) ? X[base + gj * Pb] : (T)0;
-    }
-  };
-  if (q0 < q1) fetch(q0);
-  for (int64_t qb = q0; qb < q1; qb += 64) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      Ti[r0 + 4 * u][qq] = (double)ci[u];
-      Tj[r0 + 4 * u][qq] = (double)cj[u];
-    }
-    __syncthreads();
-    if (qb + 64 < q1) fetch(qb + 64);
-    // wave w: the 16 x 16 output tile (w / 2, w % 2) of the 32 x 32 block on
-    // FP64 MFMA (products of the float inputs are exact in FP64)
-#pragma unroll
-    for (int k0 = 0; k0 < 64; k0 += 4)
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Ti[mi + lr][k0 + lk], Tj[nj + lr][k0 + lk], acc, 0, 0, 0);
-    __syncthreads();
-  }
-  double* out = partial + (int64_t)blockIdx.z * In * In;
-  // lane holds D[lk + 4 e][lr]
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int64_t i = (int64_t)ti * 32 + mi + lk + 4 * e, j = (int64_t)tj * 32 + nj + lr;
-    if (i < In && j < In) {
-      out[i * In + j] = acc[e];
-      out[j * In + i] = acc[e];
-    }
-  }
-}
-
-__global__ void sum_gram_partials_kernel(const double* __restrict__ partial, int64_t nn, int splits,
-                                         double* __restrict__ G) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nn) return;
-  double s = 0.0;
-  for (int k = 0; k < splits; ++k) s += partial[(int64_t)k * nn + e];
-  G[e] = s;
-}
-
 static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
-
-static int gram_splits(int64_t In, int64_t Q) {
-  const int64_t tiles = ((In + 31) / 32) * ((In + 31) / 32 + 1) / 2;
-  int64_t s = std::max<int64_t>(1, 1024 / std::max<int64_t>(tiles, 1));
-  s = std::min<int64_t>(s, (Q + 63) / 64);
-  s = std::min<int64_t>(s, 64);
-  return (int)std::max<int64_t>(1, s);
-}
 
 }  // namespace tla
 
 using namespace tla;
-
-extern "C" size_t tla_mode_gram64_workspace_size(int ndim, const int64_t* shape, int mode) {
-  if (mode < 0 || mode >= ndim) return 0;
-  int64_t In = shape[mode], Q = 1;
-  for (int m = 0; m < ndim; ++m)
-    if (m != mode) Q *= shape[m];
-  return align256(size_t(gram_splits(In, Q)) * In * In * 8);
-}
-
-extern "C" int tla_mode_gram64(int dtype, const void* X, int ndim, const int64_t* shape, int mode, double* G,
-                               void* ws, size_t ws_bytes, void* stream) {
-  TLA_REQUIRE(dtype == TLA_F32 || dtype == TLA_F64, "mode_gram64: bad dtype %d", dtype);
-  TLA_REQUIRE(ndim >= 1 && ndim <= kMaxOrder && mode >= 0 && mode < ndim, "mode_gram64: bad mode");
-  TLA_REQUIRE(ws_bytes >= tla_mode_gram64_workspace_size(ndim, shape, mode), "mode_gram64: workspace too small");
-  int64_t Pa = 1, Pb = 1;
-  for (int m = 0; m < mode; ++m) Pa *= shape[m];
-  for (int m = mode + 1; m < ndim; ++m) Pb *= shape[m];
-  const int64_t In = shape[mode];
-  const int splits = gram_splits(In, Pa * Pb);
-  const int64_t Q = Pa * Pb;
-  const int64_t chunk = ((Q + splits - 1) / splits + 63) / 64 * 64;
-  const int nti = ceil_div(In, 32);
-  hipStream_t st = (hipStream_t)stream;
-  double* partial = (double*)ws;
-  dim3 grid(nti, nti, splits);
-  if (dtype == TLA_F32)
-    mode_gram_kernel<float><<<grid, 256, 0, st>>>((const float*)X, Pa, In, Pb, chunk, partial);
-  else
-    mode_gram_kernel<double><<<grid, 256, 0, st>>>((const double*)X, Pa, In, Pb, chunk, partial);
-  TLA_LAUNCH_CHECK();
-  const int64_t nn = In * In;
-  sum_gram_partials_kernel<<<ceil_div(nn, 256), 256, 0, st>>>(partial, nn, splits, G);
-  TLA_LAUNCH_CHECK();
-  return TLA_OK;
-}
 
 static int64_t eig_np(int n) { return (int64_t)(n + 15) / 16 * 16; }
 

@@ -276,3 +276,17 @@ def test_sym_eig_warm_block_of_a_moved_matrix(cuda, n, k, move):
         assert np.max(np.abs(w - np.linalg.eigvalsh(b)[::-1][:k])) < 2e-10
         assert np.max(np.abs(b @ u - u * w)) < 2e-10
         assert np.max(np.abs(u.T @ u - np.eye(k))) < 1e-11
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(1, 1), (2, 1), (1, 40), (33, 16), (32, 13), (32, 14), (31, 17), (65, 1, 64), (5, 33, 16),
+                                   (3, 70, 19), (2, 1, 16), (130, 40, 2), (7, 64, 8, 2), (257, 1030), (40, 3, 37)])
+def test_mode_gram_any_shape(cuda, shape, dtype):
+    """Every mode, over the edges of tiles (32 rows) and pieces (16 columns),
+    against the same product in float64: sums of n products of float64."""
+    from tensorly_amd.svd import mode_gram
+    x = torch.randn(shape, dtype=dtype, generator=torch.Generator().manual_seed(len(shape))).to(cuda)
+    for m in range(len(shape)):
+        u = torch.movedim(x, m, 0).reshape(shape[m], -1).double().cpu()
+        bound = 2.3e-16 * u.shape[1] * (u.abs() @ u.abs().T)
+        assert bool(((mode_gram(x, m).cpu() - u @ u.T).abs() <= bound).all()), m
