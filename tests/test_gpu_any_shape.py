@@ -290,3 +290,13 @@ def test_mode_gram_any_shape(cuda, shape, dtype):
         u = torch.movedim(x, m, 0).reshape(shape[m], -1).double().cpu()
         bound = 2.3e-16 * u.shape[1] * (u.abs() @ u.abs().T)
         assert bool(((mode_gram(x, m).cpu() - u @ u.T).abs() <= bound).all()), m
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n", [1, 1023, 4096, 8192 * 3 + 5, 1024 * 4096 + 4097])
+def test_sqnorm_any_size_and_alignment(cuda, n, dtype):
+    """From an odd element on: n products summed in float64."""
+    from tensorly_amd.decomposition._tucker import _sqnorm64
+    x = torch.randn(n + 1, dtype=dtype, generator=torch.Generator().manual_seed(n))[1:].to(cuda)
+    ref = float((x.double().cpu() ** 2).sum())
+    assert abs(float(_sqnorm64(x)) - ref) <= 2.3e-16 * n * ref
