@@ -60,6 +60,7 @@ __device__ __forceinline__ bool block_gj_inverse(const double* V, int R, double*
 #pragma unroll
     for (int kk = 0; kk < CPT; ++kk) {
       const int k = kb * CPT + kk;
+      if (k >= R) break;  // rows past R are the identity's: nothing to do
       double* row = pbuf + (k & 1) * (3 * RP);
       double* col = row + 2 * RP;
       if (i == k) {
