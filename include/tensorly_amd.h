@@ -399,6 +399,14 @@ int tla_gram_svd_block(int n, int k);
 int tla_gram_left_singular(const double* G, int n, int k, const double* W0, int k0, int dtype, void* U,
                            void* s, double* U64, double* W_out, double tol, int max_iter, int* iters_out,
                            void* workspace, size_t workspace_bytes, void* stream);
+/* count (<= 8) cold-started tla_gram_left_singular problems of one dtype, one
+ * launch per solver kind and one workgroup each (the SVD inits of all modes,
+ * tensorly/decomposition/_cp.py:65-86 and _tucker.py:63-79).  Per-problem
+ * arrays; entries of s and W_out may be NULL. */
+int tla_gram_left_singular_batch(int count, const double* const* G, const int* n, const int* k, int dtype,
+                                 void* const* U, void* const* s, double* const* W_out, double tol,
+                                 int max_iter, void* const* workspace, const size_t* workspace_bytes,
+                                 void* stream);
 
 /* ---------------------------------------------------------------------
  * Native CP-ALS sweep driver: the mode loop of

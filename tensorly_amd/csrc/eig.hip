@@ -1700,23 +1700,48 @@ extern "C" int tla_gram_svd_block(int n, int k) {
   return k <= 40 ? 48 : (k <= 56 ? 64 : kEigCapLarge);
 }
 
+static int svd_args(const double* G, int n, int k, const double* W0, int k0, int dtype, void* U, void* s, double* U64,
+                    double* W_out, double tol, int max_iter, int* iters_out, void* ws, size_t ws_bytes, EigArgs* a,
+                    int* kind) {
+  TLA_REQUIRE(dtype == TLA_F32 || dtype == TLA_F64, "gram_left_singular: bad dtype %d", dtype);
+  TLA_REQUIRE(U, "gram_left_singular: NULL U");
+  const int rc = eig_args(G, n, k, W0, W0 ? k0 : 0, nullptr, U64, tol, max_iter, iters_out, ws, ws_bytes, a, kind);
+  if (rc != TLA_OK) return rc;
+  const int b = tla_gram_svd_block(n, k);
+  a->flip = 1;
+  a->out_dtype = dtype;
+  a->u_out = U;
+  a->s_out = s;
+  a->wblk = b > 0 ? W_out : nullptr;
+  a->wblock = (b > 0 && W0 && k0 == b && a->max_iter >= 2) ? 1 : 0;
+  return TLA_OK;
+}
+
 extern "C" int tla_gram_left_singular(const double* G, int n, int k, const double* W0, int k0, int dtype, void* U,
                                       void* s, double* U64, double* W_out, double tol, int max_iter, int* iters_out,
                                       void* ws, size_t ws_bytes, void* stream) {
-  TLA_REQUIRE(dtype == TLA_F32 || dtype == TLA_F64, "gram_left_singular: bad dtype %d", dtype);
-  TLA_REQUIRE(U, "gram_left_singular: NULL U");
   EigArgs a;
   int kind = 0;
-  const int rc = eig_args(G, n, k, W0, W0 ? k0 : 0, nullptr, U64, tol, max_iter, iters_out, ws, ws_bytes, &a, &kind);
+  const int rc = svd_args(G, n, k, W0, k0, dtype, U, s, U64, W_out, tol, max_iter, iters_out, ws, ws_bytes, &a, &kind);
   if (rc != TLA_OK) return rc;
-  const int b = tla_gram_svd_block(n, k);
-  a.flip = 1;
-  a.out_dtype = dtype;
-  a.u_out = U;
-  a.s_out = s;
-  a.wblk = b > 0 ? W_out : nullptr;
-  a.wblock = (b > 0 && W0 && k0 == b && a.max_iter >= 2) ? 1 : 0;
   return eig_launch(&a, &kind, 1, (hipStream_t)stream);
+}
+
+extern "C" int tla_gram_left_singular_batch(int count, const double* const* G, const int* n, const int* k, int dtype,
+                                            void* const* U, void* const* s, double* const* W_out, double tol,
+                                            int max_iter, void* const* workspace, const size_t* workspace_bytes,
+                                            void* stream) {
+  TLA_REQUIRE(count >= 1 && count <= kEigMaxBatch, "gram_left_singular_batch: count %d not in [1, %d]", count,
+              kEigMaxBatch);
+  TLA_REQUIRE(G && n && k && U && s && W_out && workspace && workspace_bytes, "gram_left_singular_batch: NULL array");
+  EigArgs args[kEigMaxBatch];
+  int kinds[kEigMaxBatch];
+  for (int i = 0; i < count; ++i) {
+    const int rc = svd_args(G[i], n[i], k[i], nullptr, 0, dtype, U[i], s[i], nullptr, W_out[i], tol, max_iter, nullptr,
+                            workspace[i], workspace_bytes[i], &args[i], &kinds[i]);
+    if (rc != TLA_OK) return rc;
+  }
+  return eig_launch(args, kinds, count, (hipStream_t)stream);
 }
 
 extern "C" int tla_sym_eig_batch(int count, const double* const* G, const int* n, const int* k,

@@ -62,13 +62,25 @@ def initialize_cp(tensor, rank, init="svd", svd="truncated_svd", non_negative=Fa
         factors = [torch.tensor(rng.random_sample((s, rank)), dtype=dt, device=dev) for s in tensor.shape]
         weights = torch.ones(rank, dtype=dt, device=dev)
     elif isinstance(init, str) and init == "svd":
-        from ..svd import svd_interface
+        from ..svd import SVD_FUNS, leading_left_singular_vectors_batch, svd_interface
         from ..base import unfold
         factors = []
+        # only U and S of the built-in SVD are needed: all modes' side by side
+        # (ranks above both sizes of an unfolding take the warning there, and
+        # orders above 8 the unfolded path)
+        batch = None
+        if (mask is None and not non_negative and isinstance(svd, str) and svd in SVD_FUNS and tensor.numel() > 0
+                and tensor.dim() <= 8
+                and all(rank <= max(s, tensor.numel() // s) for s in tensor.shape)):
+            _lib.require_gpu_tensor(tensor, "tensor")
+            batch = leading_left_singular_vectors_batch(tensor, list(range(tensor.dim())), [rank] * tensor.dim())
         for mode in range(tensor.dim()):
-            U, S, _ = svd_interface(unfold(tensor, mode), n_eigenvecs=rank, method=svd, non_negative=non_negative,
-                                    mask=None if mask is None else unfold(mask, mode),
-                                    n_iter_mask_imputation=svd_mask_repeats)
+            if batch is not None:
+                U, S, _ = batch[mode]
+            else:
+                U, S, _ = svd_interface(unfold(tensor, mode), n_eigenvecs=rank, method=svd, non_negative=non_negative,
+                                        mask=None if mask is None else unfold(mask, mode),
+                                        n_iter_mask_imputation=svd_mask_repeats)
             if mode == 0:
                 k = min(rank, S.shape[0])
                 U = U.clone()

@@ -39,8 +39,8 @@ def initialize_tucker(tensor, rank, modes, random_state, init="svd", svd="trunca
                       mask=None, svd_mask_repeats=5, warm64=None):
     """``_tucker.py:25-102`` (no mask).  With init='svd' the modes' SVDs are
     independent: their Gram eigensolves run side by side in one launch.
-    ``warm64`` (a list, optional) receives the FP64 factors of the SVD
-    init."""
+    ``warm64`` (a list, optional) receives the SVD init's final FP64 blocks
+    (None for modes without one)."""
     if mask is not None:
         raise NotImplementedError("mask is not supported by tensorly_amd.tucker")
     if isinstance(init, str) and init == "svd":
@@ -86,9 +86,9 @@ def partial_tucker(tensor, rank, modes=None, n_iter_max=100, init="svd", tol=10e
     else:
         rank = tuple(rank)
     with precision_ctx(precision or get_precision()):
-        # FP64 warm starts for the next eigensolve of each mode: the init's
-        # FP64 vectors, then the solver's whole final block (accurate past
-        # float32, and its guard columns need no re-orthonormalising)
+        # FP64 warm starts for the next eigensolve of each mode: the solver's
+        # whole final block (accurate past float32, and its guard columns
+        # need no re-orthonormalising)
         warm64 = []
         core, factors = initialize_tucker(tensor, rank, modes, init=init, svd=svd, random_state=random_state,
                                           warm64=warm64)

@@ -252,21 +252,28 @@ def leading_left_singular_vectors(tensor, mode, k, warm=None, return_warm=False)
 
 def leading_left_singular_vectors_batch(tensor, modes, ks):
     """:func:`leading_left_singular_vectors` of several modes of one tensor,
-    cold-started, the eigensolves in one batched launch (the Tucker SVD
-    init): a list of ``(U, S, U64)``, U64 the FP64 vectors (the first warm
-    start of each mode's HOOI solves)."""
-    Gs, kk, dims = [], [], []
-    for mode, k in zip(modes, ks):
-        n = tensor.shape[mode]
-        q = tensor.numel() // max(n, 1)
-        Gs.append(mode_gram(tensor, mode))
-        kk.append(min(k, n))
-        dims.append(min(n, q))
-    res = []
-    for (evals, evecs), k, md in zip(gram_eigh_batch(Gs, kk), ks, dims):
-        s = torch.sqrt(torch.clamp(evals, min=0.0))[: min(k, md)]
-        U, _ = svd_flip(evecs, None)
-        res.append((U.to(tensor.dtype), s.to(tensor.dtype), U))
+    cold-started, the eigensolves side by side (the SVD inits;
+    ``tla_gram_left_singular_batch``): a list of ``(U, S, block)``."""
+    tensor = tensor.contiguous()
+    dev, res = tensor.device, []
+    Ip, Zp = _lib.ctypes.c_int, _lib.ctypes.c_size_t
+    for c0 in range(0, len(modes), 8):
+        Gs = [mode_gram(tensor, m) for m in modes[c0 : c0 + 8]]
+        n = [int(G.shape[0]) for G in Gs]
+        k = [min(int(kk), nn) for kk, nn in zip(ks[c0 : c0 + 8], n)]
+        b = [int(lib().tla_gram_svd_block(nn, kk)) for nn, kk in zip(n, k)]
+        U = [torch.empty((nn, kk), dtype=tensor.dtype, device=dev) for nn, kk in zip(n, k)]
+        S = [torch.empty(kk, dtype=tensor.dtype, device=dev) for kk in k]
+        W = [torch.empty((nn, bb), dtype=torch.float64, device=dev) if bb else None for nn, bb in zip(n, b)]
+        nbs = [int(lib().tla_sym_eig_workspace_size(nn)) for nn in n]
+        wss = [workspace(nb, dev) for nb in nbs]
+        cnt = len(n)
+        arrays = [_lib.ptr_array(t) for t in (Gs, U, S, W, wss)]
+        gp, up, sp, bp, wp = (x[0] for x in arrays)
+        check(lib().tla_gram_left_singular_batch(cnt, gp, (Ip * cnt)(*n), (Ip * cnt)(*k), _lib.dtype_code(tensor), up,
+                                                 sp, bp, 1e-11, 300, wp, (Zp * cnt)(*nbs), stream(dev)),
+              "gram_left_singular_batch")
+        res.extend((u, s[: tensor.numel() // max(nn, 1)], w) for u, s, w, nn in zip(U, S, W, n))
     return res
 
 

@@ -9,6 +9,8 @@ sqrt(q) terms large, so their roundings add up to about sqrt(q) eps of the
 result in one chain.  The chains here have at most 4,900 terms: 70 eps, halved
 because the partial sums grow to that size only at the end: 32 eps, 2e-6 for
 float32 and 4e-15 for float64."""
+import warnings
+
 import pytest
 import torch
 
@@ -300,3 +302,36 @@ def test_sqnorm_any_size_and_alignment(cuda, n, dtype):
     x = torch.randn(n + 1, dtype=dtype, generator=torch.Generator().manual_seed(n))[1:].to(cuda)
     ref = float((x.double().cpu() ** 2).sum())
     assert abs(float(_sqnorm64(x)) - ref) <= 2.3e-16 * n * ref
+
+
+@pytest.mark.parametrize("shape,rank", [((149, 40, 300), 6), ((5, 70, 131), 9), ((260, 3), 3), ((2, 3, 2, 2, 2, 2, 2, 3), 2)])
+def test_svd_init_batch_equals_single_modes(cuda, shape, rank):
+    """All modes' solves in one call against one by one: the same solver on
+    the same Grams, up to eight at a time."""
+    from tensorly_amd.svd import leading_left_singular_vectors, leading_left_singular_vectors_batch
+    x = torch.rand(shape, dtype=torch.float64, generator=torch.Generator().manual_seed(rank)).to(cuda)
+    n = len(shape)
+    for m, (U, S, blk) in enumerate(leading_left_singular_vectors_batch(x, list(range(n)), [rank] * n)):
+        U1, S1, blk1 = leading_left_singular_vectors(x, m, rank, return_warm=True)
+        assert torch.equal(U, U1) and torch.equal(S, S1)
+        assert (blk is None) == (blk1 is None) and (blk is None or torch.equal(blk, blk1))
+
+
+@pytest.mark.parametrize("shape,rank", [((2, 3, 2, 2, 2, 2, 2, 2, 3), 2), ((4, 100), 100), ((3, 4), 6), ((1, 1), 1)])
+def test_svd_init_of_any_order_and_rank(cuda, shape, rank):
+    """Orders above the kernels' eight, and ranks above a mode's size (random
+    columns after U's) or above both sizes (a warning): U and S of numpy's
+    SVD, to the rounding of the squared spectrum (1e-7 of the largest)."""
+    import numpy as np
+    from tensorly_amd.decomposition._cp import initialize_cp
+    x = torch.rand(shape, dtype=torch.float64, generator=torch.Generator().manual_seed(3)).to(cuda)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        factors = initialize_cp(x, rank, init="svd", random_state=0)[1]
+    for m, f in enumerate(factors):
+        assert tuple(f.shape) == (shape[m], rank)
+        u, s, _ = np.linalg.svd(torch.movedim(x, m, 0).reshape(shape[m], -1).cpu().numpy(), full_matrices=False)
+        k = min(rank, len(s))
+        got = f[:, :k].cpu().numpy()
+        want = u[:, :k] * (s[:k] if m == 0 else 1.0)
+        assert np.max(np.abs(np.abs(got) - np.abs(want))) < 1e-7 * max(1.0, s[0])
