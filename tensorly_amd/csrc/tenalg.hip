@@ -268,9 +268,9 @@ __global__ __launch_bounds__(256) void rankdiag_axis1_kernel(const float* __rest
   red[threadIdx.x] = (s0 + s1) + (s2 + s3);
   __syncthreads();
   if (threadIdx.x < R) {
-    float t = 0.0f;
+    double t = 0.0;  // (up to 256 terms: in float32 their serial sum would round most)
     for (int k = 0; k < L; ++k) t += red[k * R + threadIdx.x];
-    out[i * R + threadIdx.x] = t;
+    out[i * R + threadIdx.x] = (float)t;
   }
 }
 
@@ -335,12 +335,12 @@ __global__ __launch_bounds__(256) void rankdiag_axis1_v4_kernel(const float* __r
   __syncthreads();
   if (threadIdx.x < R) {
     const int cc = threadIdx.x >> 2, comp = threadIdx.x & 3;
-    float t = 0.0f;
+    double t = 0.0;  // (as above)
     for (int k = 0; k < L; ++k) {
       const float4 v = red[k * C + cc];
       t += comp == 0 ? v.x : (comp == 1 ? v.y : (comp == 2 ? v.z : v.w));
     }
-    out[i * R + threadIdx.x] = t;
+    out[i * R + threadIdx.x] = (float)t;
   }
 }
 

@@ -262,6 +262,16 @@ def mttkrp_partial(tensor, cp_tensor, keep, precision_name=None):
     return out
 
 
+def mttkrp_partial_supported(tensor, rank, keep):
+    """Whether :func:`mttkrp_partial` has a matrix-core kernel for the tensor
+    in the current precision."""
+    code, prec = _lib.dtype_code(tensor), _prec_code()
+    if code != _lib.F32 or prec == _lib.PREC_VALU:
+        return False
+    sh, _ks = shape_array(tensor.shape)
+    return bool(lib().tla_mttkrp_partial_supported(code, _ndim(tensor), sh, rank, keep[0], keep[1], prec))
+
+
 def rankdiag_contract(Y, F, axis):
     """``Y`` is (I, J, R): axis 1 -> sum_j Y[i,j,r] F[j,r]; axis 0 -> sum_i Y[i,j,r] F[i,r]."""
     _lib.require_gpu_tensor(Y, "Y")

@@ -335,3 +335,39 @@ def test_svd_init_of_any_order_and_rank(cuda, shape, rank):
         got = f[:, :k].cpu().numpy()
         want = u[:, :k] * (s[:k] if m == 0 else 1.0)
         assert np.max(np.abs(np.abs(got) - np.abs(want))) < 1e-7 * max(1.0, s[0])
+
+
+@pytest.mark.parametrize("shape,rank,precision", [((256, 256, 256), 16, "fp32"), ((512, 512, 64), 16, "fp32"),
+                                                  ((64, 128, 2048), 33, "fp32"), ((256, 256, 260), 5, "fp32"),
+                                                  ((256, 256, 256), 24, "bf16x3"), ((256, 256, 256), 4, "valu")])
+def test_cp_lstsq_grad_shared_contraction(cuda, shape, rank, precision):
+    """Sizes on both sides of the shared contraction's rule (2^24 entries,
+    shape[2] >= 4 rank, a matrix-core kernel), with weights, against float64.
+    The MTTKRP's tolerance above on the larger of the two terms."""
+    import tensorly_amd as tla
+    gen = torch.Generator(device=cuda).manual_seed(rank)
+    x = torch.randn(shape, device=cuda, generator=gen)
+    w = torch.rand(rank, device=cuda, generator=gen) + 0.5
+    F = [torch.randn(s, rank, device=cuda, generator=gen) for s in shape]
+    with tla.tenalg.precision(precision):
+        grads = tla.cp_lstsq_grad((w, F), x).factors
+    D, wd, xd = [f.double() for f in F], w.double(), x.double()
+    G = [d.T @ d for d in D]
+    for m in range(3):
+        i, j = (k for k in range(3) if k != m)
+        acc = G[i] * G[j] * (wd[:, None] * wd[None, :])
+        model = D[m] @ acc
+        mt = reference(xd, wd, D, m)
+        err = (grads[m].double() - (model - mt)).norm()
+        assert float(err / max(model.norm(), mt.norm())) < (2e-6 if precision != "bf16x3" else 2e-5)
+
+
+@pytest.mark.parametrize("rows,rank", [(1, 1), (63, 16), (64, 17), (65, 33), (577, 64), (1500, 10)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_gram64_edges(cuda, rows, rank, dtype):
+    """Row blocks of 64, rank tiles of 16, eight partials at a time: sums of
+    `rows` float64 products."""
+    from tensorly_amd.cp_tensor import grams64
+    a = torch.randn(rows, rank, dtype=dtype, generator=torch.Generator().manual_seed(rows)).to(cuda)
+    g, d = grams64([a])[0].cpu(), a.double().cpu()
+    assert bool(((g - d.T @ d).abs() <= 2.3e-16 * (rows + 8) * (d.abs().T @ d.abs())).all())
