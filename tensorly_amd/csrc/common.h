@@ -43,7 +43,7 @@ constexpr int kMaxOrder = 8;
 constexpr int kMaxRank = 64;  // CP rank limit of the ALS solve / Gram kernels
 constexpr int kWave = 64;
 
-// A side job for a persistent MTTKRP launch: invert the normal-equations
+// A side job for an MTTKRP launch: invert the normal-equations
 // matrix of `mode` (see inverse.h) in one extra workgroup.  R == 0: none.
 struct InvJob {
   const double* grams;  // ndim Grams, R x R FP64, back to back
@@ -143,7 +143,8 @@ int cp_solve_launch(int dtype, const double* const* grams, int ndim, int mode, c
                     int* vist_next, int* status_max, void* stream);
 
 // tla_mttkrp (ke == kb + 1) / tla_mttkrp_partial keeping modes [kb, ke),
-// with an optional side job (InvJob, nullable) that the persistent kernels
+// with an optional side job (InvJob, nullable) that the persistent kernels, and
+// the sum of partials of mttkrp_any.hip,
 // run in one extra workgroup; *job_taken (nullable) reports whether this
 // launch ran it (otherwise the caller must do it some other way).
 int mttkrp_launch(int x_dtype, const void* X, int ndim, const int64_t* shape, const void* const* factors,

@@ -152,7 +152,7 @@ static void invalidate_inverses(CpAls* h) {
 
 // Where each solve's V^-1 comes from: the MTTKRP launch that precedes the
 // solve runs it in one extra workgroup (side job) when its kernel is a
-// persistent one; for the second mode of a dimension-tree half (only a short
+// persistent one or it ends in a sum of partials; for the second mode of a dimension-tree half (only a short
 // rank-diagonal contraction in between) the previous solve's finalising
 // block forms it; otherwise the solve inverts V itself.
 static InvJob inv_job(const CpAls* h, int n) {

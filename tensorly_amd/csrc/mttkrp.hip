@@ -1802,7 +1802,10 @@ static int run_plan(const Plan& p0, int x_dtype, const void* X, int ndim, const 
   }
   if (p.path == Path::Any && ws_bytes >= p.ws_bytes && (ws || p.ws_bytes == 0)) {
     any_plan(x_dtype == TLA_F64, ndim, shape, R, kb, weights != nullptr, &p.any);
-    return any_launch(x_dtype == TLA_F64, p.any, X, ndim, shape, factors, weights, R, kb, out, ws, st);
+    const bool takes = job && job->R > 0 && any_takes_job(p.any, R);
+    if (job_taken) *job_taken = takes;
+    return any_launch(x_dtype == TLA_F64, p.any, X, ndim, shape, factors, weights, R, kb, out, ws,
+                      takes ? job : nullptr, st);
   }
   // (a caller with less scratch than the plan's gets the vector kernel, which needs none)
   if (p.path == Path::Generic || p.path == Path::Any) {

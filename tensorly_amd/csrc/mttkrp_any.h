@@ -23,8 +23,12 @@ struct AnyPlan {
 // Fills *p and returns true when the kernels take this contraction.
 bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, bool weights, AnyPlan* p);
 
-// Runs it: factors and weights in the tensor's dtype, ws of any_plan's size.
+// Whether the launch takes a side job: its sum of partials is one launch.
+inline bool any_takes_job(const AnyPlan& p, int R) { return R <= 64 && p.nblk > 1; }
+
+// Runs it: factors and weights in the tensor's dtype, ws of any_plan's size;
+// job (nullable): a side job, only where any_takes_job.
 int any_launch(bool f64, const AnyPlan& p, const void* X, int ndim, const int64_t* shape, const void* const* factors,
-               const void* weights, int R, int mode, void* out, void* ws, hipStream_t st);
+               const void* weights, int R, int mode, void* out, void* ws, const InvJob* job, hipStream_t st);
 
 }  // namespace tla

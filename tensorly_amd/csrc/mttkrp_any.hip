@@ -29,6 +29,7 @@
 //   149 x 120 x 90,  R = 10, float32: 172 (mean) -> 8 / 8 / 11 us
 #include <algorithm>
 
+#include "inverse.h"
 #include "mma_any.h"
 #include "mttkrp_any.h"
 
@@ -351,9 +352,16 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
 // elements x 8 lanes of b per block.  In float64: the sums of a hundred
 // float32 partials would round more than all that came before (149 x 120 x 90,
 // positive data: relative error 5.2e-8 against 2.6e-8).
-template <typename T>
+// JOB: the grid's last block inverts the normal-equations matrix of the solve
+// that follows (inverse.h) instead, so that the solve need not (rank 10, 150
+// rows, sum and solve: 4.4 + 11.8 -> 6.4 + 7.9 us).
+template <typename T, bool JOB>
 __global__ __launch_bounds__(256) void any_reduce_kernel(const T* __restrict__ partial, int64_t n, int64_t nblk, int R,
-                                                         int64_t ldo, T* __restrict__ out) {
+                                                         int64_t ldo, T* __restrict__ out, InvJob job) {
+  if constexpr (JOB) {
+    extern __shared__ char job_lds[];
+    if (take_inv_job<256>(job, job_lds)) return;
+  }
   __shared__ double red[8][32];
   const int el = threadIdx.x & 31, bl = threadIdx.x >> 5;
   const int64_t e = (int64_t)blockIdx.x * 32 + el;
@@ -495,7 +503,7 @@ static void any_run_last(int TN, unsigned grid, const AnyLastArgs<T>& a, hipStre
 
 template <typename T>
 static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* shape, const void* const* factors,
-                        const T* weights, int R, int mode, T* out, void* ws, hipStream_t st) {
+                        const T* weights, int R, int mode, T* out, void* ws, const InvJob* job, hipStream_t st) {
   for (int m = 0; m < ndim; ++m) TLA_REQUIRE(m == mode || factors[m] != nullptr, "factor %d is NULL", m);
   // modes of the table: all but the output mode and the one the kernel reads itself
   const int own = p.last ? ndim - 2 : ndim - 1;
@@ -559,7 +567,16 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
     TLA_LAUNCH_CHECK();
     if (!direct) {
       const int64_t n = p.In * Rs;
-      any_reduce_kernel<T><<<(unsigned)((n + 31) / 32), 256, 0, st>>>(part, n, p.nblk, Rs, R, out + r0);
+      const unsigned blocks = (unsigned)((n + 31) / 32);
+      if (job) {
+        const size_t lds = inv_job_lds_bytes(job->R);
+        const auto kernel = any_reduce_kernel<T, true>;
+        if (lds > 64 * 1024)
+          TLA_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        kernel<<<blocks + 1, 256, lds, st>>>(part, n, p.nblk, Rs, R, out + r0, *job);
+      } else {
+        any_reduce_kernel<T, false><<<blocks, 256, 0, st>>>(part, n, p.nblk, Rs, R, out + r0, InvJob{});
+      }
       TLA_LAUNCH_CHECK();
     }
   }
@@ -567,11 +584,11 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
 }
 
 int any_launch(bool f64, const AnyPlan& p, const void* X, int ndim, const int64_t* shape, const void* const* factors,
-               const void* weights, int R, int mode, void* out, void* ws, hipStream_t st) {
+               const void* weights, int R, int mode, void* out, void* ws, const InvJob* job, hipStream_t st) {
   return f64 ? any_launch_t<double>(p, (const double*)X, ndim, shape, factors, (const double*)weights, R, mode,
-                                    (double*)out, ws, st)
+                                    (double*)out, ws, job, st)
              : any_launch_t<float>(p, (const float*)X, ndim, shape, factors, (const float*)weights, R, mode,
-                                   (float*)out, ws, st);
+                                   (float*)out, ws, job, st);
 }
 
 }  // namespace tla

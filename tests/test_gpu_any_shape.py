@@ -371,3 +371,23 @@ def test_gram64_edges(cuda, rows, rank, dtype):
     a = torch.randn(rows, rank, dtype=dtype, generator=torch.Generator().manual_seed(rows)).to(cuda)
     g, d = grams64([a])[0].cpu(), a.double().cpu()
     assert bool(((g - d.T @ d).abs() <= 2.3e-16 * (rows + 8) * (d.abs().T @ d.abs())).all())
+
+
+@pytest.mark.parametrize("rank", [1, 10, 17, 40, 64])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_parafac_any_shape_sweeps(cuda, rank, dtype):
+    """Two sweeps from given factors, the next solve's inverse formed beside
+    the sum of partials, against the normal equations in float64: cond(V) is
+    below 1e3 for such factors, times 100 eps for the sums."""
+    import tensorly_amd as tla
+    shape = (131, 145, 270)
+    x, F, _ = problem(cuda, shape, rank, dtype, rank)
+    got = tla.parafac(x, rank, n_iter_max=2, tol=0, init=(None, [f.clone() for f in F])).factors
+    D, xd = [f.double() for f in F], x.double()
+    for _ in range(2):
+        for m in range(3):
+            i, j = (k for k in range(3) if k != m)
+            D[m] = torch.linalg.solve((D[i].T @ D[i]) * (D[j].T @ D[j]), reference(xd, None, D, m).T).T
+    tol = 1e5 * torch.finfo(dtype).eps
+    for a, b in zip(got, D):
+        assert float((a.double() - b).norm() / b.norm()) < tol
