@@ -356,7 +356,7 @@ int tla_admm_update(int dtype, void* factor, double* x_split, double* dual, cons
  *   tla_mode_gram64: G = unfold(X, mode) unfold(X, mode)^T (I_mode^2 FP64),
  *                    without forming the unfolding.
  *   tla_sym_eig:     k leading eigenpairs (descending) of symmetric FP64 G
- *                    (n x n).  n <= 128: Jacobi on the whole matrix (any
+ *                    (n x n).  n <= 128: the whole matrix (a direct solver, any
  *                    k <= n); n > 128: subspace iteration with Rayleigh-Ritz,
  *                    block 48 / 64 / 128 for k <= 40 / 56 / 120 (larger k
  *                    returns TLA_ERR_UNSUPPORTED), optional warm start Q0
@@ -393,7 +393,7 @@ int tla_sym_eig_batch(int count, const double* const* G, const int* n, const int
  * HOOI step of the same mode, tensorly/decomposition/_tucker.py:194-202)
  * without re-orthonormalising it; 0 < k0 < b columns are a partial warm
  * start as for tla_sym_eig.  tla_gram_svd_block returns 0 where no block
- * exists (n <= 128: Jacobi on the whole matrix, W0 and W_out unused).
+ * exists (n <= 128: the whole matrix is solved, W0 and W_out unused).
  * Workspace: tla_sym_eig_workspace_size(n). */
 int tla_gram_svd_block(int n, int k);
 int tla_gram_left_singular(const double* G, int n, int k, const double* W0, int k0, int dtype, void* U,

@@ -1,5 +1,4 @@
-// FP64 symmetric eigensolver for the leading eigenpairs of a Gram matrix,
-// and the mode-n Gram G = unfold(X, n) unfold(X, n)^T.
+// FP64 symmetric eigensolver for the leading eigenpairs of a Gram matrix.
 //
 // These replace the LAPACK SVDs of tensorly/tenalg/svd.py:211-235
 // (truncated_svd) on the Tucker / CP-init path: the left singular vectors of
@@ -12,11 +11,12 @@
 //    in parallel).
 //  * n  > 128: block subspace iteration with Rayleigh-Ritz, block b = 48 for
 //    k <= 40, 64 for k <= 56 or 128 for k <= 120.  Each step: Z = G V, H = V^T Z on FP64
-//    MFMA, Jacobi(H) = W diag(t) W^T (warm: the previous Ritz basis nearly
-//    diagonalises H), Ritz vectors Y = V W and U = Z W = G Y, residuals of
-//    the k leading pairs, V <- orth(U) by two shifted Cholesky-QR passes
-//    (S = M^T M on MFMA, forward elimination of [S | I] in registers).
-//    Converged when every leading residual is below tol * t_1.
+//    MFMA, H = W diag(t) W^T (perturbation theory where the previous Ritz
+//    basis nearly diagonalises H, else the direct solver for block 48, else
+//    Jacobi), Ritz vectors Y = V W and U = Z W = G Y, residuals of the k
+//    leading pairs, V <- orth(U) by one Cholesky-QR pass or a shifted and a
+//    plain one (S = M^T M on MFMA, forward elimination of [S | I] in
+//    registers).  Converged when every leading residual is below tol * t_1.
 // One workgroup per problem; the padded np x b blocks live in the caller's
 // workspace (L2-resident).
 #include <math.h>
