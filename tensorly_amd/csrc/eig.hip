@@ -1472,9 +1472,11 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
       // panel staging area); else the direct solver (block 48, its scratch in
       // the staging area too); else Jacobi sweeps
       direct = false;
-      // (not twice in a row with what cannot end the iteration)
+      // (not twice in a row with what cannot end the iteration, nor in the
+      // last step allowed, whose vectors are returned whatever they are)
       if constexpr (B == 48)
-        pert = perturb_eigvecs<LDH, LDW>(H, W, B, k, stage, stage + B * k, scratch, pert == 1 ? 1e-5 : 1e-3);
+        pert = perturb_eigvecs<LDH, LDW>(H, W, B, k, stage, stage + B * k, scratch,
+                                         pert == 1 || it + 1 == a.max_iter ? 1e-5 : 1e-3);
       const bool sep = pert == 0 && k < B && lead_block_separated<LDH>(H, B, k, jthr, scratch);
       if constexpr (B == 48) {
         // (a separated leading block of few columns sweeps in less)

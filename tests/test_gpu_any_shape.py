@@ -391,3 +391,26 @@ def test_parafac_any_shape_sweeps(cuda, rank, dtype):
     tol = 1e5 * torch.finfo(dtype).eps
     for a, b in zip(got, D):
         assert float((a.double() - b).norm() / b.norm()) < tol
+
+
+@pytest.mark.parametrize("n,k", [(200, 5), (256, 24), (256, 32), (300, 40)])
+@pytest.mark.parametrize("move", [1e-2, 8e-4, 5e-4, 1e-4])
+@pytest.mark.parametrize("max_iter", [2, 3])
+def test_sym_eig_iteration_limit_returns_orthonormal_vectors(cuda, n, k, move, max_iter):
+    """A warm solve that the iteration limit ends: whatever step was the last,
+    its vectors are orthonormal (to 1e-11, as above) and its values are their
+    Ritz values.  The moves of 8e-4 and 5e-4 leave a Ritz matrix that second-order
+    perturbation would diagonalise to 1e-10 only."""
+    import numpy as np
+    from tensorly_amd.svd import gram_left_singular
+    rng = np.random.default_rng(n + k)
+    lam = np.concatenate([np.linspace(10.0, 2.0, k), rng.uniform(3e-3, 5e-3, n - k)])
+    q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+    a = (q * lam) @ q.T
+    d = rng.standard_normal((n, n))
+    b = a + move * (d + d.T) / np.sqrt(n)
+    _, _, blk = gram_left_singular(torch.tensor((a + a.T) / 2, device=cuda), k, torch.float64, want_block=True)
+    u, s, _ = gram_left_singular(torch.tensor(b, device=cuda), k, torch.float64, warm=blk, max_iter=max_iter)
+    u, w = u.cpu().numpy(), s.cpu().numpy() ** 2
+    assert np.max(np.abs(u.T @ u - np.eye(k))) < 1e-11
+    assert np.max(np.abs(np.einsum("ij,ik,kj->j", u, b, u) - w)) < 2e-10
