@@ -384,8 +384,8 @@ int tla_sym_eig_batch(int count, const double* const* G, const int* n, const int
  * the same launch: the k leading left singular vectors U (n x k, row-major,
  * dtype TLA_F32 / TLA_F64) of a matrix whose row Gram is G, with the sign
  * rule of svd_flip(u_based_decision=True) (tensorly/tenalg/svd.py:13-42:
- * each column times the sign of its entry of largest magnitude, the first
- * such row on ties), s = sqrt(max(eigenvalue, 0)) (k, dtype; nullable) and
+ * each column times the sign of its entry of largest magnitude in dtype, the
+ * first such row on ties), s = sqrt(max(eigenvalue, 0)) (k, dtype; nullable) and
  * U64 (the same vectors in FP64; nullable).  For n > 128,
  * tla_gram_svd_block(n, k) = b is the subspace block: W_out (n x b FP64,
  * nullable) receives the final block, and W0 = that block with k0 = b (it

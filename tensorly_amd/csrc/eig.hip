@@ -1054,7 +1054,9 @@ struct EigArgs {
 // without a map) of Ysrc (ld ldy) and theta[r].  evals / evecs as
 // tla_sym_eig writes them (when non-NULL); with a.flip the reference's
 // u-based sign rule first (each column multiplied by the sign of its entry
-// of largest magnitude, the first such row on ties; sgn: k doubles of LDS);
+// of largest magnitude, as rounded to the output's type, the first such row
+// on ties: entries that are equal but for the last bits of the solve do not
+// decide by those; sgn: k doubles of LDS);
 // u_out / s_out in a.out_dtype; with a.wblk the first nb columns of Ysrc.
 __device__ void eig_emit(const EigArgs& a, const double* Ysrc, int ldy, const int* colmap, const double* theta,
                          double* sgn, int nb) {
@@ -1065,7 +1067,8 @@ __device__ void eig_emit(const EigArgs& a, const double* Ysrc, int ldy, const in
       double best = -1.0;
       int bi = 0;
       for (int i = tid & 63; i < n; i += 64) {
-        const double v = fabs(Ysrc[i * ldy + c]);
+        double v = fabs(Ysrc[i * ldy + c]);
+        if (a.out_dtype == TLA_F32) v = (float)v;
         if (v > best) {
           best = v;
           bi = i;

@@ -414,3 +414,25 @@ def test_sym_eig_iteration_limit_returns_orthonormal_vectors(cuda, n, k, move, m
     u, w = u.cpu().numpy(), s.cpu().numpy() ** 2
     assert np.max(np.abs(u.T @ u - np.eye(k))) < 1e-11
     assert np.max(np.abs(np.einsum("ij,ik,kj->j", u, b, u) - w)) < 2e-10
+
+
+@pytest.mark.parametrize("half", [1, 2, 5, 16, 40])
+def test_svd_init_signs_of_tied_entries(cuda, half):
+    """Left singular vectors [u, u] and [u, -u], whose largest entries tie but
+    for the rounding of the solve: the sign rule looks at the vectors in the
+    tensor's type, where the first of equal entries decides, in the init as in
+    the SVD of one unfolding."""
+    from tensorly_amd.decomposition._cp import initialize_cp
+    from tensorly_amd.svd import svd_interface
+    g = torch.Generator().manual_seed(half)
+    a, b = (torch.randint(-8, 9, (half, 60), generator=g).float() for _ in range(2))
+    # rows i and half + i have the Gram of the pair swapped
+    x = torch.cat([torch.cat([a, b], 1), torch.cat([b, a], 1)], 0).reshape(2 * half, 12, 10).to(cuda)
+    rank = min(2 * half, 10)
+    U = initialize_cp(x, rank, init="svd")[1][0]
+    V, S, _ = svd_interface(x.reshape(2 * half, -1), n_eigenvecs=rank)
+    V = V[:, :rank] * S[:rank]
+    for r in range(rank):  # (columns of equal values may turn)
+        if all(abs(float(S[r] - S[q])) > 1e-3 * float(S[0]) for q in range(rank) if q != r):
+            assert float((U[:, r] - V[:, r]).norm()) < 1e-5 * float(S[0]), r
+            assert float(U[U[:, r].abs().argmax(), r]) > 0
