@@ -668,8 +668,9 @@ extern "C" int tla_mode_dot(int dtype, const void* X, int ndim, const int64_t* s
   }
   // everything else in the tensor's own arithmetic; precision "valu" and the
   // sizes that the matrix kernels do not index stay on the vector ALU
-  if ((dtype == TLA_F64 || precision != TLA_PREC_VALU) && ttm_any_ok(dtype == TLA_F64, Pa, Im, Pb, J))
-    return ttm_any_launch(dtype == TLA_F64, X, Pa, Im, Pb, U, ldj, ldm, J, out, st);
+  TtmPlan plan;
+  if ((dtype == TLA_F64 || precision != TLA_PREC_VALU) && ttm_any_plan(dtype == TLA_F64, Pa, Im, Pb, J, &plan))
+    return ttm_any_launch(dtype == TLA_F64, plan, X, Pa, Im, Pb, U, ldj, ldm, J, out, st);
   if (dtype == TLA_F32)
     ttm_generic_kernel<float><<<ceil_div(ne, 256), 256, 0, st>>>((const float*)X, Pa, Im, Pb, (const float*)U, J,
                                                                  ldj, ldm, (float*)out);

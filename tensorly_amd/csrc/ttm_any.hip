@@ -19,14 +19,10 @@
 // Odd sizes, more than 64 rows j and float64 ran one thread per output
 // element, which read X once per row j: 250 x 331 x 190 to 25 x 30 x 20 and
 // back 772 -> 89 us.
-#include <algorithm>
-
 #include "mma_any.h"
 #include "ttm_any.h"
 
 namespace tla {
-
-constexpr int kTtmWaves = 4;
 
 template <typename T>
 struct TtmAnyArgs {
@@ -234,65 +230,37 @@ __global__ __launch_bounds__(64 * kTtmWaves, 2) void ttm_any_rows_kernel(TtmAnyA
 }
 
 template <typename T, int JT>
-static void ttm_any_run(const TtmAnyArgs<T>& a0, hipStream_t st) {
-  constexpr int VL = AnyT<T>::V;
-  TtmAnyArgs<T> a = a0;
-  const unsigned gy = (unsigned)((a.J + 16 * JT - 1) / (16 * JT));
+static void ttm_any_run(const TtmPlan& p, const TtmAnyArgs<T>& a, hipStream_t st) {
+  const dim3 grid((unsigned)p.gx, (unsigned)p.gy);
+  constexpr int TNR = JT <= 2 ? 4 : 2, TNC = JT <= 2 ? 2 : 1;
   if (a.Pb == 1) {
-    const int64_t tiles = (a.Pa + 15) / 16;
-    // more tiles per wave share the rows of U, fewer fill the GPU
-    constexpr int TNR = JT <= 2 ? 4 : 2;
-    if (tiles * gy >= TNR * 4096) {
-      const int64_t w = kTtmWaves * TNR;
-      ttm_any_rows_kernel<T, TNR, JT><<<dim3((unsigned)((tiles + w - 1) / w), gy), 64 * kTtmWaves, 0, st>>>(a);
-    } else {
-      ttm_any_rows_kernel<T, 1, JT><<<dim3((unsigned)((tiles + 3) / 4), gy), 64 * kTtmWaves, 0, st>>>(a);
-    }
-    return;
+    if (p.TN == 1) ttm_any_rows_kernel<T, 1, JT><<<grid, 64 * kTtmWaves, 0, st>>>(a);
+    else ttm_any_rows_kernel<T, TNR, JT><<<grid, 64 * kTtmWaves, 0, st>>>(a);
+  } else {
+    if (p.TN == 1) ttm_any_cols_kernel<T, 1, JT><<<grid, 64 * kTtmWaves, 0, st>>>(a);
+    else ttm_any_cols_kernel<T, TNC, JT><<<grid, 64 * kTtmWaves, 0, st>>>(a);
   }
-  constexpr int TNL = JT <= 2 ? 2 : 1;  // accumulators of TNL tiles fit the register file
-  const int64_t narrow = (a.Pb + 16 * VL - 1) / (16 * VL), wide = (a.Pb + 16 * VL * TNL - 1) / (16 * VL * TNL);
-  const bool one = a.Pa * wide * gy < 4096;
-  a.tiles = one ? narrow : wide;
-  const int64_t tiles = a.Pa * a.tiles;
-  a.split = tiles * gy < 4096 && a.Im > 32 ? 1 : 0;
-  const dim3 grid((unsigned)(a.split ? tiles : (tiles + kTtmWaves - 1) / kTtmWaves), gy);
-  if (one) ttm_any_cols_kernel<T, 1, JT><<<grid, 64 * kTtmWaves, 0, st>>>(a);
-  else ttm_any_cols_kernel<T, TNL, JT><<<grid, 64 * kTtmWaves, 0, st>>>(a);
 }
 
 template <typename T>
-static int ttm_any_t(const TtmAnyArgs<T>& a, hipStream_t st) {
-  const int64_t jt = std::min<int64_t>((a.J + 15) / 16, 4);
-  // J > 64: groups of 16 jt rows with the least padding
-  int best = (int)jt;
-  if (a.J > 64)
-    for (int t = 3; t >= 2; --t)
-      if ((a.J + 16 * t - 1) / (16 * t) * t < (a.J + 16 * best - 1) / (16 * best) * best) best = t;
-  switch (best) {
-    case 1: ttm_any_run<T, 1>(a, st); break;
-    case 2: ttm_any_run<T, 2>(a, st); break;
-    case 3: ttm_any_run<T, 3>(a, st); break;
-    default: ttm_any_run<T, 4>(a, st); break;
+static int ttm_any_t(const TtmPlan& p, TtmAnyArgs<T> a, hipStream_t st) {
+  a.tiles = p.tiles;
+  a.split = p.split;
+  switch (p.JT) {
+    case 1: ttm_any_run<T, 1>(p, a, st); break;
+    case 2: ttm_any_run<T, 2>(p, a, st); break;
+    case 3: ttm_any_run<T, 3>(p, a, st); break;
+    default: ttm_any_run<T, 4>(p, a, st); break;
   }
   TLA_LAUNCH_CHECK();
   return TLA_OK;
 }
 
-bool ttm_any_ok(bool f64, int64_t Pa, int64_t Im, int64_t Pb, int64_t J) {
-  constexpr int64_t kBig = 0x7fffff00;
-  const int sz = f64 ? 8 : 4;
-  if (Pb > 1 && Pb < (f64 ? 2 : 4)) return false;
-  // 32-bit indices: m, the bytes of 16 rows (cols) or 64 rows (rows) of X; the grid
-  if (Im > kBig / (64 * sz) || Pb > kBig / (16 * sz) || J > 16 * 65535) return false;
-  if (Pb == 1) return Pa <= kBig * 16;
-  return Pa <= kBig && (Pb + 31) / 32 <= kBig / Pa;
-}
-
-int ttm_any_launch(bool f64, const void* X, int64_t Pa, int64_t Im, int64_t Pb, const void* U, int64_t ldj,
-                   int64_t ldm, int64_t J, void* out, hipStream_t st) {
-  if (f64) return ttm_any_t<double>({(const double*)X, Pa, Im, Pb, (const double*)U, ldj, ldm, J, (double*)out, 0, 0}, st);
-  return ttm_any_t<float>({(const float*)X, Pa, Im, Pb, (const float*)U, ldj, ldm, J, (float*)out, 0, 0}, st);
+int ttm_any_launch(bool f64, const TtmPlan& p, const void* X, int64_t Pa, int64_t Im, int64_t Pb, const void* U,
+                   int64_t ldj, int64_t ldm, int64_t J, void* out, hipStream_t st) {
+  if (f64)
+    return ttm_any_t<double>(p, {(const double*)X, Pa, Im, Pb, (const double*)U, ldj, ldm, J, (double*)out, 0, 0}, st);
+  return ttm_any_t<float>(p, {(const float*)X, Pa, Im, Pb, (const float*)U, ldj, ldm, J, (float*)out, 0, 0}, st);
 }
 
 }  // namespace tla

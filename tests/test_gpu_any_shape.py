@@ -436,3 +436,16 @@ def test_svd_init_signs_of_tied_entries(cuda, half):
         if all(abs(float(S[r] - S[q])) > 1e-3 * float(S[0]) for q in range(rank) if q != r):
             assert float((U[:, r] - V[:, r]).norm()) < 1e-5 * float(S[0]), r
             assert float(U[U[:, r].abs().argmax(), r]) > 0
+
+
+@pytest.mark.parametrize("shape", [(70_000_000, 2, 4), (67_108_864, 4, 4)])
+def test_mode_dot_past_the_tiles_of_a_launch(cuda, shape):
+    """More short runs than one launch has tiles for (2.2 and 4.3 GB): sums of
+    two and four products."""
+    import tensorly_amd as tla
+    X = torch.arange(shape[0], device=cuda, dtype=torch.float32).remainder_(1024)[:, None, None].expand(shape).contiguous()
+    U = torch.tensor([[1.0, 2.0, 4.0, 8.0][: shape[1]], [3.0, 5.0, 7.0, 9.0][: shape[1]]], device=cuda)
+    for J in (1, 2):
+        out = tla.mode_dot(X, U[:J], 1)
+        for j in range(J):
+            assert bool((out[:, j] == X[:, 0] * U[j].sum()).all())
