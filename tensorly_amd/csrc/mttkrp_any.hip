@@ -35,20 +35,6 @@
 
 namespace tla {
 
-constexpr int kAnyWaves = 4;
-
-// rows per lane of one visit of any_last_kernel
-__host__ __device__ constexpr int any_last_rows(int TN, int RT) { return TN > 1 || RT > 1 ? 4 : 8; }
-// Waves per SIMD that a kernel's registers are cut for: two sets of loaded
-// values, the factor rows, the accumulators and some 40 for addresses.
-__host__ __device__ constexpr int any_occ(int TN, int RT, bool last, bool f64) {
-  const int d = f64 ? 2 : 1;
-  const int nr = any_last_rows(TN, RT);
-  const int regs = last ? 8 * TN * nr + 16 * TN * RT + d * RT * (nr + 2) + (RT == 4 ? 56 : 40)
-                        : 16 * TN + 4 * d * TN * RT + (8 + 2 * d) * RT + (f64 ? 54 : 40);
-  return regs <= 128 ? 4 : regs <= 168 ? 3 : 2;
-}
-
 // G[q, r] = w[r] * product over the listed modes' factor rows (q row-major
 // over those modes).
 template <typename T>
@@ -81,12 +67,14 @@ struct AnyRowsArgs {
   int64_t In, Q;
   int K, Pb;
   int R, ldr;       // columns of this slab, row stride of the factors
-  const T* G;       // (A Pb) x ldr, nullable
+  const T* G;       // rows g0, ... of the A Pb scale rows, nullable
+  int64_t g0;
+  int ldg;
   AnyGArgs<T> ga;   // GD: the factors of G instead
   const T* Fk;      // K x ldr
   T* partial;       // [nblk][In][R]
   int nqc;
-  int64_t nchunks, nblk;
+  int64_t first, nchunks, nblk;  // chunks [first, nchunks)
 };
 
 // GD: every wave forms its scale rows from the factors (small problems, where
@@ -100,7 +88,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int64_t grp = blockIdx.x / a.nblk, blk = blockIdx.x - grp * a.nblk;
-  const int K = a.K, R = a.R, ldr = a.ldr;
+  const int K = a.K, R = a.R;
   const int64_t Q = a.Q, In = a.In, i0 = grp * (16 * TN);
   // rows past the mode's end read its last row; their results are dropped
   uint32_t roff[TN];  // bytes
@@ -110,7 +98,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
   uint32_t rr[RT];  // rank columns, in bytes; those past the slab read its last one
 #pragma unroll
   for (int n = 0; n < RT; ++n) rr[n] = min(n * 16 + c, R - 1) * sizeof(T);
-  const uint32_t ldb = ldr * sizeof(T);
+  const uint32_t ldb = a.ldr * sizeof(T), ldgb = a.ldg * sizeof(T);
   Acc acc[TN * RT];
 #pragma unroll
   for (int n = 0; n < TN * RT; ++n) acc[n] = Acc{0, 0, 0, 0};
@@ -147,10 +135,10 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
     const int q = left > 0 ? q0 + NV * g : (int)Q - 1;
     const int b0 = q / K;
     int k0 = q - b0 * K;
-    const T* Gb = !GD && a.G ? a.G + ia * a.Pb * ldr : nullptr;
+    const T* Gb = !GD && a.G ? a.G + (ia * a.Pb - a.g0) * a.ldg : nullptr;
     auto scale = [&](int b, uint32_t rb) -> T {
       if constexpr (GD) return g_entry(a.ga, (uint32_t)ia * a.Pb + b, rb, ldb);
-      else return Gb ? at<T>(Gb, b * ldb + rb) : (T)1;
+      else return Gb ? at<T>(Gb, b * ldgb + rb) : (T)1;
     };
     if (K >= NV) {
       const int b1 = min(b0 + 1, a.Pb - 1);
@@ -188,7 +176,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
 #pragma unroll
         for (int n = 0; n < RT; ++n) acc[t * RT + n] = AnyT<T>::mma(x[t][v], f[n][v], acc[t * RT + n]);
   };
-  int64_t ch = blk * kAnyWaves + wave;
+  int64_t ch = a.first + blk * kAnyWaves + wave;
   T x0[TN][NV], x1[TN][NV];
   if (ch < a.nchunks) load(ch, x0);
   while (ch < a.nchunks) {
@@ -216,11 +204,12 @@ struct AnyLastArgs {
   int64_t P, K;
   int J, nG;    // P = nG J
   int R, ldr;
-  const T* G;   // (P / J) x ldr, nullable
+  const T* G;   // rows g0, ... of the P / J scale rows, nullable
+  int g0, ldg;
   AnyGArgs<T> ga;  // GD: the factors of G instead
   const T* Fj;  // J x ldr
   T* partial;   // [nblk][K][R]
-  int64_t nvisits, nblk;
+  int64_t first, nvisits, nblk;  // visits [first, nvisits)
 };
 
 template <typename T, int TN, int RT, bool GD = false>
@@ -234,7 +223,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int64_t grp = blockIdx.x / a.nblk, blk = blockIdx.x - grp * a.nblk;
-  const int R = a.R, ldr = a.ldr, J = a.J;
+  const int R = a.R, J = a.J;
   const int64_t K = a.K, k0 = grp * (16 * VL * TN);
   // lanes that would read past the row's end read its last 16 bytes (and
   // write those columns, with the same values as the lane they belong to)
@@ -247,7 +236,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
   uint32_t rr[RT];  // rank columns, in bytes; those past the slab read its last one
 #pragma unroll
   for (int n = 0; n < RT; ++n) rr[n] = min(n * 16 + c, R - 1) * sizeof(T);
-  const uint32_t ldb = ldr * sizeof(T);
+  const uint32_t ldb = a.ldr * sizeof(T), ldgb = a.ldg * sizeof(T);
   Acc acc[TN * VL * RT];
 #pragma unroll
   for (int n = 0; n < TN * VL * RT; ++n) acc[n] = Acc{0, 0, 0, 0};
@@ -282,7 +271,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
     int j0 = (int)(p - (uint32_t)a0 * J);
     auto scale = [&](int i, uint32_t rb) -> T {
       if constexpr (GD) return g_entry(a.ga, (uint32_t)i, rb, ldb);
-      else return a.G ? at<T>(a.G, i * ldb + rb) : (T)1;
+      else return a.G ? at<T>(a.G, (i - a.g0) * ldgb + rb) : (T)1;
     };
     if (J >= NR) {
       const int a1 = min(a0 + 1, a.nG - 1);
@@ -325,7 +314,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
             d = AnyT<T>::mma(f[n][u], x[u][t][e], d);
           }
   };
-  int v = (int)blk * kAnyWaves + wave;
+  int v = (int)(a.first + blk * kAnyWaves) + wave;
   V x0[NR][TN], x1[NR][TN];
   if (v < nv) load(v, x0);
   while (v < nv) {
@@ -387,12 +376,13 @@ __global__ __launch_bounds__(256) void any_reduce_kernel(const T* __restrict__ p
   }
 }
 
+// Rows g0, ... of the table, ld columns of the factors' R.
 template <typename T>
-__global__ void any_g_kernel(AnyGArgs<T> a, T* __restrict__ out) {
+__global__ void any_g_kernel(AnyGArgs<T> a, int64_t g0, int ld, T* __restrict__ out) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= a.rows * a.R) return;
-  const int r = (int)(e % a.R);
-  int64_t q = e / a.R;
+  if (e >= a.rows * ld) return;
+  const int r = (int)(e % ld);
+  int64_t q = g0 + e / ld;
   T v = a.weights ? a.weights[r] : (T)1;
 #pragma unroll
   for (int m = kMaxOrder - 1; m >= 0; --m)
@@ -402,81 +392,6 @@ __global__ void any_g_kernel(AnyGArgs<T> a, T* __restrict__ out) {
       v *= a.fac[m][i * a.R + r];
     }
   out[e] = v;
-}
-
-static size_t any_align(size_t b) { return (b + 255) & ~size_t(255); }
-
-bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, bool weights, AnyPlan* p) {
-  *p = AnyPlan{};
-  const int V = f64 ? 2 : 4, sz = f64 ? 8 : 4;
-  const int Rs = std::min(R, 64);
-  p->RT = (Rs + 15) / 16;
-  p->last = mode == ndim - 1;
-  p->K = shape[ndim - 1];
-  p->In = shape[mode];
-  p->A = 1;
-  p->Q = 1;
-  for (int m = 0; m < mode; ++m) p->A *= shape[m];
-  for (int m = mode + 1; m < ndim; ++m) p->Q *= shape[m];
-  // the kernels' 32-bit indices: q or p, an element of a factor or of the
-  // scale rows of one a, a byte within the rows of a wave's tiles
-  constexpr int64_t kBig = 0x7fffff00;
-  for (int m = 0; m < ndim; ++m)
-    if (shape[m] > kBig / (R * sz)) return false;
-  int64_t tiles;
-  int most;  // tiles per wave that the registers hold
-  if (p->last) {
-    if (p->K < V) return false;
-    p->J = shape[ndim - 2];
-    p->g_rows = p->A / p->J;
-    if (p->A > kBig || p->g_rows > kBig / (R * sz) || p->K > kBig / (32 * sz)) return false;
-    tiles = (p->K + 16 * V - 1) / (16 * V);
-    most = p->RT == 1 ? 3 : p->RT == 2 ? 2 : 1;
-  } else {
-    p->Pb = p->Q / p->K;
-    if (p->Q > kBig / (32 * sz) || p->Pb > kBig / (R * sz)) return false;
-    p->g_rows = p->A * p->Pb;
-    p->nqc = (int)((p->Q + 8 * V - 1) / (8 * V));
-    tiles = (p->In + 15) / 16;
-    most = !f64 || p->RT <= 2 ? 4 : p->RT == 3 ? 3 : 2;
-  }
-  // Tiles per wave: every wave forms its part of B once for all its tiles
-  // (about the cost of one more tile), and the chunks are dealt to the waves
-  // that fit the GPU at once in equal numbers: the least sum over a wave's
-  // chunks wins.
-  int64_t best = -1;
-  for (int tn = most; tn >= 1; --tn) {
-    const int64_t groups = (tiles + tn - 1) / tn;
-    const int TN = (int)((tiles + groups - 1) / groups);
-    const int RV = 4 * any_last_rows(TN, p->RT);
-    const int64_t chunks = p->last ? (p->A + RV - 1) / RV : p->A * p->nqc;
-    const int64_t waves = std::max<int64_t>(1, 256 * 4 * any_occ(TN, p->RT, p->last, f64) / groups);
-    const int64_t per = (chunks + waves - 1) / waves;
-    const int64_t cost = per * (TN + 1) * (p->last ? RV : 16);
-    if (best >= 0 && cost >= best) continue;
-    best = cost;
-    p->TN = TN;
-    p->groups = groups;
-    p->nchunks = chunks;
-    p->nblk = (chunks + kAnyWaves * per - 1) / (kAnyWaves * per);
-  }
-  if (ndim == 2) p->g_rows = 0;
-  // the table is a factor as it is when it covers one mode and no weights
-  p->build_g = p->g_rows > 0 && !(ndim == 3 && !weights);
-  // Small problems are short of launches, not of work: up to 24 chunks, a few
-  // per wave, one workgroup per group writes the output itself (5 us, where
-  // the sum of partials is another launch of 3 us on the host and 2.5 us on
-  // the GPU); up to 1024 chunks, a fraction of the GPU's waves, the scale
-  // rows are formed in place of a table (one launch of 3 us).
-  p->direct_g = p->build_g && p->TN == 1 && p->nchunks * p->groups <= 1024 && p->g_rows <= kBig;
-  if (p->nchunks <= 24) p->nblk = 1;
-  // bounded scratch: at most 32 MiB of partial sums (one set: written to the output)
-  const int64_t set = p->In * Rs * sz;
-  p->nblk = std::max<int64_t>(1, std::min<int64_t>(p->nblk, (int64_t(32) << 20) / set));
-  if (p->groups * p->nblk > kBig) return false;
-  p->ws_bytes = (p->build_g && !p->direct_g ? any_align(size_t(p->g_rows) * R * sz) : 0) +
-                (p->nblk > 1 || R > 64 ? any_align(size_t(p->nblk) * set) : 0);
-  return true;
 }
 
 template <typename T, int RT>
@@ -507,64 +422,80 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
   for (int m = 0; m < ndim; ++m) TLA_REQUIRE(m == mode || factors[m] != nullptr, "factor %d is NULL", m);
   // modes of the table: all but the output mode and the one the kernel reads itself
   const int own = p.last ? ndim - 2 : ndim - 1;
-  const T* G = nullptr;
   AnyGArgs<T> ga{};
-  char* w = (char*)ws;
   if (p.g_rows > 0) {
     ga.R = R;
     ga.weights = weights;
-    ga.rows = p.g_rows;
     for (int m = 0; m < ndim; ++m)
       if (m != mode && m != own) {
         ga.sz[ga.n] = shape[m];
         ga.fac[ga.n++] = (const T*)factors[m];
       }
-    if (p.direct_g) {
-      // (the kernels take it from ga)
-    } else if (p.build_g) {
-      const int64_t ne = p.g_rows * R;
-      TLA_REQUIRE(ne <= int64_t(0x7fffffff) * 256, "scale table too large");
-      any_g_kernel<T><<<(unsigned)((ne + 255) / 256), 256, 0, st>>>(ga, (T*)w);
-      TLA_LAUNCH_CHECK();
-      G = (const T*)w;
-      w += any_align(size_t(ne) * sizeof(T));
-    } else {
-      G = ga.fac[0];
-    }
   }
+  const bool table = p.build_g && !p.direct_g;
+  const int64_t sets = p.nblk * p.slices;
   const unsigned grid = (unsigned)(p.groups * p.nblk);
   for (int r0 = 0; r0 < R; r0 += 64) {
     const int Rs = std::min(64, R - r0), RT = (Rs + 15) / 16;
-    const bool direct = p.nblk == 1 && Rs == R;
-    T* part = direct ? out : (T*)w;
-    const T* Gs = G ? G + r0 : nullptr;
-    AnyGArgs<T> gs{};  // of this slab's columns; R = 0: not used
-    if (p.direct_g) {
-      gs = ga;
-      if (gs.weights) gs.weights += r0;
-      for (int m = 0; m < gs.n; ++m) gs.fac[m] += r0;
-    }
-    if (p.last) {
-      const int RV = 4 * any_last_rows(p.TN, RT);
-      AnyLastArgs<T> a{X,    p.A, p.K, (int)p.J, (int)(p.A / p.J), Rs, R, Gs, gs, (const T*)factors[own] + r0,
-                       part, (p.A + RV - 1) / RV, p.nblk};
-      switch (RT) {
-        case 1: any_run_last<T, 1>(p.TN, grid, a, st); break;
-        case 2: any_run_last<T, 2>(p.TN, grid, a, st); break;
-        case 3: any_run_last<T, 3>(p.TN, grid, a, st); break;
-        default: any_run_last<T, 4>(p.TN, grid, a, st); break;
+    const bool direct = sets == 1 && Rs == R;
+    T* const sums = direct ? out : (T*)((char*)ws + (table ? any_align(size_t(p.g_slice) * std::min(R, 64) * sizeof(T)) : 0));
+    AnyGArgs<T> gs = ga;  // of this slab's columns
+    if (gs.weights) gs.weights += r0;
+    for (int m = 0; m < gs.n; ++m) gs.fac[m] += r0;
+    const int RV = 4 * any_last_rows(p.TN, RT);
+    const int64_t chunks = p.last ? (p.A + RV - 1) / RV : p.nchunks;
+    const int64_t per = chunks == p.nchunks ? p.per : (chunks + p.slices - 1) / p.slices;
+    for (int64_t s = 0; s < p.slices; ++s) {
+      const int64_t c0 = std::min(chunks, s * per), c1 = std::min(chunks, c0 + per);
+      T* part = sums + s * p.nblk * p.In * Rs;
+      const T* G = nullptr;
+      int64_t g0 = 0;
+      int ldg = R;
+      if (table) {
+        // the rows of chunks c0, ..., c1 - 1 and the one after
+        int64_t g1 = p.g_rows;
+        if (p.slices > 1 && c0 < c1) {
+          if (p.last) {
+            g0 = c0 * RV / p.J;
+            g1 = std::min(p.g_rows, (c1 * RV - 1) / p.J + 2);
+          } else {
+            constexpr int CH = 8 * AnyT<T>::V;
+            g0 = c0 / p.nqc * p.Pb + c0 % p.nqc * CH / p.K;
+            g1 = (c1 - 1) / p.nqc * p.Pb + std::min(((c1 - 1) % p.nqc + 1) * CH / p.K + 2, p.Pb);
+          }
+        }
+        TLA_REQUIRE(g1 - g0 <= p.g_slice, "scale table of %lld rows", (long long)(g1 - g0));
+        gs.rows = g1 - g0;
+        ldg = Rs;
+        const int64_t ne = gs.rows * Rs;
+        any_g_kernel<T><<<(unsigned)((ne + 255) / 256), 256, 0, st>>>(gs, g0, Rs, (T*)ws);
+        TLA_LAUNCH_CHECK();
+        G = (const T*)ws;
+      } else if (p.g_rows > 0 && !p.direct_g) {
+        G = gs.fac[0];
       }
-    } else {
-      AnyRowsArgs<T> a{X, p.In, p.Q, (int)p.K, (int)p.Pb, Rs, R, Gs, gs, (const T*)factors[own] + r0, part, p.nqc,
-                       p.nchunks, p.nblk};
-      switch (RT) {
-        case 1: any_run_rows<T, 1>(p.TN, grid, a, st); break;
-        case 2: any_run_rows<T, 2>(p.TN, grid, a, st); break;
-        case 3: any_run_rows<T, 3>(p.TN, grid, a, st); break;
-        default: any_run_rows<T, 4>(p.TN, grid, a, st); break;
+      const AnyGArgs<T> gd = p.direct_g ? gs : AnyGArgs<T>{};  // R = 0: not used
+      if (p.last) {
+        AnyLastArgs<T> a{X,  p.A, p.K,  (int)p.J, (int)(p.A / p.J), Rs, R, G, (int)g0, ldg, gd,
+                         (const T*)factors[own] + r0, part, c0, c1, p.nblk};
+        switch (RT) {
+          case 1: any_run_last<T, 1>(p.TN, grid, a, st); break;
+          case 2: any_run_last<T, 2>(p.TN, grid, a, st); break;
+          case 3: any_run_last<T, 3>(p.TN, grid, a, st); break;
+          default: any_run_last<T, 4>(p.TN, grid, a, st); break;
+        }
+      } else {
+        AnyRowsArgs<T> a{X, p.In, p.Q, (int)p.K, (int)p.Pb, Rs, R, G, g0, ldg, gd, (const T*)factors[own] + r0, part,
+                         p.nqc, c0, c1, p.nblk};
+        switch (RT) {
+          case 1: any_run_rows<T, 1>(p.TN, grid, a, st); break;
+          case 2: any_run_rows<T, 2>(p.TN, grid, a, st); break;
+          case 3: any_run_rows<T, 3>(p.TN, grid, a, st); break;
+          default: any_run_rows<T, 4>(p.TN, grid, a, st); break;
+        }
       }
+      TLA_LAUNCH_CHECK();
     }
-    TLA_LAUNCH_CHECK();
     if (!direct) {
       const int64_t n = p.In * Rs;
       const unsigned blocks = (unsigned)((n + 31) / 32);
@@ -573,9 +504,9 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
         const auto kernel = any_reduce_kernel<T, true>;
         if (lds > 64 * 1024)
           TLA_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        kernel<<<blocks + 1, 256, lds, st>>>(part, n, p.nblk, Rs, R, out + r0, *job);
+        kernel<<<blocks + 1, 256, lds, st>>>(sums, n, sets, Rs, R, out + r0, *job);
       } else {
-        any_reduce_kernel<T, false><<<blocks, 256, 0, st>>>(part, n, p.nblk, Rs, R, out + r0, InvJob{});
+        any_reduce_kernel<T, false><<<blocks, 256, 0, st>>>(sums, n, sets, Rs, R, out + r0, InvJob{});
       }
       TLA_LAUNCH_CHECK();
     }

@@ -449,3 +449,33 @@ def test_mode_dot_past_the_tiles_of_a_launch(cuda, shape):
         out = tla.mode_dot(X, U[:J], 1)
         for j in range(J):
             assert bool((out[:, j] == X[:, 0] * U[j].sum()).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape,rank,mode", [((3, 1200, 1001, 8), 64, 0), ((5, 1100, 1301, 6), 50, 0), ((1100, 1001, 3, 3), 64, 2),
+                                             ((1100, 1009, 2, 5), 64, 3), ((1100, 2003, 3, 5), 100, 3),
+                                             ((2, 3001, 3, 166, 4), 70, 0), ((3, 1_100_003, 5), 64, 0),
+                                             ((1500, 4, 901, 3), 64, 1)])
+def test_mttkrp_any_shape_scale_rows_in_slices(cuda, shape, rank, mode, dtype):
+    """Output and contiguous mode both short: a table of the other modes'
+    scale rows would be larger than the tensor, and is made 256 MiB at a time.
+    Sums of up to 9.6 million terms in chains of at most a hundredth of them:
+    sqrt(q / 100) eps.  The reference's own float64 sums are taken 4,096 terms
+    at a time and those added up pairwise."""
+    import tensorly_amd as tla
+    from tensorly_amd import _lib
+    X, F, w = problem(cuda, shape, rank, dtype, rank)
+    n, size = X.numel(), X.element_size()
+    sh, _k = _lib.shape_array(shape)
+    ws = _lib.lib().tla_mttkrp_workspace_size(_lib.dtype_code(X), len(shape), sh, rank, mode, _lib.PREC_FP32)
+    assert ws <= (256 << 20) + (32 << 20) + 512
+    for weights in (None, w):
+        out = tla.unfolding_dot_khatri_rao(X, (weights, F), mode)
+        k = w.double()[None, :] if weights is not None else torch.ones((1, rank), dtype=torch.float64, device=cuda)
+        for m, f in enumerate(F):
+            if m != mode:
+                k = (k[:, None, :] * f.double()[None, :, :]).reshape(-1, rank)
+        u = torch.movedim(X.double(), mode, 0).reshape(shape[mode], -1)
+        ref = torch.stack([u[:, q : q + 4096] @ k[q : q + 4096] for q in range(0, u.shape[1], 4096)], -1).sum(-1)
+        err = float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref))
+        assert err < max(1.0, 0.05 * (n / shape[mode]) ** 0.5 / 16) * TOL[dtype], err

@@ -26,6 +26,27 @@ int main() {
 """
 
 
+ANY = r"""
+#include <cstdio>
+#include "mttkrp_any_plan.h"
+int main() {
+  long long f64, R, mode, weights, n;
+  while (std::scanf("%lld %lld %lld %lld %lld", &f64, &R, &mode, &weights, &n) == 5) {
+    int64_t shape[8];
+    for (int m = 0; m < n; ++m) {
+      long long s = 0;
+      if (std::scanf("%lld", &s) != 1) return 1;
+      shape[m] = s;
+    }
+    tla::AnyPlan p;
+    const bool ok = tla::any_plan(f64, n, shape, R, mode, weights, &p);
+    std::printf("%d %d %d %d %lld %lld %lld %lld %d %d %zu\n", ok, p.last, p.TN, p.RT, (long long)p.groups,
+                (long long)p.slices, (long long)p.nblk, (long long)p.nchunks, p.build_g, p.direct_g, p.ws_bytes);
+  }
+}
+"""
+
+
 def compiled(tmp_path_factory, name, text):
     d = tmp_path_factory.mktemp(name)
     src, exe = d / "main.cpp", d / "main"
@@ -74,3 +95,48 @@ def test_mode_dot_plans_cover_every_output(ttm_plan):
             assert p["TN"] in ((1, 2) if p["JT"] <= 2 else (1,))
             assert p["tiles"] * 16 * (2 if f64 else 4) * p["TN"] >= Pb
             assert p["gx"] * (1 if p["split"] else 4) >= Pa * p["tiles"]
+
+
+@pytest.fixture(scope="module")
+def any_plan(tmp_path_factory):
+    ask = compiled(tmp_path_factory, "any", ANY)
+    keys = ("ok", "last", "TN", "RT", "groups", "slices", "nblk", "nchunks", "build_g", "direct_g", "ws")
+    return lambda rows: [dict(zip(keys, r)) for r in ask([(f, R, m, w, len(s), *s) for f, s, R, m, w in rows])]
+
+
+def _shapes(rng, count, most):
+    for _ in range(count):
+        nd = rng.choice([2, 3, 3, 4, 4, 5, 6])
+        side = 2 ** (rng.uniform(3, most) / nd)
+        s = [max(1, int(side * 2 ** rng.uniform(-most / 4, most / 4))) for _ in range(nd)]
+        for m in range(nd):
+            yield rng.random() < 0.5, s, rng.choice([1, 7, 16, 33, 64, 65, 200]), m, rng.random() < 0.5
+
+
+def test_mttkrp_scratch_is_bounded(any_plan):
+    """Scale rows: at most 256 MiB; partial sums: 32 MiB, or one set of a rank
+    slab for each slice of the scale rows (past rank 64, for one); and a call
+    without weights needs no more than the query said."""
+    rng = random.Random(3)
+    rows = [(0, s, 64, 0, 1) for s in ((2, 8192, 8192, 2), (6, 4096, 682, 8))]
+    rows += [(0, (4096, 4096, 4, 6), 64, 2, 1), (0, (2000, 4096, 4, 6), 64, 3, 1)]
+    rows += list(_shapes(rng, 1500, 38))
+    plans = any_plan(rows)
+    bare = any_plan([(f, s, R, m, 0) for f, s, R, m, _ in rows])
+    full = any_plan([(f, s, R, m, 1) for f, s, R, m, _ in rows])
+    for (f, s, R, m, _), p, b, w in zip(rows, plans, bare, full):
+        if p["ok"]:
+            assert p["ws"] <= (256 << 20) + max(32 << 20, p["slices"] * s[m] * 64 * (8 if f else 4)) + 512, (f, s, R, m, p)
+        assert b["ok"] == w["ok"] and b["ws"] <= w["ws"], (f, s, R, m)
+    assert [p["slices"] for p in plans[2:4]] == [16, 8]
+
+
+def test_mttkrp_grids_fit_a_launch(any_plan):
+    rng = random.Random(4)
+    rows = [(0, (500_000_000, 2, 2), 1, 0, 1), (0, (2 ** 28, 4), 1, 0, 1)] + list(_shapes(rng, 1500, 50))
+    for row, p in zip(rows, any_plan(rows)):
+        if p["ok"]:
+            rows_out = row[1][row[3]]
+            assert 0 < p["groups"] * p["nblk"] * 256 <= MAX_THREADS, (row, p)
+            assert (rows_out * min(row[2], 64) + 31) // 32 * 256 + 256 <= MAX_THREADS, (row, p)
+            assert p["groups"] * p["TN"] * (16 * (2 if row[0] else 4) if p["last"] else 16) >= rows_out
