@@ -87,17 +87,23 @@ inline bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, 
   if (ndim == 2) p->g_rows = 0;
   // Tiles per wave: every wave forms its part of B once for all its tiles
   // (about the cost of one more tile), and the chunks are dealt to the waves
-  // that fit the GPU at once in equal numbers: the least sum over a wave's
-  // chunks wins.
+  // that fit the GPU at once in equal numbers, at least the four of one
+  // workgroup per group: the least sum over a wave's chunks, times the rounds
+  // that the groups of a long mode take, wins.  Tiles per wave against one,
+  // long mode: 200000 x 30 x 41, float32, rank 16 / 32: 220 / 254 us with
+  // three, 220 / 287 with one; 100000 x 33 x 35, rank 20: 125, 145; 5 x 9 x
+  // 500001, rank 8: 34, 42.
   int64_t best = -1;
   for (int tn = most; tn >= 1; --tn) {
     const int64_t groups = (tiles + tn - 1) / tn;
     const int TN = (int)((tiles + groups - 1) / groups);
     const int RV = 4 * any_last_rows(TN, p->RT);
     const int64_t chunks = p->last ? (p->A + RV - 1) / RV : p->A * p->nqc;
-    const int64_t waves = std::max<int64_t>(1, 256 * 4 * any_occ(TN, p->RT, p->last, f64) / groups);
+    const int64_t slots = 256 * 4 * any_occ(TN, p->RT, p->last, f64);
+    const int64_t waves = std::max<int64_t>(kAnyWaves, slots / groups);
     const int64_t per = (chunks + waves - 1) / waves;
-    const int64_t cost = per * (TN + 1) * (p->last ? RV : 16);
+    const int64_t rounds = (groups * waves + slots - 1) / slots;
+    const int64_t cost = per * rounds * (TN + 1) * (p->last ? RV : 16);
     if (best >= 0 && cost >= best) continue;
     best = cost;
     p->TN = TN;

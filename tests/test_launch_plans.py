@@ -140,3 +140,11 @@ def test_mttkrp_grids_fit_a_launch(any_plan):
             assert 0 < p["groups"] * p["nblk"] * 256 <= MAX_THREADS, (row, p)
             assert (rows_out * min(row[2], 64) + 31) // 32 * 256 + 256 <= MAX_THREADS, (row, p)
             assert p["groups"] * p["TN"] * (16 * (2 if row[0] else 4) if p["last"] else 16) >= rows_out
+
+
+def test_mttkrp_tiles_of_long_modes(any_plan):
+    """With more groups than waves fit the GPU, several tiles per wave share
+    the rows of the Khatri-Rao product."""
+    rows = [(0, (200_000, 30, 41), 16, 0, 0), (0, (1_000_000, 7, 9), 16, 0, 1), (1, (100_000, 33, 35), 20, 0, 0),
+            (0, (5, 9, 500_001), 8, 2, 0), (0, (9, 70_001, 31), 33, 1, 1)]
+    assert all(p["TN"] >= 2 for p in any_plan(rows))
