@@ -90,9 +90,9 @@ inline bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, 
   // that fit the GPU at once in equal numbers, at least the four of one
   // workgroup per group: the least sum over a wave's chunks, times the rounds
   // that the groups of a long mode take, wins.  Tiles per wave against one,
-  // long mode: 200000 x 30 x 41, float32, rank 16 / 32: 220 / 254 us with
-  // three, 220 / 287 with one; 100000 x 33 x 35, rank 20: 125, 145; 5 x 9 x
-  // 500001, rank 8: 34, 42.
+  // long mode: 200000 x 30 x 41, float32, rank 32 / 64: 253 / 389 us with
+  // several, 286 / 456 with one; 100000 x 33 x 35, rank 20: 125, 139, and float64
+  // 252, 307; 5 x 9 x 500001, rank 8: 34, 42.
   int64_t best = -1;
   for (int tn = most; tn >= 1; --tn) {
     const int64_t groups = (tiles + tn - 1) / tn;
@@ -104,7 +104,9 @@ inline bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, 
     const int64_t per = (chunks + waves - 1) / waves;
     const int64_t rounds = (groups * waves + slots - 1) / slots;
     const int64_t cost = per * rounds * (TN + 1) * (p->last ? RV : 16);
-    if (best >= 0 && cost >= best) continue;
+    // (over several rounds the sharing of two and more rank tiles gives a
+    // little more than this counts: fewer tiles have to win by a seventh)
+    if (best >= 0 && cost >= (rounds > 1 && p->RT > 1 ? best - best / 7 : best)) continue;
     best = cost;
     p->TN = TN;
     p->groups = groups;
