@@ -471,13 +471,18 @@ struct CooArgs {
   const void* weights;
   int ndim, mode, R;
   int n_other, other[kMaxOrder - 1];  // the modes that are contracted
+  bool wide;  // one of them has more than 2^32 entries
   int64_t rows;
   void* partial;  // n_seg x R
   void* out;
 };
 
-// NO: the number of other modes (7: at most 7).
-template <typename T, int LR, int NO>
+__device__ __forceinline__ uint32_t coo_shfl(uint32_t v, int src) { return (uint32_t)__shfl((int)v, src, 64); }
+__device__ __forceinline__ int64_t coo_shfl(int64_t v, int src) { return __shfl((long long)v, src, 64); }
+
+// NO: the number of other modes (7: at most 7).  Index: uint32_t, or int64_t
+// where a mode has more than 2^32 entries.
+template <typename T, int LR, int NO, typename Index = uint32_t>
 __global__ __launch_bounds__(256) void mttkrp_coo_segments_kernel(CooArgs a) {
   constexpr int G = 64 / LR;
   constexpr int UN = G >= 16 ? 2 : 4;  // nonzeros of a lane group in flight
@@ -507,11 +512,11 @@ __global__ __launch_bounds__(256) void mttkrp_coo_segments_kernel(CooArgs a) {
     for (int64_t base = p0; base < p1; base += 64) {
       const int n = (int)min((int64_t)64, p1 - base);
       T val = (T)0;
-      uint32_t idx[NO];
+      Index idx[NO];
       const int64_t q = a.perm[base + min(lane, n - 1)];
       val = vals[q];
 #pragma unroll
-      for (int m = 0; m < NO; ++m) idx[m] = m < a.n_other ? (uint32_t)a.coords[(int64_t)a.other[m] * a.nnz + q] : 0;
+      for (int m = 0; m < NO; ++m) idx[m] = m < a.n_other ? (Index)a.coords[(int64_t)a.other[m] * a.nnz + q] : 0;
       for (int s = 0; s * G < n; s += UN) {
         T t[UN], f[UN][NO];
 #pragma unroll
@@ -520,7 +525,7 @@ __global__ __launch_bounds__(256) void mttkrp_coo_segments_kernel(CooArgs a) {
           t[u] = __shfl(val, src, 64);
 #pragma unroll
           for (int m = 0; m < NO; ++m)
-            if (m < a.n_other) f[u][m] = ((const T*)a.factors[a.other[m]])[(int64_t)(uint32_t)__shfl((int)idx[m], src, 64) * R + r];
+            if (m < a.n_other) f[u][m] = ((const T*)a.factors[a.other[m]])[(int64_t)coo_shfl(idx[m], src) * R + r];
         }
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
@@ -585,7 +590,8 @@ template <typename T, int LR>
 static void launch_coo(const CooArgs& a, hipStream_t st) {
   if (a.n_seg > 0) {
     const unsigned blocks = (unsigned)std::min<int64_t>((a.n_seg + 3) / 4, 65536);
-    switch (a.n_other) {
+    if (a.wide) mttkrp_coo_segments_kernel<T, 64, kMaxOrder - 1, int64_t><<<blocks, 256, 0, st>>>(a);
+    else switch (a.n_other) {
       case 1: mttkrp_coo_segments_kernel<T, LR, 1><<<blocks, 256, 0, st>>>(a); break;
       case 2: mttkrp_coo_segments_kernel<T, LR, 2><<<blocks, 256, 0, st>>>(a); break;
       case 3: mttkrp_coo_segments_kernel<T, LR, 3><<<blocks, 256, 0, st>>>(a); break;
@@ -756,8 +762,10 @@ extern "C" int tla_mttkrp_coo(int dtype, int64_t nnz, int ndim, const int64_t* s
     TLA_REQUIRE(shape[m] >= 1, "mttkrp_coo: shape[%d] = %lld", m, (long long)shape[m]);
     TLA_REQUIRE(m == mode || factors[m] != nullptr, "mttkrp_coo: factor %d is NULL", m);
     a.factors[m] = factors[m];
-    TLA_REQUIRE(m == mode || shape[m] <= 0xffffffffll, "mttkrp_coo: shape[%d] = %lld", m, (long long)shape[m]);
-    if (m != mode) a.other[a.n_other++] = m;
+    if (m != mode) {
+      a.other[a.n_other++] = m;
+      a.wide = a.wide || shape[m] > 0xffffffffll;
+    }
   }
   a.coords = coords; a.nnz = nnz; a.vals = values; a.perm = perm; a.row_ptr = row_ptr;
   a.seg_row = seg_row; a.seg_start = seg_start; a.seg_row_ptr = seg_row_ptr; a.n_seg = n_seg; a.seg_len = seg_len;

@@ -479,3 +479,26 @@ def test_mttkrp_any_shape_scale_rows_in_slices(cuda, shape, rank, mode, dtype):
         ref = torch.stack([u[:, q : q + 4096] @ k[q : q + 4096] for q in range(0, u.shape[1], 4096)], -1).sum(-1)
         err = float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref))
         assert err < max(1.0, 0.05 * (n / shape[mode]) ** 0.5 / 16) * TOL[dtype], err
+
+
+@pytest.mark.parametrize("order", [2, 3])
+def test_mttkrp_coo_mode_of_more_than_32_bits(cuda, order):
+    """A contracted mode of more than 2^32 entries (a factor of 17 GB, zero but
+    where the nonzeros look), alone and beside another."""
+    from tensorly_amd.tenalg import unfolding_dot_khatri_rao_coo
+    n = 2 ** 32 + 1000
+    at = torch.tensor([0, 1000, 2 ** 31, 2 ** 32 - 1, 2 ** 32, 2 ** 32 + 7, n - 1], device=cuda)
+    big = torch.zeros((n, 1), device=cuda)
+    big[at, 0] = torch.arange(1.0, 8.0, device=cuda)
+    F = [torch.tensor([[2.0], [3.0]], device=cuda), big]
+    coords = torch.stack([torch.arange(7, device=cuda) % 2, at])
+    values = torch.arange(10.0, 17.0, device=cuda)
+    if order == 2:
+        out = unfolding_dot_khatri_rao_coo(coords, values, (2, n), (None, F), 0)
+        t = values * big[at, 0]
+        assert out[:, 0].tolist() == [float(t[0::2].sum()), float(t[1::2].sum())]
+    else:
+        F3, c3 = [F[0], big, torch.ones((3, 1), device=cuda)], torch.cat([coords, coords[:1]], 0)
+        out = unfolding_dot_khatri_rao_coo(c3, values, (2, n, 3), (None, F3), 2)
+        t = values * big[at, 0] * F[0][coords[0], 0]
+        assert out[:, 0].tolist() == [float(t[0::2].sum()), float(t[1::2].sum()), 0.0]
