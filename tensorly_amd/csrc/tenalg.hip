@@ -497,12 +497,16 @@ __global__ __launch_bounds__(256) void mttkrp_coo_segments_kernel(CooArgs a) {
     if (a.seg_row) {
       row = a.seg_row[j];
       p0 = a.seg_start[j];
-    } else {  // the row with seg_row_ptr[row] <= j < seg_row_ptr[row + 1]
+    } else {
+      // the last row with seg_row_ptr[row] <= j, 64 candidates at a time (one
+      // at a time, 22 dependent loads for 3M rows, the search was most of the
+      // kernel's time)
       int64_t lo = 0, hi = a.rows;
       while (hi - lo > 1) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (a.seg_row_ptr[mid] <= j) lo = mid;
-        else hi = mid;
+        const int64_t step = (hi - lo + 63) >> 6, at = lo + lane * step;
+        const bool le = lane == 0 || (at < hi && a.seg_row_ptr[at] <= j);
+        lo += (__popcll(__ballot(le)) - 1) * step;
+        hi = min(hi, lo + step);
       }
       row = lo;
       p0 = a.row_ptr[row] + (j - a.seg_row_ptr[row]) * a.seg_len;
@@ -542,33 +546,77 @@ __global__ __launch_bounds__(256) void mttkrp_coo_segments_kernel(CooArgs a) {
   }
 }
 
-// One row per workgroup: 256 / LR lanes over the row's segments.
+// The sum of segments [j0, j1) by the workgroup, 256 / LR lanes side by side
+// (part: column of the lane's rank); in threads below LR.
+template <typename T, int LR>
+__device__ __forceinline__ T coo_block_row(const T* part, int64_t j0, int64_t j1, int R, T* red) {
+  constexpr int KL = 256 / LR;
+  const int kl = threadIdx.x / LR;
+  T s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+  int64_t j = j0 + kl;
+  for (; j + 3 * KL < j1; j += 4 * KL) {
+    s0 += part[j * R];
+    s1 += part[(j + KL) * R];
+    s2 += part[(j + 2 * KL) * R];
+    s3 += part[(j + 3 * KL) * R];
+  }
+  for (; j < j1; j += KL) s0 += part[j * R];
+  red[threadIdx.x] = (s0 + s1) + (s2 + s3);
+  __syncthreads();
+  for (int h = KL / 2; h >= 1; h >>= 1) {
+    if (kl < h) red[threadIdx.x] += red[threadIdx.x + h * LR];
+    __syncthreads();
+  }
+  return red[threadIdx.x % LR];
+}
+
+// One row per workgroup.
 template <typename T, int LR>
 __global__ __launch_bounds__(256) void mttkrp_coo_rows_kernel(CooArgs a) {
-  constexpr int KL = 256 / LR;
   __shared__ T red[256];
-  const int r = threadIdx.x % LR, kl = threadIdx.x / LR, R = a.R;
+  const int r = threadIdx.x % LR, R = a.R;
   const T* w = (const T*)a.weights;
   const T* part = (const T*)a.partial + min(r, R - 1);
   for (int64_t i = blockIdx.x; i < a.rows; i += gridDim.x) {
-    const int64_t j1 = a.seg_row_ptr[i + 1];
-    T s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-    int64_t j = a.seg_row_ptr[i] + kl;
-    for (; j + 3 * KL < j1; j += 4 * KL) {
-      s0 += part[j * R];
-      s1 += part[(j + KL) * R];
-      s2 += part[(j + 2 * KL) * R];
-      s3 += part[(j + 3 * KL) * R];
-    }
-    for (; j < j1; j += KL) s0 += part[j * R];
-    red[threadIdx.x] = (s0 + s1) + (s2 + s3);
+    const T s = coo_block_row<T, LR>(part, a.seg_row_ptr[i], a.seg_row_ptr[i + 1], R, red);
+    if (threadIdx.x < R) ((T*)a.out)[i * R + r] = w ? s * w[r] : s;
     __syncthreads();
-    for (int h = KL / 2; h >= 1; h >>= 1) {
-      if (kl < h) red[threadIdx.x] += red[threadIdx.x + h * LR];
+  }
+}
+
+constexpr int64_t kCooManyRows = 8192;
+
+// Many rows: four per workgroup, a wave each, and the whole workgroup only for
+// those of more than 64 segments.  A workgroup per row costs eight barriers
+// for what is mostly one segment.  With the row search, 3M rows, 1M nonzeros,
+// rank 16, the whole call: 2120 -> 1186 us; 300000 rows, rank 8: 623 -> 476.
+template <typename T, int LR>
+__global__ __launch_bounds__(256) void mttkrp_coo_many_rows_kernel(CooArgs a) {
+  constexpr int KW = 64 / LR;
+  __shared__ T red[256];
+  const int lane = threadIdx.x & 63, r = lane % LR, R = a.R;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const T* w = (const T*)a.weights;
+  const T* part = (const T*)a.partial + min(r, R - 1);
+  for (int64_t base = (int64_t)blockIdx.x * 4; base < a.rows; base += (int64_t)gridDim.x * 4) {
+    const int64_t i = base + wave;
+    const int64_t j0 = i < a.rows ? a.seg_row_ptr[i] : 0, j1 = i < a.rows ? a.seg_row_ptr[i + 1] : 0;
+    const bool heavy = j1 - j0 > 64;
+    if (!heavy) {
+      T s = 0;
+      for (int64_t j = j0 + lane / LR; j < j1; j += KW) s += part[j * R];
+#pragma unroll
+      for (int off = LR; off < 64; off <<= 1) s += __shfl_xor(s, off, 64);
+      if (i < a.rows && lane < R) ((T*)a.out)[i * R + r] = w ? s * w[r] : s;
+    }
+    if (!__syncthreads_or(heavy)) continue;
+    for (int64_t k = base; k < min(base + 4, a.rows); ++k) {
+      const int64_t k0 = a.seg_row_ptr[k], k1 = a.seg_row_ptr[k + 1];
+      if (k1 - k0 <= 64) continue;
+      const T s = coo_block_row<T, LR>(part, k0, k1, R, red);
+      if (threadIdx.x < R) ((T*)a.out)[k * R + r] = w ? s * w[r] : s;
       __syncthreads();
     }
-    if (kl == 0 && r < R) ((T*)a.out)[i * R + r] = w ? red[r] * w[r] : red[r];
-    __syncthreads();
   }
 }
 
@@ -598,7 +646,11 @@ static void launch_coo(const CooArgs& a, hipStream_t st) {
       default: mttkrp_coo_segments_kernel<T, LR, kMaxOrder - 1><<<blocks, 256, 0, st>>>(a); break;
     }
   }
-  mttkrp_coo_rows_kernel<T, LR><<<(unsigned)std::min<int64_t>(a.rows, 65536), 256, 0, st>>>(a);
+  // (fewer rows: the workgroups per row fill the GPU with the segments of each)
+  if (a.rows > kCooManyRows)
+    mttkrp_coo_many_rows_kernel<T, LR><<<(unsigned)std::min<int64_t>((a.rows + 3) / 4, 65536), 256, 0, st>>>(a);
+  else
+    mttkrp_coo_rows_kernel<T, LR><<<(unsigned)a.rows, 256, 0, st>>>(a);
 }
 
 template <typename T>

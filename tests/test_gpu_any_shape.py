@@ -502,3 +502,30 @@ def test_mttkrp_coo_mode_of_more_than_32_bits(cuda, order):
         out = unfolding_dot_khatri_rao_coo(c3, values, (2, n, 3), (None, F3), 2)
         t = values * big[at, 0] * F[0][coords[0], 0]
         assert out[:, 0].tolist() == [float(t[0::2].sum()), float(t[1::2].sum()), 0.0]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rank", [1, 5, 16, 33, 64])
+@pytest.mark.parametrize("rows,heavy", [(8192, 0), (8193, 0), (20001, 1), (100003, 5)])
+def test_mttkrp_coo_many_rows(cuda, rows, heavy, rank, dtype):
+    """Four rows per workgroup, rows of more than 64 segments (16,384 nonzeros)
+    by the whole of it, most rows empty or of one nonzero.  Sums of up to
+    20,000 terms in chains of 256 and fewer: tolerance as above."""
+    from tensorly_amd.tenalg import unfolding_dot_khatri_rao_coo
+    g = torch.Generator(device=cuda).manual_seed(rows + rank)
+    idx = [torch.randint(0, rows, (30_000,), generator=g, device=cuda)]
+    for h in range(heavy):
+        idx.append(torch.full((16_300 + 60 * h,), (rows - 1) * (h + 1) // heavy, device=cuda))
+    idx = torch.cat(idx)
+    nnz, shape = idx.shape[0], (rows, 7, 9)
+    coords = torch.stack([idx] + [torch.randint(0, s, (nnz,), generator=g, device=cuda) for s in shape[1:]])
+    values = torch.randn(nnz, generator=g, device=cuda, dtype=dtype)
+    F = [torch.randn((s, rank), generator=g, device=cuda, dtype=dtype) for s in shape]
+    w = torch.rand(rank, generator=g, device=cuda, dtype=dtype) + 0.5
+    out = unfolding_dot_khatri_rao_coo(coords, values, shape, (w, F), 0)
+    t = values.double()[:, None] * F[1].double()[coords[1]] * F[2].double()[coords[2]] * w.double()
+    ref = torch.zeros((rows, rank), dtype=torch.float64, device=cuda).index_add_(0, idx, t)
+    for h in range(heavy):  # (one after another, so many would round more than the kernel)
+        ref[(rows - 1) * (h + 1) // heavy] = t[idx == (rows - 1) * (h + 1) // heavy].sum(0)
+    assert float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref)) < TOL[dtype]
+    assert bool((out[torch.bincount(idx, minlength=rows) == 0] == 0).all())
