@@ -132,7 +132,10 @@ __global__ __launch_bounds__(kHalsThreads) void hals_nnls_kernel(HalsArgs a) {
 // multiply-add, one maximum, a broadcast among the four lanes and one
 // multiply-add into the next column's gradient, where a dot product per
 // update is a chain of R multiply-adds.  The gradient is formed afresh every
-// kHalsRefresh iterations.  The chain of dependent FP64 operations bounds it:
+// kHalsRefresh iterations, and in each of the first four: from a start far
+// above the solution it falls by orders of magnitude there, and would keep
+// the rounding of its first size (a start 200 times too large, rank 64, two
+// iterations: 6e-12 of the largest entry, now below 1e-12).  The chain of dependent FP64 operations bounds it:
 // 256 rows, rank 16, 100 iterations take 92 us and 96 us with the decision and
 // the last launch (one launch per iteration, a thread per row and a dot
 // product per update: 1362 us); 512 rows, rank 64: 992 us (16.2 ms).
@@ -235,7 +238,7 @@ __global__ __launch_bounds__(64) void hals_run_kernel(HalsRun h) {
     }
 #pragma unroll 1
   for (int it = 0; it < iters; ++it) {
-    if (it % kHalsRefresh == 0) {
+    if (it % kHalsRefresh == 0 || (chunk == 0 && it < 4)) {
 #pragma unroll
       for (int e = 0; e < E; ++e) g[e] = -m[e];
       if constexpr (!kReg) read_u(0, 0);

@@ -529,3 +529,37 @@ def test_mttkrp_coo_many_rows(cuda, rows, heavy, rank, dtype):
         ref[(rows - 1) * (h + 1) // heavy] = t[idx == (rows - 1) * (h + 1) // heavy].sum(0)
     assert float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref)) < TOL[dtype]
     assert bool((out[torch.bincount(idx, minlength=rows) == 0] == 0).all())
+
+
+def _hals(F, M, n_iter, tol, dtype):
+    """tla_hals_nnls on F[0] in place; the iterations run."""
+    from tensorly_amd import _lib
+    from tensorly_amd.cp_tensor import grams64
+    L, (rows, rank) = _lib.lib(), F[0].shape
+    grams = grams64(F[1:])
+    gp, _k = _lib.ptr_array([grams[0]] + grams)
+    iters = torch.zeros(1, dtype=torch.int32, device=F[0].device)
+    nb = L.tla_hals_nnls_workspace_size(rows, rank)
+    ws = _lib.workspace(nb, F[0].device)
+    _lib.check(L.tla_hals_nnls(_lib.dtype_code(F[0]), _lib.ptr(F[0]), _lib.ptr(M), rows, rank, gp, len(F), 0, None,
+                               _lib.F64, 0.0, 0, n_iter, tol, _lib.ptr(iters), _lib.ptr(ws), nb,
+                               _lib.stream(F[0].device)), "hals")
+    return int(iters)
+
+
+@pytest.mark.parametrize("rows,rank,n_iter,tol", [(40, 64, 100, 0.6), (40, 64, 2, 0.0), (40, 33, 3, 0.0), (40, 16, 5, 0.0),
+                                                  (40, 5, 7, 0.0)])
+def test_hals_from_a_start_far_above_the_solution(cuda, rows, rank, n_iter, tol):
+    """The gradient falls by orders of magnitude in the first iteration: its
+    rounding must not stay at the first size.  Against the oracle in FP64;
+    tolerance as above."""
+    import numpy as np
+    from oracle import tensorly_np as T
+    g = torch.Generator(device=cuda).manual_seed(rows + rank)
+    F = [torch.rand((s, rank), generator=g, device=cuda, dtype=torch.float64) for s in (rows, 130, 110)]
+    M = torch.rand((rows, rank), generator=g, device=cuda, dtype=torch.float64) * 3 + 1
+    Fn = [f.cpu().numpy() for f in F]
+    utu = (Fn[1].T @ Fn[1]) * (Fn[2].T @ Fn[2])
+    ref = T.hals_nnls(M.cpu().numpy().T, utu, Fn[0].T.copy(), n_iter_max=n_iter, tol=tol).T
+    _hals(F, M, n_iter, tol, torch.float64)
+    np.testing.assert_allclose(F[0].cpu().numpy(), ref, rtol=1e-9, atol=1e-12 * np.abs(ref).max())
