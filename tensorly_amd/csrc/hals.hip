@@ -1,6 +1,8 @@
 // HALS non-negative least squares of one CP factor.
 #include <math.h>
 
+#include <algorithm>
+
 #include "common.h"
 #include "inverse.h"
 
@@ -140,7 +142,9 @@ __global__ __launch_bounds__(kHalsThreads) void hals_nnls_kernel(HalsArgs a) {
 // the last launch (one launch per iteration, a thread per row and a dot
 // product per update: 1362 us); 512 rows, rank 64: 992 us (16.2 ms).
 constexpr int kHalsRows = 16;     // rows per workgroup of one wave
-constexpr int kHalsChunk = 128;   // iterations per launch
+constexpr int kHalsChunk = 128;   // iterations per launch, at most
+constexpr int kHalsBlocks = 65536;  // workgroups, at most: more rows take turns
+constexpr int kHalsSums = 256;      // sets that more than 1024 workgroups' error sums are added up to
 constexpr int kHalsRefresh = 8;
 
 // state: [0] the rule fired, [1] iterations run, [2] chunk in which it fired,
@@ -149,11 +153,13 @@ struct HalsRun {
   HalsArgs a;
   double* vbuf[2];   // rows x R FP64: V after the odd / even chunks
   double* partial;   // [workgroup][iteration of the chunk]
+  double* sums;      // [kHalsSums][iteration of the chunk]
   int* state;
   double* err0;
   int chunk, iters;  // this chunk and its iterations
-  int final;
-  int nblk;
+  int begin;         // iterations before it
+  int final, only;   // the last launch; the only one (one iteration)
+  int nblk;          // workgroups, each every nblk-th group of rows
 };
 
 template <int Q>
@@ -171,8 +177,8 @@ __device__ __forceinline__ double quad_get(double v, int q) {
 
 // h.final: replays the chunk in which the rule fired (state), or takes the
 // last chunk's values, and writes the factor.
-// FULL: R == RT.
-template <typename T, int RT, bool FULL>
+// FULL: R == RT.  LOOP: more groups of rows than workgroups.
+template <typename T, int RT, bool FULL, bool LOOP>
 __global__ __launch_bounds__(64) void hals_run_kernel(HalsRun h) {
   constexpr int E = RT / 4;
   __shared__ double U[RT * RT];  // zero outside R x R
@@ -180,11 +186,11 @@ __global__ __launch_bounds__(64) void hals_run_kernel(HalsRun h) {
   __shared__ double errs[16 * 65];
   const HalsArgs& a = h.a;
   const int lane = threadIdx.x, q = lane & 3, R = a.R;
-  const int64_t i = (int64_t)blockIdx.x * kHalsRows + (lane >> 2);
-  const bool live = i < a.rows;
   int chunk = h.chunk, iters = h.iters;
   if (h.final) {
-    if (h.state[0]) {
+    if (h.only) {  // one iteration: it runs whatever the rule says
+      if (blockIdx.x == 0 && lane == 0) h.state[1] = iters;
+    } else if (h.state[0]) {
       chunk = h.state[2];
       iters = h.state[3];
     } else {
@@ -197,26 +203,33 @@ __global__ __launch_bounds__(64) void hals_run_kernel(HalsRun h) {
   T* A = (T*)a.A;
   const T* M = (const T*)a.M;
   const double* src = h.vbuf[chunk & 1];
-  double v[E], m[E], g[E];
-  const int64_t base = live ? i * R : 0;
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int l = q * E + e;
-    const bool on = live && l < R;
-    v[e] = !on ? 0.0 : chunk == 0 ? (double)A[base + l] : src[base + l];
-    m[e] = on ? (double)M[base + l] - (a.has_sparsity ? a.sparsity : 0.0) : 0.0;
-  }
   if (iters > 0) {
-    for (int e = lane; e < RT * RT; e += 64) {
-      const int k = e / RT, l = e % RT;
-      double u = 0.0;
-      if (k < R && l < R) {
-        u = 1.0;
-        for (int n = 0; n < a.ndim; ++n)
-          if (n != a.mode) u *= a.grams[n][k * R + l];
-        if (a.weights) u *= weight_at(a.weights, a.wdt, k) * weight_at(a.weights, a.wdt, l);
+    // (16 loads of a Gram in flight)
+    constexpr int NU = RT * RT / 64 > 0 ? RT * RT / 64 : 1, NB = NU < 16 ? NU : 16;
+#pragma unroll 1
+    for (int b = 0; b < (RT * RT + 64 * NB - 1) / (64 * NB); ++b) {
+      double u[NB], w[NB];
+      int at[NB];
+#pragma unroll
+      for (int x = 0; x < NB; ++x) {
+        const int e = (b * NB + x) * 64 + lane, k = e / RT, l = e % RT;
+        at[x] = k < R && l < R ? k * R + l : -1;
+        u[x] = at[x] >= 0 ? 1.0 : 0.0;
       }
-      U[e] = u;
+      for (int n = 0; n < a.ndim; ++n)
+        if (n != a.mode) {
+          const double* G = a.grams[n];
+#pragma unroll
+          for (int x = 0; x < NB; ++x) w[x] = at[x] >= 0 ? G[at[x]] : 0.0;
+#pragma unroll
+          for (int x = 0; x < NB; ++x) u[x] *= w[x];
+        }
+#pragma unroll
+      for (int x = 0; x < NB; ++x) {
+        const int e = (b * NB + x) * 64 + lane;
+        if (a.weights && at[x] >= 0) u[x] *= weight_at(a.weights, a.wdt, e / RT) * weight_at(a.weights, a.wdt, e % RT);
+        if (e < RT * RT) U[e] = u[x];
+      }
     }
     __syncthreads();
     for (int k = lane; k < RT; k += 64) rd[k] = U[k * RT + k] != 0.0 ? 1.0 / U[k * RT + k] : 0.0;
@@ -237,131 +250,185 @@ __global__ __launch_bounds__(64) void hals_run_kernel(HalsRun h) {
       for (int k = 0; k < RT; ++k) read_u(k, k);
     }
 #pragma unroll 1
-  for (int it = 0; it < iters; ++it) {
-    if (it % kHalsRefresh == 0 || (chunk == 0 && it < 4)) {
+  for (int64_t i0 = (int64_t)blockIdx.x * kHalsRows; !LOOP || i0 < a.rows; i0 += (int64_t)h.nblk * kHalsRows) {
+    const int64_t i = i0 + (lane >> 2);
+    const bool live = i < a.rows;
+    double v[E], m[E], g[E];
+    const int64_t base = live ? i * R : 0;
 #pragma unroll
-      for (int e = 0; e < E; ++e) g[e] = -m[e];
-      if constexpr (!kReg) read_u(0, 0);
-#pragma unroll
-      for (int l = 0; l < RT; ++l) {
-        if constexpr (!kReg) read_u((l + 1) % RT, (l + 1) & 1);
-        const double vl = quad_get(v[l % E], l / E);
-#pragma unroll
-        for (int e = 0; e < E; ++e) g[e] = fma(ur[kReg ? l : l & 1][e], vl, g[e]);
-      }
-    } else if constexpr (!kReg) {
-      read_u(0, 0);
+    for (int e = 0; e < E; ++e) {
+      const int l = q * E + e;
+      const bool on = live && l < R;
+      v[e] = !on ? 0.0 : chunk == 0 ? (double)A[base + l] : src[base + l];
+      m[e] = on ? (double)M[base + l] - (a.has_sparsity ? a.sparsity : 0.0) : 0.0;
     }
-    double err = 0.0;
+    int fresh = 0;  // the next iteration with a gradient formed afresh
+#pragma unroll 1
+    for (int it = 0; it < iters; ++it) {
+      if (it == fresh) {
+        fresh = chunk == 0 && it < 3 ? it + 1 : (it | (kHalsRefresh - 1)) + 1;
 #pragma unroll
-    for (int k = 0; k < RT; ++k) {
-      // no branches: the whole iteration is one run of instructions.  A
-      // skipped column (and the padding past R) has rr = 0.
-      if constexpr (!kReg) read_u((k + 1) % RT, (k + 1) & 1);
-      const double r = rr[kReg ? k : k & 1];
-      const double mine = r != 0.0 ? fmax(fma(-g[k % E], r, v[k % E]), 0.0) : v[k % E];
-      const double nv = quad_get(mine, k / E), dv = quad_get(mine - v[k % E], k / E);
-      // the stopping sum subtracts the new value from every entry of this
-      // row of A as it is before the update (the reference's broadcast
-      // ||V - newV||^2)
-      double s = 0.0;
+        for (int e = 0; e < E; ++e) g[e] = -m[e];
+        if constexpr (!kReg) read_u(0, 0);
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const double df = FULL || q * E + e < R ? v[e] - nv : 0.0;
-        s = fma(df, df, s);
-      }
-      err += r != 0.0 ? s : 0.0;
-      v[k % E] = q == k / E ? nv : v[k % E];
+        for (int l = 0; l < RT; ++l) {
+          if constexpr (!kReg) read_u((l + 1) % RT, (l + 1) & 1);
+          const double vl = quad_get(v[l % E], l / E);
 #pragma unroll
-      for (int e = 0; e < E; ++e) g[e] = fma(ur[kReg ? k : k & 1][e], dv, g[e]);
-    }
-    // sixteen iterations' lane sums at a time, added up in lane order
-    errs[(it & 15) * 65 + lane] = live ? err : 0.0;
-    if ((it & 15) == 15 || it + 1 == iters) {
-      __syncthreads();
-      if (!h.final && lane <= (it & 15)) {
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-#pragma unroll
-        for (int t = 0; t < 64; t += 4) {
-          s0 += errs[lane * 65 + t];
-          s1 += errs[lane * 65 + t + 1];
-          s2 += errs[lane * 65 + t + 2];
-          s3 += errs[lane * 65 + t + 3];
+          for (int e = 0; e < E; ++e) g[e] = fma(ur[kReg ? l : l & 1][e], vl, g[e]);
         }
-        h.partial[(int64_t)blockIdx.x * kHalsChunk + (it & ~15) + lane] = (s0 + s1) + (s2 + s3);
+      } else if constexpr (!kReg) {
+        read_u(0, 0);
       }
-      __syncthreads();
-    }
-  }
+      double err = 0.0;
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int l = q * E + e;
-    if (live && l < R) {
-      if (h.final) A[base + l] = (T)v[e];
-      else h.vbuf[(chunk + 1) & 1][base + l] = v[e];
+      for (int k = 0; k < RT; ++k) {
+        // no branches: the whole iteration is one run of instructions.  A
+        // skipped column (and the padding past R) has rr = 0.
+        if constexpr (!kReg) read_u((k + 1) % RT, (k + 1) & 1);
+        const double r = rr[kReg ? k : k & 1];
+        const double mine = r != 0.0 ? fmax(fma(-g[k % E], r, v[k % E]), 0.0) : v[k % E];
+        const double nv = quad_get(mine, k / E), dv = quad_get(mine - v[k % E], k / E);
+        // the stopping sum subtracts the new value from every entry of this
+        // row of A as it is before the update (the reference's broadcast
+        // ||V - newV||^2)
+        double s = 0.0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const double df = FULL || q * E + e < R ? v[e] - nv : 0.0;
+          s = fma(df, df, s);
+        }
+        err += r != 0.0 ? s : 0.0;
+        v[k % E] = q == k / E ? nv : v[k % E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) g[e] = fma(ur[kReg ? k : k & 1][e], dv, g[e]);
+      }
+      // sixteen iterations' lane sums at a time, added up in lane order
+      errs[(it & 15) * 65 + lane] = live ? err : 0.0;
+      if ((it & 15) == 15 || it + 1 == iters) {
+        __syncthreads();
+        if (!h.final && lane <= (it & 15)) {
+          double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+#pragma unroll
+          for (int t = 0; t < 64; t += 4) {
+            s0 += errs[lane * 65 + t];
+            s1 += errs[lane * 65 + t + 1];
+            s2 += errs[lane * 65 + t + 2];
+            s3 += errs[lane * 65 + t + 3];
+          }
+          double* p = h.partial + (int64_t)blockIdx.x * kHalsChunk + (it & ~15) + lane;
+          double sum = (s0 + s1) + (s2 + s3);
+          if (LOOP && i0 >= (int64_t)h.nblk * kHalsRows) sum += *p;  // this workgroup's earlier rows
+          *p = sum;
+        }
+        __syncthreads();
+      }
     }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int l = q * E + e;
+      if (live && l < R) {
+        if (h.final) A[base + l] = (T)v[e];
+        else h.vbuf[(chunk + 1) & 1][base + l] = v[e];
+      }
+    }
+    if constexpr (!LOOP) break;
   }
 }
 
-// Every iteration's error sum over the workgroups (eight interleaved sums per
-// iteration, added up in order), then the first iteration at which the rule
-// fires.
-__global__ __launch_bounds__(8 * kHalsChunk) void hals_decide_kernel(HalsRun h) {
-  __shared__ double part[8][kHalsChunk];
+// Many workgroups' error sums: kHalsSums of every so many each, in order.
+__global__ __launch_bounds__(kHalsChunk) void hals_sum_kernel(HalsRun h) {
+  if (h.chunk > 0 && h.state[0]) return;
+  const int it = threadIdx.x;
+  if (it >= h.iters) return;
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  const double* p = h.partial + it;
+  int b = blockIdx.x;
+  for (; b + 3 * kHalsSums < h.nblk; b += 4 * kHalsSums) {
+    s0 += p[(int64_t)b * kHalsChunk];
+    s1 += p[(int64_t)(b + kHalsSums) * kHalsChunk];
+    s2 += p[(int64_t)(b + 2 * kHalsSums) * kHalsChunk];
+    s3 += p[(int64_t)(b + 3 * kHalsSums) * kHalsChunk];
+  }
+  for (; b < h.nblk; b += kHalsSums) s0 += p[(int64_t)b * kHalsChunk];
+  h.sums[blockIdx.x * kHalsChunk + it] = (s0 + s1) + (s2 + s3);
+}
+
+// Every iteration's error sum over n sets of them (interleaved sums per
+// iteration, 8 and more, added up in order), then the first iteration at which
+// the rule fires.
+__global__ __launch_bounds__(8 * kHalsChunk) void hals_decide_kernel(HalsRun h, const double* sets, int n) {
+  __shared__ double part[8 * kHalsChunk];
   __shared__ int first;
   if (h.chunk > 0 && h.state[0]) return;
-  const int it = threadIdx.x % kHalsChunk, lane = threadIdx.x / kHalsChunk;
+  int W = kHalsChunk;  // threads beside each other: the iterations, rounded up
+  while (W > 8 && W / 2 >= h.iters) W /= 2;
+  const int it = threadIdx.x % W, lane = threadIdx.x / W, lanes = 8 * kHalsChunk / W;
   double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
   if (it < h.iters) {
-    const double* p = h.partial + it;
+    const double* p = sets + it;
     int b = lane;
-    for (; b + 24 < h.nblk; b += 32) {
+    for (; b + 3 * lanes < n; b += 4 * lanes) {
       s0 += p[(int64_t)b * kHalsChunk];
-      s1 += p[(int64_t)(b + 8) * kHalsChunk];
-      s2 += p[(int64_t)(b + 16) * kHalsChunk];
-      s3 += p[(int64_t)(b + 24) * kHalsChunk];
+      s1 += p[(int64_t)(b + lanes) * kHalsChunk];
+      s2 += p[(int64_t)(b + 2 * lanes) * kHalsChunk];
+      s3 += p[(int64_t)(b + 3 * lanes) * kHalsChunk];
     }
-    for (; b < h.nblk; b += 8) s0 += p[(int64_t)b * kHalsChunk];
+    for (; b < n; b += lanes) s0 += p[(int64_t)b * kHalsChunk];
   }
-  part[lane][it] = (s0 + s1) + (s2 + s3);
+  part[threadIdx.x] = (s0 + s1) + (s2 + s3);
   if (threadIdx.x == 0) first = h.iters;
   __syncthreads();
   double sum = 0.0;
   if (lane == 0) {
+    for (int l = 0; l < lanes; l += 8)
 #pragma unroll
-    for (int l = 0; l < 8; ++l) sum += part[l][it];
-    part[0][it] = sum;
+      for (int x = 0; x < 8; ++x) sum += part[(l + x) * W + it];
+    part[it] = sum;
   }
   __syncthreads();
-  const double err0 = h.chunk == 0 ? part[0][0] : *h.err0;
+  const double err0 = h.chunk == 0 ? part[0] : *h.err0;
   if (lane == 0 && it < h.iters && sum < h.a.tol * err0) atomicMin(&first, it);
   __syncthreads();
   if (threadIdx.x != 0) return;
   const bool done = first < h.iters;
   if (h.chunk == 0) *h.err0 = err0;
   h.state[0] = done;
-  h.state[1] = h.chunk * kHalsChunk + (done ? first + 1 : h.iters);
+  h.state[1] = h.begin + (done ? first + 1 : h.iters);
   h.state[2] = h.chunk;
   h.state[3] = first + 1;
 }
 
-template <typename T, int RT, bool FULL>
+// Chunks grow from 16 iterations where one iteration of all rows takes more than
+// some 4 us (by R^2 and the rounds of workgroups on the GPU): there a rule that
+// fires early would leave most of a long chunk for nothing.  20000 rows, rank
+// 64, firing at the second of 100 iterations: 502 us so, 2263 with one chunk
+// (862 with a launch per iteration); never firing: 2227 and 2165.
+template <typename T, int RT, bool FULL, bool LOOP>
 static void hals_run(HalsRun h, int n_iter_max, hipStream_t st) {
-  for (int it = 0; it < n_iter_max; it += kHalsChunk) {
-    h.chunk = it / kHalsChunk;
-    h.iters = n_iter_max - it < kHalsChunk ? n_iter_max - it : kHalsChunk;
-    hals_run_kernel<T, RT, FULL><<<(unsigned)h.nblk, 64, 0, st>>>(h);
-    hals_decide_kernel<<<1, 8 * kHalsChunk, 0, st>>>(h);
+  const bool heavy = (int64_t)RT * RT * std::max<int64_t>(1024, (h.a.rows + kHalsRows - 1) / kHalsRows) > 1700000;
+  const bool sum = h.nblk > 1024;
+  int chunk = heavy ? 16 : kHalsChunk;
+  h.only = n_iter_max == 1;
+  for (h.begin = 0; h.begin < n_iter_max && !h.only; h.begin += h.iters, ++h.chunk) {
+    h.iters = std::min(chunk, n_iter_max - h.begin);
+    chunk = std::min(4 * chunk, kHalsChunk);
+    hals_run_kernel<T, RT, FULL, LOOP><<<(unsigned)h.nblk, 64, 0, st>>>(h);
+    if (sum) hals_sum_kernel<<<kHalsSums, kHalsChunk, 0, st>>>(h);
+    hals_decide_kernel<<<1, 8 * kHalsChunk, 0, st>>>(h, sum ? h.sums : h.partial, sum ? kHalsSums : h.nblk);
   }
+  if (h.only) h.iters = 1;
+  else --h.chunk;
   h.final = 1;
-  hals_run_kernel<T, RT, FULL><<<(unsigned)h.nblk, 64, 0, st>>>(h);
+  hals_run_kernel<T, RT, FULL, LOOP><<<(unsigned)h.nblk, 64, 0, st>>>(h);
 }
 
 template <typename T, int RT>
 static bool hals_try(const HalsRun& h, int n_iter_max, hipStream_t st) {
   if (h.a.R > RT) return false;
-  if (h.a.R == RT) hals_run<T, RT, true>(h, n_iter_max, st);
-  else hals_run<T, RT, false>(h, n_iter_max, st);
+  if (h.a.rows > (int64_t)kHalsBlocks * kHalsRows) hals_run<T, RT, false, true>(h, n_iter_max, st);
+  else if (h.a.R == RT) hals_run<T, RT, true, false>(h, n_iter_max, st);
+  else hals_run<T, RT, false, false>(h, n_iter_max, st);
   return true;
 }
 
@@ -385,9 +452,9 @@ static size_t hals_align(size_t b) { return (b + 255) & ~size_t(255); }
 constexpr int kHalsMaxIters = 1000;
 
 extern "C" size_t tla_hals_nnls_workspace_size(int64_t rows, int rank) {
-  const int64_t r = rows > 0 ? rows : 1, nb = (r + kHalsRows - 1) / kHalsRows;
-  return 2 * hals_align(size_t(r) * rank * 8) + hals_align(size_t(nb) * kHalsChunk * 8) + hals_align(16) +
-         hals_align(8);
+  const int64_t r = rows > 0 ? rows : 1, nb = std::min<int64_t>((r + kHalsRows - 1) / kHalsRows, kHalsBlocks);
+  return 2 * hals_align(size_t(r) * rank * 8) + hals_align(size_t(nb) * kHalsChunk * 8) +
+         hals_align(size_t(kHalsSums) * kHalsChunk * 8) + hals_align(16) + hals_align(8);
 }
 
 extern "C" int tla_hals_nnls(int dtype, void* factor, const void* mttkrp, int64_t rows, int rank,
@@ -417,8 +484,7 @@ extern "C" int tla_hals_nnls(int dtype, void* factor, const void* mttkrp, int64_
   const int rt = rank <= 16 ? 16 : rank <= 32 ? 32 : rank <= 48 ? 48 : 64;
   if (workspace && n_iter_max <= kHalsMaxIters) {
     TLA_REQUIRE(workspace_bytes >= tla_hals_nnls_workspace_size(rows, rank), "hals_nnls: workspace too small");
-    const int64_t nb = (rows + kHalsRows - 1) / kHalsRows;
-    TLA_REQUIRE(nb <= (int64_t)1 << 30, "hals_nnls: %lld rows", (long long)rows);
+    const int64_t nb = std::min<int64_t>((rows + kHalsRows - 1) / kHalsRows, kHalsBlocks);
     HalsRun h{};
     h.a = a;
     h.nblk = (int)nb;
@@ -427,7 +493,8 @@ extern "C" int tla_hals_nnls(int dtype, void* factor, const void* mttkrp, int64_
     h.vbuf[0] = (double*)w;
     h.vbuf[1] = (double*)(w + vb);
     h.partial = (double*)(w + 2 * vb);
-    h.state = (int*)(w + 2 * vb + hals_align(size_t(nb) * kHalsChunk * 8));
+    h.sums = (double*)(w + 2 * vb + hals_align(size_t(nb) * kHalsChunk * 8));
+    h.state = (int*)((char*)h.sums + hals_align(size_t(kHalsSums) * kHalsChunk * 8));
     h.err0 = (double*)((char*)h.state + hals_align(16));
     if (dtype == TLA_F32) hals_run_rank<float>(h, n_iter_max, st);
     else hals_run_rank<double>(h, n_iter_max, st);

@@ -157,3 +157,12 @@ def test_batched_launch_shape_checked_on_the_host():
     for waves in (1, 3, 16):
         assert call(waves, 32) == _lib.ERR_ARG
         assert b"waves" in lib.tla_last_error()
+
+
+def test_hals_scratch_of_many_rows():
+    """Two float64 copies of the factor and, for the error sums, no more than
+    65,536 workgroups' (64 MiB)."""
+    from tensorly_amd import _lib
+    lib = _lib.lib()
+    for rows, rank in ((1, 1), (1000, 64), (10 ** 8, 3), (2 ** 30, 1)):
+        assert lib.tla_hals_nnls_workspace_size(rows, rank) <= 16 * rows * rank + (65 << 20)

@@ -563,3 +563,33 @@ def test_hals_from_a_start_far_above_the_solution(cuda, rows, rank, n_iter, tol)
     ref = T.hals_nnls(M.cpu().numpy().T, utu, Fn[0].T.copy(), n_iter_max=n_iter, tol=tol).T
     _hals(F, M, n_iter, tol, torch.float64)
     np.testing.assert_allclose(F[0].cpu().numpy(), ref, rtol=1e-9, atol=1e-12 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("rows,rank,n_iter,tol", [(40, 64, 300, 1e-8), (40, 48, 100, 0.9), (40, 64, 100, 0.6), (17, 64, 9, 0.0),
+                                                  (110_000, 16, 30, 1e-8), (1_100_003, 3, 20, 1e-8), (1_100_003, 3, 100, 0.5),
+                                                  (33, 7, 1, 1e-8), (1_050_000, 1, 1, 0.5)])
+def test_hals_growing_chunks_and_many_rows(cuda, rows, rank, n_iter, tol):
+    """Chunks that grow from 8 iterations (long ones, and many rows), rules
+    that fire in one of them, more rows than workgroups, and single
+    iterations, against the oracle in FP64; tolerance as above."""
+    import numpy as np
+    from oracle import tensorly_np as T
+    g = torch.Generator(device=cuda).manual_seed(rows + rank)
+    F = [torch.rand((s, rank), generator=g, device=cuda, dtype=torch.float64) for s in (rows, 130, 110)]
+    M = torch.rand((rows, rank), generator=g, device=cuda, dtype=torch.float64) * 3 + 1
+    Fn = [f.cpu().numpy() for f in F]
+    utu = (Fn[1].T @ Fn[1]) * (Fn[2].T @ Fn[2])
+    ref = T.hals_nnls(M.cpu().numpy().T, utu, Fn[0].T.copy(), n_iter_max=n_iter, tol=tol).T
+    _hals(F, M, n_iter, tol, torch.float64)
+    np.testing.assert_allclose(F[0].cpu().numpy(), ref, rtol=1e-9, atol=1e-12 * np.abs(ref).max())
+
+
+def test_hals_rows_past_a_launch(cuda):
+    """2^30 rows: more than one launch has workgroups of 16 rows for.  At rank
+    1 every iteration gives max(m / u, 0)."""
+    rows = 2 ** 30 + 5
+    F = [torch.ones((rows, 1), device=cuda), torch.full((2, 1), 2.0, device=cuda), torch.full((2, 1), 0.5, device=cuda)]
+    M = torch.arange(rows, device=cuda, dtype=torch.float32).remainder_(64).sub_(16)[:, None]
+    iters = _hals(F, M, 2, 0.0, torch.float32)
+    wrong = int((F[0] != M.clamp_(min=0) / 4).sum())
+    assert iters == 2 and wrong == 0
