@@ -71,9 +71,17 @@ __global__ void ttm_generic_kernel(const T* __restrict__ X, int64_t Pa, int64_t 
   const int64_t j = t % J, a = t / J;
   const T* x = X + a * Im * Pb + b;
   const T* u = U + j * ldj;
-  T acc = 0;
-  for (int64_t m = 0; m < Im; ++m) acc += u[m * ldm] * x[m * Pb];
-  out[e] = acc;
+  // (four sums: shorter chains round less, and their loads are in flight together)
+  T s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+  int64_t m = 0;
+  for (; m + 4 <= Im; m += 4) {
+    s0 += u[m * ldm] * x[m * Pb];
+    s1 += u[(m + 1) * ldm] * x[(m + 1) * Pb];
+    s2 += u[(m + 2) * ldm] * x[(m + 2) * Pb];
+    s3 += u[(m + 3) * ldm] * x[(m + 3) * Pb];
+  }
+  for (; m < Im; ++m) s0 += u[m * ldm] * x[m * Pb];
+  out[e] = (s0 + s1) + (s2 + s3);
 }
 
 // ---------------------------------------------------------------------------
@@ -727,7 +735,8 @@ extern "C" int tla_mode_dot(int dtype, const void* X, int ndim, const int64_t* s
   // everything else in the tensor's own arithmetic; precision "valu" and the
   // sizes that the matrix kernels do not index stay on the vector ALU
   TtmPlan plan;
-  if ((dtype == TLA_F64 || precision != TLA_PREC_VALU) && ttm_any_plan(dtype == TLA_F64, Pa, Im, Pb, J, &plan))
+  if ((dtype == TLA_F64 || precision != TLA_PREC_VALU) && ttm_any_plan(dtype == TLA_F64, Pa, Im, Pb, J, &plan) &&
+      !plan.vector)
     return ttm_any_launch(dtype == TLA_F64, plan, X, Pa, Im, Pb, U, ldj, ldm, J, out, st);
   if (dtype == TLA_F32)
     ttm_generic_kernel<float><<<ceil_div(ne, 256), 256, 0, st>>>((const float*)X, Pa, Im, Pb, (const float*)U, J,

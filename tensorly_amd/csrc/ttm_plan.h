@@ -16,7 +16,36 @@ struct TtmPlan {
   int64_t tiles;  // cols: wave tiles of b per a
   bool split;     // cols: the block's waves share a tile and split m
   int64_t gx, gy;
+  bool vector;    // the vector kernel (one thread per output element) takes less
 };
+
+// Whether one thread per output element takes less than the plan's matrix
+// tiles: short runs b (a tile is 64 or 32 columns however few there are), few
+// rows j (a tile is 16) and short sums m.  Both estimated in ns from sweeps
+// over b = 1 ... 4096, m = 2 ... 512, j = 1 ... 64 at 64 and 128 MiB: a wave
+// costs a start and its steps over m, an output element a store and its
+// products (less where neighbouring lanes share X's lines).  Measured, float32,
+// vector / tiles: 2M x 2 x 4, mode 1, 1 row: 24 / 1115 us, 64 rows
+// 1490 / 4820; 8192 x 512 x 4, 8 / 16 rows: 91 / 124, 145 / 127; 819 x 5 x
+// 4096, 1 / 4 rows: 19 / 41, 58 / 46; 3.4M x 5, mode 1, 1 / 8 rows: 21 / 65,
+// 109 / 67.
+inline bool ttm_vector_wins(const TtmPlan& p, bool f64, int64_t Pa, int64_t Im, int64_t Pb, int64_t J) {
+  const double out = double(Pa) * J * Pb, waves = double(p.gx) * kTtmWaves * p.gy;
+  if (out > 4.2e9) return false;  // (past one launch)
+  if (Pb == 1) {
+    if (Im > 8) return false;
+    const double tiles = waves * ((f64 ? 1.1 : 0.85) + 0.1 * Im);
+    const double vector = out * (f64 ? 0.0024 + 0.00055 * Im : 0.0013 + 0.00065 * Im);
+    return vector + 1000 < tiles;
+  }
+  const double steps = double((Im + 15) / 16) / (p.split ? kTtmWaves : 1);
+  const double start[2][4] = {{0.2, 0.4, 0.75, 1.1}, {0.25, 0.6, 0.85, 1.1}};  // by JT
+  const double step[2][4] = {{0.43, 0.63, 0.9, 1.19}, {0.34, 0.66, 1.0, 1.31}};
+  const double tiles = waves * (p.TN == 1 ? start[f64][p.JT - 1] + step[f64][p.JT - 1] * steps
+                                          : (f64 ? 0.5 : 0.55) * p.JT + (f64 ? 0.7 : 0.72) * p.JT * steps);
+  const double vector = out * (f64 ? 0.002 + 0.00075 * Im : 0.0017 + (Pb % 4 == 0 ? 0.00053 : Im <= 8 ? 0.0007 : 0.0012) * Im);
+  return std::max(vector, 100.0 * Im) + 1000 < tiles;  // (a chain of Im loads)
+}
 
 // Fills *p and returns true when ttm_any_launch takes these sizes.
 inline bool ttm_any_plan(bool f64, int64_t Pa, int64_t Im, int64_t Pb, int64_t J, TtmPlan* p) {
@@ -39,16 +68,19 @@ inline bool ttm_any_plan(bool f64, int64_t Pa, int64_t Im, int64_t Pb, int64_t J
     const int most = p->JT <= 2 ? 4 : 2;
     p->TN = rows16 * p->gy >= most * 4096 ? most : 1;
     p->gx = (rows16 + kTtmWaves * p->TN - 1) / (kTtmWaves * p->TN);
+    p->vector = ttm_vector_wins(*p, f64, Pa, Im, Pb, J);
     return grid_fits(p->gx, 64 * kTtmWaves);
   }
   const int most = p->JT <= 2 ? 2 : 1;  // accumulators of 2 tiles fit the register file
   const int64_t narrow = (Pb + 16 * VL - 1) / (16 * VL), wide = (Pb + 16 * VL * most - 1) / (16 * VL * most);
   if (Pa > kBig || narrow > kBig / Pa) return false;
-  p->TN = Pa * wide * p->gy < 4096 ? 1 : most;
+  // (a second tile that is mostly padding costs as much as the first)
+  p->TN = Pa * wide * p->gy < 4096 || 4 * wide * most > 5 * narrow ? 1 : most;
   p->tiles = p->TN == 1 ? narrow : wide;
   const int64_t tiles = Pa * p->tiles;
   p->split = tiles * p->gy < 4096 && Im > 32;
   p->gx = p->split ? tiles : (tiles + kTtmWaves - 1) / kTtmWaves;
+  p->vector = ttm_vector_wins(*p, f64, Pa, Im, Pb, J);
   return grid_fits(p->gx, 64 * kTtmWaves);
 }
 

@@ -20,7 +20,7 @@ int main() {
   while (std::scanf("%lld %lld %lld %lld %lld", &f64, &Pa, &Im, &Pb, &J) == 5) {
     tla::TtmPlan p;
     const bool ok = tla::ttm_any_plan(f64, Pa, Im, Pb, J, &p);
-    std::printf("%d %d %d %lld %d %lld %lld\n", ok, p.JT, p.TN, (long long)p.tiles, p.split, (long long)p.gx, (long long)p.gy);
+    std::printf("%d %d %d %lld %d %lld %lld %d\n", ok, p.JT, p.TN, (long long)p.tiles, p.split, (long long)p.gx, (long long)p.gy, p.vector);
   }
 }
 """
@@ -63,7 +63,7 @@ def compiled(tmp_path_factory, name, text):
 @pytest.fixture(scope="module")
 def ttm_plan(tmp_path_factory):
     ask = compiled(tmp_path_factory, "ttm", TTM)
-    keys = ("ok", "JT", "TN", "tiles", "split", "gx", "gy")
+    keys = ("ok", "JT", "TN", "tiles", "split", "gx", "gy", "vector")
     return lambda rows: [dict(zip(keys, r)) for r in ask(rows)]
 
 
@@ -148,3 +148,20 @@ def test_mttkrp_tiles_of_long_modes(any_plan):
     rows = [(0, (200_000, 30, 41), 16, 0, 0), (0, (1_000_000, 7, 9), 16, 0, 1), (1, (100_000, 33, 35), 20, 0, 0),
             (0, (5, 9, 500_001), 8, 2, 0), (0, (9, 70_001, 31), 33, 1, 1)]
     assert all(p["TN"] >= 2 for p in any_plan(rows))
+
+
+def test_mode_dot_short_runs_keep_the_vector_kernel(ttm_plan):
+    """Tiles that would be mostly padding: short contiguous runs, few rows,
+    short sums; and not where the tiles are full."""
+    vector = [(0, 2_000_000, 4, 4, 1), (1, 2_000_000, 4, 4, 1), (0, 100_000, 2, 4, 2), (1, 100_000, 2, 4, 2),
+              (0, 1, 2, 3_000_000, 1), (0, 1_000_000, 5, 1, 1), (0, 262_144, 16, 4, 4)]
+    tiles = [(0, 1, 256, 65536, 32), (0, 256, 256, 256, 32), (0, 65536, 256, 1, 32), (0, 250, 30, 20, 331),
+             (1, 25, 331, 190, 30), (0, 82_750, 190, 1, 20), (0, 82_750, 20, 1, 190), (0, 100, 100, 100, 16)]
+    assert all(p["vector"] for p in ttm_plan(vector))
+    assert not any(p["vector"] for p in ttm_plan(tiles))
+
+
+def test_mode_dot_narrow_runs_take_one_tile(ttm_plan):
+    rows = [(0, 100_000, 64, 64, 16), (0, 100_000, 64, 4, 16), (1, 100_000, 64, 32, 16), (0, 100_000, 64, 130, 16)]
+    assert all(p["TN"] == 1 for p in ttm_plan(rows))
+    assert ttm_plan([(0, 100_000, 64, 128, 16)])[0]["TN"] == 2
