@@ -1373,8 +1373,10 @@ static int make_plan(int x_dtype, int ndim, const int64_t* shape, int R, int kb,
   auto unaligned = [&]() -> int {
     p->path = Path::Generic;
     p->ws_bytes = 0;
-    if ((x_dtype == TLA_F64 || prec_ok(x_dtype, precision)) &&
-        any_plan(x_dtype == TLA_F64, ndim, shape, R, kb, true, &p->any)) {
+    const bool f64 = x_dtype == TLA_F64;
+    AnyPlan bare;  // (a call without weights may have less to do)
+    if ((f64 || prec_ok(x_dtype, precision)) && any_plan(f64, ndim, shape, R, kb, true, &p->any) &&
+        !(p->any.vector && any_plan(f64, ndim, shape, R, kb, false, &bare) && bare.vector)) {
       p->path = Path::Any;
       p->out_rows = shape[kb];
       p->ws_bytes = p->any.ws_bytes;
@@ -1802,10 +1804,12 @@ static int run_plan(const Plan& p0, int x_dtype, const void* X, int ndim, const 
   }
   if (p.path == Path::Any && ws_bytes >= p.ws_bytes && (ws || p.ws_bytes == 0)) {
     any_plan(x_dtype == TLA_F64, ndim, shape, R, kb, weights != nullptr, &p.any);
-    const bool takes = job && job->R > 0 && any_takes_job(p.any, R);
-    if (job_taken) *job_taken = takes;
-    return any_launch(x_dtype == TLA_F64, p.any, X, ndim, shape, factors, weights, R, kb, out, ws,
-                      takes ? job : nullptr, st);
+    if (!p.any.vector) {
+      const bool takes = job && job->R > 0 && any_takes_job(p.any, R);
+      if (job_taken) *job_taken = takes;
+      return any_launch(x_dtype == TLA_F64, p.any, X, ndim, shape, factors, weights, R, kb, out, ws,
+                        takes ? job : nullptr, st);
+    }
   }
   // (a caller with less scratch than the plan's gets the vector kernel, which needs none)
   if (p.path == Path::Generic || p.path == Path::Any) {

@@ -67,9 +67,7 @@ struct AnyRowsArgs {
   int64_t In, Q;
   int K, Pb;
   int R, ldr;       // columns of this slab, row stride of the factors
-  const T* G;       // rows g0, ... of the A Pb scale rows, nullable
-  int64_t g0;
-  int ldg;
+  const T* G;       // (A Pb) x ldr scale rows (a slice of them, from where row 0 would be), nullable
   AnyGArgs<T> ga;   // GD: the factors of G instead
   const T* Fk;      // K x ldr
   T* partial;       // [nblk][In][R]
@@ -98,7 +96,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
   uint32_t rr[RT];  // rank columns, in bytes; those past the slab read its last one
 #pragma unroll
   for (int n = 0; n < RT; ++n) rr[n] = min(n * 16 + c, R - 1) * sizeof(T);
-  const uint32_t ldb = a.ldr * sizeof(T), ldgb = a.ldg * sizeof(T);
+  const uint32_t ldb = a.ldr * sizeof(T);
   Acc acc[TN * RT];
 #pragma unroll
   for (int n = 0; n < TN * RT; ++n) acc[n] = Acc{0, 0, 0, 0};
@@ -135,10 +133,10 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, false, sizeof(T) ==
     const int q = left > 0 ? q0 + NV * g : (int)Q - 1;
     const int b0 = q / K;
     int k0 = q - b0 * K;
-    const T* Gb = !GD && a.G ? a.G + (ia * a.Pb - a.g0) * a.ldg : nullptr;
+    const T* Gb = !GD && a.G ? a.G + ia * a.Pb * a.ldr : nullptr;
     auto scale = [&](int b, uint32_t rb) -> T {
       if constexpr (GD) return g_entry(a.ga, (uint32_t)ia * a.Pb + b, rb, ldb);
-      else return Gb ? at<T>(Gb, b * ldgb + rb) : (T)1;
+      else return Gb ? at<T>(Gb, b * ldb + rb) : (T)1;
     };
     if (K >= NV) {
       const int b1 = min(b0 + 1, a.Pb - 1);
@@ -204,8 +202,7 @@ struct AnyLastArgs {
   int64_t P, K;
   int J, nG;    // P = nG J
   int R, ldr;
-  const T* G;   // rows g0, ... of the P / J scale rows, nullable
-  int g0, ldg;
+  const T* G;   // (P / J) x ldr scale rows (a slice of them, from where row 0 would be), nullable
   AnyGArgs<T> ga;  // GD: the factors of G instead
   const T* Fj;  // J x ldr
   T* partial;   // [nblk][K][R]
@@ -236,7 +233,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
   uint32_t rr[RT];  // rank columns, in bytes; those past the slab read its last one
 #pragma unroll
   for (int n = 0; n < RT; ++n) rr[n] = min(n * 16 + c, R - 1) * sizeof(T);
-  const uint32_t ldb = a.ldr * sizeof(T), ldgb = a.ldg * sizeof(T);
+  const uint32_t ldb = a.ldr * sizeof(T);
   Acc acc[TN * VL * RT];
 #pragma unroll
   for (int n = 0; n < TN * VL * RT; ++n) acc[n] = Acc{0, 0, 0, 0};
@@ -271,7 +268,7 @@ __global__ __launch_bounds__(64 * kAnyWaves, any_occ(TN, RT, true, sizeof(T) == 
     int j0 = (int)(p - (uint32_t)a0 * J);
     auto scale = [&](int i, uint32_t rb) -> T {
       if constexpr (GD) return g_entry(a.ga, (uint32_t)i, rb, ldb);
-      else return a.G ? at<T>(a.G, (i - a.g0) * ldgb + rb) : (T)1;
+      else return a.G ? at<T>(a.G, i * ldb + rb) : (T)1;
     };
     if (J >= NR) {
       const int a1 = min(a0 + 1, a.nG - 1);
@@ -376,13 +373,14 @@ __global__ __launch_bounds__(256) void any_reduce_kernel(const T* __restrict__ p
   }
 }
 
-// Rows g0, ... of the table, ld columns of the factors' R.
+// Rows g0, ... of the table, `cols` of its R columns.
 template <typename T>
-__global__ void any_g_kernel(AnyGArgs<T> a, int64_t g0, int ld, T* __restrict__ out) {
+__global__ void any_g_kernel(AnyGArgs<T> a, int64_t g0, int cols, T* __restrict__ out) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= a.rows * ld) return;
-  const int r = (int)(e % ld);
-  int64_t q = g0 + e / ld;
+  if (e >= a.rows * cols) return;
+  const int r = (int)(e % cols);
+  const int64_t row = e / cols;
+  int64_t q = g0 + row;
   T v = a.weights ? a.weights[r] : (T)1;
 #pragma unroll
   for (int m = kMaxOrder - 1; m >= 0; --m)
@@ -391,7 +389,7 @@ __global__ void any_g_kernel(AnyGArgs<T> a, int64_t g0, int ld, T* __restrict__ 
       q /= a.sz[m];
       v *= a.fac[m][i * a.R + r];
     }
-  out[e] = v;
+  out[row * a.R + r] = v;
 }
 
 template <typename T, int RT>
@@ -438,7 +436,7 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
   for (int r0 = 0; r0 < R; r0 += 64) {
     const int Rs = std::min(64, R - r0), RT = (Rs + 15) / 16;
     const bool direct = sets == 1 && Rs == R;
-    T* const sums = direct ? out : (T*)((char*)ws + (table ? any_align(size_t(p.g_slice) * std::min(R, 64) * sizeof(T)) : 0));
+    T* const sums = direct ? out : (T*)((char*)ws + (table ? any_align(size_t(p.g_slice) * R * sizeof(T)) : 0));
     AnyGArgs<T> gs = ga;  // of this slab's columns
     if (gs.weights) gs.weights += r0;
     for (int m = 0; m < gs.n; ++m) gs.fac[m] += r0;
@@ -450,7 +448,6 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
       T* part = sums + s * p.nblk * p.In * Rs;
       const T* G = nullptr;
       int64_t g0 = 0;
-      int ldg = R;
       if (table) {
         // the rows of chunks c0, ..., c1 - 1 and the one after
         int64_t g1 = p.g_rows;
@@ -465,18 +462,25 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
           }
         }
         TLA_REQUIRE(g1 - g0 <= p.g_slice, "scale table of %lld rows", (long long)(g1 - g0));
-        gs.rows = g1 - g0;
-        ldg = Rs;
-        const int64_t ne = gs.rows * Rs;
-        any_g_kernel<T><<<(unsigned)((ne + 255) / 256), 256, 0, st>>>(gs, g0, Rs, (T*)ws);
-        TLA_LAUNCH_CHECK();
-        G = (const T*)ws;
+        // one slice holds every slab's columns; of several, each is made again
+        // for a slab
+        const bool whole = p.slices == 1;
+        if (!whole || r0 == 0) {
+          AnyGArgs<T> gt = whole ? ga : gs;
+          const int cols = whole ? R : Rs;
+          gt.rows = g1 - g0;
+          const int64_t ne = gt.rows * cols;
+          any_g_kernel<T><<<(unsigned)((ne + 255) / 256), 256, 0, st>>>(gt, g0, cols, (T*)ws + (whole ? 0 : r0));
+          TLA_LAUNCH_CHECK();
+        }
+        // (row 0 lies before the buffer where the slice begins later)
+        G = (const T*)((uintptr_t)ws + uintptr_t(r0 - g0 * R) * sizeof(T));
       } else if (p.g_rows > 0 && !p.direct_g) {
         G = gs.fac[0];
       }
       const AnyGArgs<T> gd = p.direct_g ? gs : AnyGArgs<T>{};  // R = 0: not used
       if (p.last) {
-        AnyLastArgs<T> a{X,  p.A, p.K,  (int)p.J, (int)(p.A / p.J), Rs, R, G, (int)g0, ldg, gd,
+        AnyLastArgs<T> a{X,  p.A, p.K,  (int)p.J, (int)(p.A / p.J), Rs, R, G, gd,
                          (const T*)factors[own] + r0, part, c0, c1, p.nblk};
         switch (RT) {
           case 1: any_run_last<T, 1>(p.TN, grid, a, st); break;
@@ -485,7 +489,7 @@ static int any_launch_t(const AnyPlan& p, const T* X, int ndim, const int64_t* s
           default: any_run_last<T, 4>(p.TN, grid, a, st); break;
         }
       } else {
-        AnyRowsArgs<T> a{X, p.In, p.Q, (int)p.K, (int)p.Pb, Rs, R, G, g0, ldg, gd, (const T*)factors[own] + r0, part,
+        AnyRowsArgs<T> a{X, p.In, p.Q, (int)p.K, (int)p.Pb, Rs, R, G, gd, (const T*)factors[own] + r0, part,
                          p.nqc, c0, c1, p.nblk};
         switch (RT) {
           case 1: any_run_rows<T, 1>(p.TN, grid, a, st); break;

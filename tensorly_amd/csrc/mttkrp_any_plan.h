@@ -40,7 +40,33 @@ struct AnyPlan {
   bool build_g;       // the table has to be built (else it is a factor itself, or absent)
   bool direct_g;      // ... but its rows are formed in the kernel
   size_t ws_bytes;
+  bool vector;        // the vector kernel (a workgroup per output row and 16 ranks) takes less
 };
+
+// Whether the vector kernel takes less, which needs no table, no sum of partials
+// and no second slab: few contracted indices q per output row, many short modes,
+// ranks above 64.  Both estimated in us from 954 calls of 2^4 to 2^19 entries,
+// orders 2 to 6, ranks 1 to 130 (the median of either within a tenth): the
+// vector kernel's passes of 256 q, times order and ranks, in rounds of 512
+// workgroups (256 where that is all a matrix product); launches, chunks per wave, and a chunk's scale rows (formed in the
+// kernel, GD, or read; one by one where the inner mode is shorter than a lane's
+// values).  Measured, vector / matrix, GPU time: 4 x 2 x 2 x 2 x 2 x 7, rank 100, mode 3: 14 / 133
+// us; 16 x 50 x 3, rank 65, mode 1: 11 / 53; 26 x 24 x 8, rank 3, mode 1: 8 / 6;
+// 14 x 27 x 5 x 5, rank 64, mode 2: 55 / 20.
+inline bool any_vector_wins(const AnyPlan& p, bool f64, int ndim, int R, bool weights) {
+  const int Rs = R < 64 ? R : 64, slabs = (R + 63) / 64;
+  const double passes = double((p.A * p.Q + 255) / 256), blocks = double(p.In) * ((R + 15) / 16);
+  const double vector = 6 + passes * ndim * (0.3 + 0.065 * std::min(R, 16)) * std::max(1.0, blocks / (ndim == 2 ? 256 : 512));
+  const int NR = p.last ? any_last_rows(p.TN, p.RT) : f64 ? 4 : 8;
+  const bool table = p.build_g && !p.direct_g;
+  const int64_t sets = p.nblk * p.slices;
+  const double launches = (!table ? 0 : p.slices == 1 ? 1 : p.slices * slabs) + slabs * (p.slices + (sets > 1 || R > 64 ? 1 : 0));
+  const double visits = double((p.per + kAnyWaves * p.nblk - 1) / (kAnyWaves * p.nblk)) * p.slices * slabs;
+  const double scales = double((Rs + 15) / 16) * ((p.last ? p.J : p.K) < NR ? NR : 2);
+  const double matrix = 3.1 * launches + visits * (0.93 + 0.0165 * p.RT * NR +
+                        (p.direct_g ? 0.099 * scales * (ndim - 2 + weights) : p.g_rows > 0 ? 0.041 * scales : 0.0));
+  return vector < 0.95 * matrix;
+}
 
 inline size_t any_align(size_t b) { return (b + 255) & ~size_t(255); }
 
@@ -131,7 +157,7 @@ inline bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, 
   p->slices = 1;
   p->per = p->nchunks;
   p->g_slice = p->g_rows;
-  const int64_t most_rows = (int64_t(256) << 20) / (Rs * sz);
+  const int64_t most_rows = (int64_t(256) << 20) / (R * sz);
   if (p->build_g && !p->direct_g && p->g_rows > most_rows) {
     const int64_t span = p->last ? 4 * any_last_rows(p->TN, p->RT) : 8 * V;  // p or q of a chunk
     const int64_t inner = p->last ? p->J : p->K;                            // ... that share a row
@@ -154,8 +180,9 @@ inline bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, 
   p->nblk = std::max<int64_t>(1, std::min<int64_t>(p->nblk, (int64_t(32) << 20) / set / p->slices));
   const int64_t sets = p->nblk * p->slices;
   if (!grid_fits(p->groups * p->nblk, 64 * kAnyWaves) || !grid_fits((p->In * Rs + 31) / 32 + 1, 256)) return false;
-  p->ws_bytes = (p->build_g && !p->direct_g ? any_align(size_t(p->g_slice) * Rs * sz) : 0) +
+  p->ws_bytes = (p->build_g && !p->direct_g ? any_align(size_t(p->g_slice) * R * sz) : 0) +
                 (sets > 1 || R > 64 ? any_align(size_t(sets) * set) : 0);
+  p->vector = any_vector_wins(*p, f64, ndim, R, weights);
   return true;
 }
 

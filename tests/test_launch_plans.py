@@ -40,8 +40,8 @@ int main() {
     }
     tla::AnyPlan p;
     const bool ok = tla::any_plan(f64, n, shape, R, mode, weights, &p);
-    std::printf("%d %d %d %d %lld %lld %lld %lld %d %d %zu\n", ok, p.last, p.TN, p.RT, (long long)p.groups,
-                (long long)p.slices, (long long)p.nblk, (long long)p.nchunks, p.build_g, p.direct_g, p.ws_bytes);
+    std::printf("%d %d %d %d %lld %lld %lld %lld %d %d %zu %d\n", ok, p.last, p.TN, p.RT, (long long)p.groups,
+                (long long)p.slices, (long long)p.nblk, (long long)p.nchunks, p.build_g, p.direct_g, p.ws_bytes, p.vector);
   }
 }
 """
@@ -100,7 +100,7 @@ def test_mode_dot_plans_cover_every_output(ttm_plan):
 @pytest.fixture(scope="module")
 def any_plan(tmp_path_factory):
     ask = compiled(tmp_path_factory, "any", ANY)
-    keys = ("ok", "last", "TN", "RT", "groups", "slices", "nblk", "nchunks", "build_g", "direct_g", "ws")
+    keys = ("ok", "last", "TN", "RT", "groups", "slices", "nblk", "nchunks", "build_g", "direct_g", "ws", "vector")
     return lambda rows: [dict(zip(keys, r)) for r in ask([(f, R, m, w, len(s), *s) for f, s, R, m, w in rows])]
 
 
@@ -165,3 +165,14 @@ def test_mode_dot_narrow_runs_take_one_tile(ttm_plan):
     rows = [(0, 100_000, 64, 64, 16), (0, 100_000, 64, 4, 16), (1, 100_000, 64, 32, 16), (0, 100_000, 64, 130, 16)]
     assert all(p["TN"] == 1 for p in ttm_plan(rows))
     assert ttm_plan([(0, 100_000, 64, 128, 16)])[0]["TN"] == 2
+
+
+def test_mttkrp_of_little_work_keeps_the_vector_kernel(any_plan):
+    """Few contracted indices, many short modes, ranks above 64; and not
+    where a launch or two of the matrix kernels do more."""
+    vector = [(0, (4, 2, 2, 2, 2, 7), 100, 3, 1), (0, (16, 50, 3), 65, 1, 1), (1, (2, 8, 9, 2), 100, 2, 1),
+              (0, (6, 4), 100, 1, 1), (0, (8, 26, 15, 6), 17, 1, 1), (1, (13, 14, 13), 100, 1, 1)]
+    matrix = [(0, (32, 12, 10, 30), 3, m, 0) for m in range(4)] + [(0, (257, 301, 203), 20, m, 0) for m in range(3)]
+    matrix += [(0, (149, 120, 90), 10, m, 1) for m in range(3)] + [(0, (14, 27, 5, 5), 64, 2, 1), (1, (40, 50, 60), 70, 0, 1)]
+    assert all(p["vector"] for p in any_plan(vector))
+    assert not any(p["vector"] for p in any_plan(matrix))
