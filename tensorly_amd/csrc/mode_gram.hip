@@ -12,7 +12,7 @@
 //    tiles; the two operands order the columns alike, so any order will do.
 //  * mode_gram_last_kernel (the contiguous mode): two consecutive rows i per
 //    lane and column, so a column's 32 rows are one piece of memory.
-//  * mode_gram_short_kernel (runs of 2 to 13 columns b, where the pieces would
+//  * mode_gram_short_kernel (runs of 2 to 13 and 17 to 24 columns b, where the pieces would
 //    be padding; 512 x 512 x 8, mode 1: 66 us against 108 of the pieces, x 12:
 //    90 against 97, x 15: 117 against 103): column by column through LDS, one
 //    matrix tile per wave.
@@ -283,13 +283,20 @@ struct GramPlan {
   int splits;
 };
 
-static GramPlan gram_plan(int64_t Pa, int64_t In, int64_t Pb) {
+static GramPlan gram_plan(bool f64, int64_t Pa, int64_t In, int64_t Pb) {
   const int64_t Q = Pa * Pb, nt = (In + 31) / 32, tiles = nt * (nt + 1) / 2;
   GramPlan p;
   // 32-bit offsets: the bytes of a tile's 32 rows, or of four columns
   constexpr int64_t kBig = 0x7fffff00;
+  // Runs of 17 to 24 columns leave a second piece that is mostly padding (300 rows,
+  // float32, 17 / 20 / 24 columns: 42 / 39 / 36 us, short 34 / 32 / 33; from 25 on,
+  // float64 from 22, the pieces win).  Float64 rows that begin off the 16-byte grid: past some 90 MB
+  // the pieces' loads fetch too many lines twice (3000 x 4001 / 3 x 3000 x 2049:
+  // 1118 / 2222 us, short 996 / 1568; 2048 x 4001: 543, short 594).
+  const bool padded = Pb >= 17 && Pb <= (f64 ? 21 : 24);
+  const bool astray = f64 && Pb % 2 != 0 && tiles >= 2048 && Q > (int64_t(90) << 20) / 8 / In;
   if (Pb == 1 && In >= 2 && In <= kBig / 64 && tiles <= 65535) p.kind = GramPlan::Last;
-  else if (Pb >= 14 && Pb <= kBig / (33 * 8) && tiles <= 65535) p.kind = GramPlan::Rows;
+  else if (!padded && !astray && Pb >= 14 && Pb <= kBig / (33 * 8) && tiles <= 65535) p.kind = GramPlan::Rows;
   else p.kind = GramPlan::Short;
   if (p.kind == GramPlan::Short) {
     int64_t s = std::max<int64_t>(1, 1024 / std::max<int64_t>(tiles, 1));
@@ -302,10 +309,12 @@ static GramPlan gram_plan(int64_t Pa, int64_t In, int64_t Pb) {
   // that many.  About two per CU, as each adds a partial tile to write and
   // sum (1000 x 1000: 36 us, with eight per CU 46), but eight where that
   // leaves a block 64 pieces, for an even finish (256^3 123-133 -> 107-114 us,
-  // 512^3 1.9 -> 1.5 ms).  At most 128: their sum is a serial chain.
+  // 512^3 1.9 -> 1.5 ms), or three (what float64 keeps in flight; 3 x 600 x 2049:
+  // 90 -> 66 us, float32 76 -> 62).  At most 128: their sum is a serial chain.
   const int64_t pieces = p.kind == GramPlan::Last ? (Q + 15) / 16 : Pa * ((Pb + 15) / 16);
-  const int64_t blocks = pieces / 64 >= 2048 / std::max<int64_t>(tiles, 1) ? 2048 : 576;
-  int64_t s = std::min<int64_t>({(pieces + 7) / 8, std::max<int64_t>(1, blocks / std::max<int64_t>(tiles, 1)), 128});
+  const int64_t nt1 = std::max<int64_t>(tiles, 1);
+  const int64_t blocks = pieces / 64 >= 2048 / nt1 ? 2048 : pieces / 48 >= 768 / nt1 ? 768 : 576;
+  int64_t s = std::min<int64_t>({(pieces + 7) / 8, std::max<int64_t>(1, blocks / nt1), 128});
   if (s > 8) s = s / 8 * 8;
   p.splits = (int)std::max<int64_t>(1, s);
   p.chunk = (pieces + p.splits - 1) / p.splits;
@@ -339,7 +348,8 @@ extern "C" size_t tla_mode_gram64_workspace_size(int ndim, const int64_t* shape,
   if (mode < 0 || mode >= ndim) return 0;
   int64_t Pa, In, Pb;
   gram_sizes(ndim, shape, mode, Pa, In, Pb);
-  return (size_t(gram_plan(Pa, In, Pb).splits) * In * In * 8 + 255) & ~size_t(255);
+  const int splits = std::max(gram_plan(false, Pa, In, Pb).splits, gram_plan(true, Pa, In, Pb).splits);
+  return (size_t(splits) * In * In * 8 + 255) & ~size_t(255);
 }
 
 extern "C" int tla_mode_gram64(int dtype, const void* X, int ndim, const int64_t* shape, int mode, double* G,
@@ -349,7 +359,7 @@ extern "C" int tla_mode_gram64(int dtype, const void* X, int ndim, const int64_t
   TLA_REQUIRE(ws_bytes >= tla_mode_gram64_workspace_size(ndim, shape, mode), "mode_gram64: workspace too small");
   int64_t Pa, In, Pb;
   gram_sizes(ndim, shape, mode, Pa, In, Pb);
-  const GramPlan p = gram_plan(Pa, In, Pb);
+  const GramPlan p = gram_plan(dtype == TLA_F64, Pa, In, Pb);
   hipStream_t st = (hipStream_t)stream;
   // one chunk is the result itself
   double* out = p.splits == 1 ? G : (double*)ws;

@@ -593,3 +593,19 @@ def test_hals_rows_past_a_launch(cuda):
     iters = _hals(F, M, 2, 0.0, torch.float32)
     wrong = int((F[0] != M.clamp_(min=0) / 4).sum())
     assert iters == 2 and wrong == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(33, 16), (33, 17), (33, 21), (33, 22), (33, 24), (33, 25), (7, 34, 20), (7, 34, 23),
+                                   (2, 65, 37), (2049, 5801), (2049, 5802), (3, 600, 515)])
+def test_mode_gram_rules(cuda, shape, dtype):
+    """Both sides of the rules on the length of the runs and on float64 rows
+    off the 16-byte grid: sums of n products of float64, and as much for the
+    reference's own."""
+    from tensorly_amd.svd import mode_gram
+    x = torch.randn(shape, dtype=dtype, generator=torch.Generator().manual_seed(len(shape))).to(cuda)
+    m = len(shape) - 2
+    u = torch.movedim(x, m, 0).reshape(shape[m], -1).double()
+    bound = 2 * 2.3e-16 * u.shape[1] * (u.abs() @ u.abs().T)
+    worst = float(((mode_gram(x, m) - u @ u.T).abs() - bound).max())
+    assert worst <= 0
