@@ -6,9 +6,9 @@
 // of its eigenvalues.
 //
 //  * n <= 128: tridiagonalisation, Sturm counts and twisted factorisations
-//    (direct_eig); where eigenvalues cluster, cyclic Jacobi on the whole
-//    matrix (round-robin pair ordering, all n/2 rotations of a round applied
-//    in parallel).
+//    (direct_eig), or QR steps where eigenvalues cluster (direct_qr); outside
+//    their range cyclic Jacobi on the whole matrix (round-robin pair ordering,
+//    all n/2 rotations of a round applied in parallel).
 //  * n  > 128: block subspace iteration with Rayleigh-Ritz, block b = 48 for
 //    k <= 40, 64 for k <= 56 or 128 for k <= 120.  Each step: Z = G V, H = V^T Z on FP64
 //    MFMA, H = W diag(t) W^T (perturbation theory where the previous Ritz
@@ -630,11 +630,12 @@ __device__ void sort_desc(const double* A, int m, int* order) {
 //  4. Back transformation, eight lanes per column.
 //  5. One Newton step towards orthonormal columns, Z <- Z (3 I - Z^T Z) / 2.
 //
-// Returns false, with nothing but scratch written, when a residual exceeds
-// 1e-13 of the norm or the vectors before step 5 are not orthogonal to 1e-8
-// (clusters of eigenvalues, where the vectors of one are not determined by
-// their own value): the caller then takes the Jacobi sweeps, which need no
-// separation.  The FP64 instructions that one workgroup issues bound it, most
+// When a residual exceeds 1e-13 of the norm or the vectors before step 5 are
+// not orthogonal to 1e-8 (clusters of eigenvalues, where the vectors of one are
+// not determined by their own value) direct_qr takes steps 2 to 5's place, from
+// the same reflectors.  Returns false, with nothing but scratch written, for
+// NaN and norms outside [1e-200, 1e150]: the caller then takes the Jacobi
+// sweeps.  The FP64 instructions that one workgroup issues bound it, most
 // of all in 1 (1.1 us a step up to 64 rows, 1.7 above).  Measured, one call:
 // n = 120, k = 10: 317 us against 9.4 ms of Jacobi sweeps; n = 128, k = 128:
 // 605 us against 11.0 ms; n = 48, k = 10: 90 us against 825; a 48 x 48 Ritz
@@ -647,8 +648,7 @@ struct DirectLds {
   double vbuf[kEigWaves][N];  // per wave; then the intervals of the eigenvalues
   double wbuf[kEigWaves][N];  // per wave; then gamma and norms
   double pbuf[4][N];          // then the Sturm counts
-  double bound[2];
-  int ok;
+  int ok;                     // 2: the matrix is diagonal
 };
 
 template <>
@@ -721,6 +721,129 @@ __device__ __forceinline__ void direct_back(const double* Vh, double* Z, int ldZ
   }
 }
 
+// place[i] = the place of d[i] in descending order (of equal ones, the first
+// first).  Begins and ends with a barrier.
+__device__ __forceinline__ void descending(const double* d, int n, int* place) {
+  __syncthreads();
+  const int tid = threadIdx.x;
+  if (tid < n) {
+    const double t = d[tid];
+    int rank = 0;
+    for (int i = 0; i < n; ++i) rank += d[i] > t || (d[i] == t && i < tid);
+    place[tid] = rank;
+  }
+  __syncthreads();
+}
+
+// All eigenpairs of the tridiagonal matrix in L.d, L.e by implicit QR steps
+// with Wilkinson's shift (Golub and Van Loan, Matrix Computations, 8.3), for
+// clusters whose vectors the twisted factorisations cannot tell apart: they
+// need no separation.  Each of NB waves holds 64 components of every vector and
+// runs the scalar recurrence for itself, so nothing waits for anything; the
+// chain of one rotation after another bounds it.  Off-diagonal entries are
+// dropped below 1.1e-16 of the norm.  Takes the reflectors in Vh and overwrites
+// them; leaves the ne leading pairs in Z and theta, or returns false after 40 n
+// steps (or for NaN).  Clusters of four, n = 128 / 64 / 16, with the attempt
+// before it: 2530 / 602 / 77 us; Jacobi sweeps instead of both 15.5 ms / 1989 / 167.
+template <int NB>
+__device__ bool direct_qr(int n, int ne, double norm, double* Vh, double* Z, int ldZ, double* theta,
+                                       DirectLds<NB>& L) {
+  constexpr int N = 64 * NB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const double sc = ldexp(1.0, -ilogb(norm)), tol = 1.1e-16;
+  // the product of the reflectors, transposed into Vh
+  for (int e = tid; e < n * n; e += kEigThreads) Z[(e / n) * ldZ + e % n] = e / n == e % n ? 1.0 : 0.0;
+  __syncthreads();
+  direct_back<NB>(Vh, Z, ldZ, n, n, L);
+  __syncthreads();
+  for (int e = tid; e < n * n; e += kEigThreads) Vh[(e / n) * N + e % n] = Z[(e % n) * ldZ + e / n];
+  if (tid == 0) L.ok = 1;
+  __syncthreads();
+  if (wave < NB) {
+    double* d = L.vbuf[wave];
+    double* e = L.wbuf[wave];
+    bool good = true;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int i = lane + 64 * b;
+      d[i] = i < n ? L.d[i] * sc : 0.0;
+      e[i] = i + 1 < n ? L.e[i] * sc : 0.0;
+      good = good && isfinite(d[i]) && isfinite(e[i]);
+    }
+    good = __all(good);
+    const int row = 64 * wave + lane;
+    double* v = Vh + row;
+    int hi = n - 1, left = 40 * n;
+    while (good && hi > 0) {
+      // the last block [lo, hi] with no negligible entry inside
+      int lo = -1;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int i = lane + 64 * b;
+        const uint64_t small = __ballot(i < hi && fabs(e[i]) <= tol);
+        if (small) lo = 64 * b + 63 - __clzll((long long)small);
+      }
+      lo = __builtin_amdgcn_readfirstlane(lo) + 1;
+      if (lo == hi) {
+        --hi;
+        continue;
+      }
+      if (--left < 0) {
+        good = false;
+        break;
+      }
+      double a = d[lo], b = e[lo];
+      // the eigenvalue of the last 2 x 2 block nearer to its last entry
+      const double eh = e[hi - 1], dh = d[hi], half = 0.5 * (d[hi - 1] - dh);
+      const double mu = dh - eh * eh / (half + copysign(sqrt(fma(half, half, eh * eh)), half));
+      double x = a - mu, z = b;
+      double v0 = v[lo * N], v1 = v[(lo + 1) * N], f = d[lo + 1], en = e[lo + 1];
+      for (int k = lo; k < hi; ++k) {
+        // (the next entries, requested before this rotation's are written)
+        const int kn = min(k + 2, N - 1);
+        const double vn = v[kn * N], fn = d[kn], enn = e[kn];
+        const double r2 = fma(x, x, z * z);
+        double c = 1.0, s = 0.0, r = x;
+        if (r2 > 1e-290) {
+          const double inv = jac_rsqrt(r2);
+          c = x * inv;
+          s = z * inv;
+          r = r2 * inv;
+        }
+        if (k > lo) e[k - 1] = r;
+        const double w = fma(f - a, s, 2.0 * c * b), p = s * w;
+        d[k] = a + p;
+        a = f - p;
+        const double off = fma(c, w, -b);
+        v[k * N] = fma(c, v0, s * v1);
+        v0 = fma(c, v1, -s * v0);
+        x = off;
+        z = s * en;
+        b = k + 1 < hi ? c * en : off;
+        f = fn;
+        en = enn;
+        v1 = vn;
+      }
+      d[hi] = a;
+      e[hi - 1] = b;
+      v[hi * N] = v0;
+    }
+    if (!good && lane == 0) L.ok = 0;
+  }
+  __syncthreads();
+  if (!L.ok) return false;
+  const double* d = L.vbuf[0];
+  int* place = (int*)L.pbuf;
+  descending(d, n, place);
+  if (tid < n && place[tid] < ne) theta[place[tid]] = d[tid] / sc;
+  for (int q = tid; q < n * n; q += kEigThreads) {
+    const int i = q / n, row = q - i * n;
+    if (place[i] < ne) Z[row * ldZ + place[i]] = Vh[i * N + row];
+  }
+  __syncthreads();
+  return true;
+}
+
 // get(i, c): the matrix.  Vh: n x 64 NB (the reflectors, then the corrected
 // vectors), S: ldS >= round16(ne), round16(n) rows; Z: likewise, the vectors
 // on return (columns in descending order of theta).  theta: ne.
@@ -743,6 +866,45 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
         x[b][s][u] = rowok && c < n ? get(row, c) : 0.0;
       }
   if (rowok && lk == 0) L.col[row] = x[0][0][0];
+  // a matrix that is diagonal already, by the measure of the Jacobi sweeps, has
+  // its entries and unit vectors (n = 128: 590 us -> 28)
+  {
+    double off = 0.0, diag = 0.0;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const double sq = x[b][s][u] * x[b][s][u];
+          if (b * 64 + s * 16 + lk * 4 + u == row) {
+            diag += sq;
+            if (rowok) L.d[row] = x[b][s][u];
+          } else {
+            off += sq;
+          }
+        }
+    off = dpp_wave_sum(off);
+    diag = dpp_wave_sum(diag);
+    if (lane == 0) L.wbuf[0][2 * wave] = off, L.wbuf[0][2 * wave + 1] = diag;
+  }
+  __syncthreads();
+  {
+    double off = 0.0, diag = 0.0;
+    for (int w = 0; w < 4 * NB; ++w) off += L.wbuf[0][2 * w], diag += L.wbuf[0][2 * w + 1];
+    if (off <= 1e-30 * (off + diag)) {  // (the same for every thread)
+      int* place = (int*)L.pbuf;
+      for (int e = tid; e < n * ne; e += kEigThreads) Z[(e / ne) * ldZ + e % ne] = 0.0;
+      descending(L.d, n, place);
+      if (tid < n && place[tid] < ne) {
+        theta[place[tid]] = L.d[tid];
+        Z[tid * ldZ + place[tid]] = 1.0;
+      }
+      if (tid == 0) L.ok = 2;
+      __syncthreads();
+      return true;
+    }
+  }
   __syncthreads();
   double* vb = L.vbuf[wave];
   double* wb = L.wbuf[wave];
@@ -999,7 +1161,10 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
     Z[i * ldZ + c] = z;
   }
   __syncthreads();
-  if (!L.ok) return false;
+  if (!L.ok) {
+    __syncthreads();
+    return direct_qr<NB>(n, ne, tn, Vh, Z, ldZ, theta, L);
+  }
   direct_back<NB>(Vh, Z, ldZ, n, ne, L);
   __syncthreads();
   block_gemm_sym_f64(Z, ldZ, Z, ldZ, S, ldS, ne16, n16);
@@ -1012,7 +1177,10 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
   }
   if (!(worst <= 1e-8)) L.ok = 0;
   __syncthreads();
-  if (!L.ok) return false;
+  if (!L.ok) {
+    __syncthreads();
+    return direct_qr<NB>(n, ne, tn, Vh, Z, ldZ, theta, L);
+  }
   block_gemm_f64<false>(Z, ldZ, S, ldS, Vh, N, n16, ne16, ne16);
   for (int e = tid; e < n * ne; e += kEigThreads) {
     const int i = e / ne, c = e - i * ne;
@@ -1154,7 +1322,7 @@ __global__ __launch_bounds__(256) void eig_prep_kernel(EigBatch batch, int gtile
 }
 
 // The whole matrix, n <= CAP: the direct solver, and Jacobi sweeps where it
-// gives up.  CAP 64 keeps everything in LDS; CAP 128 keeps the reflectors (or
+// gives up (NaN, norms outside its range).  CAP 64 keeps everything in LDS; CAP 128 keeps the reflectors (or
 // the Jacobi's matrix) in LDS and the vectors in the workspace (a.W and a.Z,
 // ld 128).
 template <int CAP>
@@ -1178,7 +1346,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_small_kernel(EigBatch bat
     auto get = [=](int i, int c) { return 0.5 * (G[i * n + c] + G[c * n + i]); };
     if (direct_eig<CAP / 64>(get, n, a.k, LOCAL ? Vl : A, LOCAL ? A : a.Z, LOCAL ? LDA : CAP, W, LDW, theta, dl)) {
       eig_emit(a, W, LDW, nullptr, theta, sgn, 0);
-      if (tid == 0 && a.iters) *a.iters = 1;
+      if (tid == 0 && a.iters) *a.iters = dl.ok == 2 ? 0 : 1;
       return;
     }
     __syncthreads();

@@ -609,3 +609,56 @@ def test_mode_gram_rules(cuda, shape, dtype):
     bound = 2 * 2.3e-16 * u.shape[1] * (u.abs() @ u.abs().T)
     worst = float(((mode_gram(x, m) - u @ u.T).abs() - bound).max())
     assert worst <= 0
+
+
+def _sym_eig(a, k, cuda):
+    """(values, vectors, iterations) of tla_sym_eig."""
+    from tensorly_amd import _lib
+    L, n = _lib.lib(), a.shape[0]
+    G = torch.tensor(a, device=cuda)
+    w, v = torch.empty(k, device=cuda, dtype=torch.float64), torch.empty((n, k), device=cuda, dtype=torch.float64)
+    it = torch.zeros(1, dtype=torch.int32, device=cuda)
+    nb = L.tla_sym_eig_workspace_size(n)
+    ws = _lib.workspace(nb, G.device)
+    _lib.check(L.tla_sym_eig(_lib.ptr(G), n, k, None, 0, _lib.ptr(w), _lib.ptr(v), 1e-11, 300, _lib.ptr(it), _lib.ptr(ws),
+                             nb, _lib.stream(G.device)))
+    return w.cpu().numpy(), v.cpu().numpy(), int(it)
+
+
+@pytest.mark.parametrize("kind", ["clusters", "low rank", "blocks", "projector", "wilkinson"])
+@pytest.mark.parametrize("n", [4, 8, 17, 33, 48, 63, 64, 65, 90, 127, 128])
+def test_sym_eig_clusters_need_no_sweeps(cuda, kind, n):
+    """Clusters, where the vectors of the twisted factorisations cannot be told
+    apart, go through QR steps (one iteration; the sweeps report several).
+    Eigenvalues, residuals and orthonormality as above."""
+    import numpy as np
+    rng = np.random.default_rng(n)
+    if kind in ("clusters", "low rank"):
+        a = _spd(kind, n, rng)[0]
+    elif kind == "blocks":  # a tridiagonal form that falls apart
+        b = rng.standard_normal((n // 2, n // 2))
+        a = np.kron(np.eye(2), b @ b.T) if n % 2 == 0 else np.pad(np.kron(np.eye(2), b @ b.T), (0, 1))
+    elif kind == "projector":
+        q = np.linalg.qr(rng.standard_normal((n, n)))[0][:, : (n + 1) // 2]
+        a = q @ q.T
+    else:  # pairs of eigenvalues that agree to all digits
+        a = np.diag(np.abs(np.arange(n) - (n - 1) / 2.0)) + np.diag(np.ones(n - 1), 1) + np.diag(np.ones(n - 1), -1)
+    a = (a + a.T) / 2
+    lam = np.linalg.eigvalsh(a)[::-1]
+    for k in sorted({n // 2, n}):
+        w, v, it = _sym_eig(a, k, cuda)
+        tol = 1e-13 * n * np.abs(lam).max()
+        assert it <= 1  # (0: diagonal)
+        assert np.max(np.abs(w - lam[:k])) < tol
+        assert np.max(np.abs(a @ v - v * w)) < tol
+        assert np.max(np.abs(v.T @ v - np.eye(k))) < 1e-13 * n
+
+
+@pytest.mark.parametrize("n", [1, 2, 5, 48, 64, 65, 128])
+def test_sym_eig_of_a_diagonal_matrix_is_exact(cuda, n):
+    """Diagonal already: no rotations, no reflections."""
+    import numpy as np
+    d = np.random.default_rng(n).permutation(n) + 0.3
+    w, v, it = _sym_eig(np.diag(d), n, cuda)
+    assert it == 0 and np.array_equal(w, np.sort(d)[::-1])
+    assert np.array_equal(v, np.eye(n)[:, np.argsort(-d)])
