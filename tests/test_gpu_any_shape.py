@@ -14,6 +14,8 @@ import warnings
 import pytest
 import torch
 
+import any_shape_cases
+
 pytestmark = pytest.mark.gpu
 
 TOL = {torch.float32: 2e-6, torch.float64: 4e-15}
@@ -662,3 +664,51 @@ def test_sym_eig_of_a_diagonal_matrix_is_exact(cuda, n):
     w, v, it = _sym_eig(np.diag(d), n, cuda)
     assert it == 0 and np.array_equal(w, np.sort(d)[::-1])
     assert np.array_equal(v, np.eye(n)[:, np.argsort(-d)])
+
+
+def reference_in_blocks(X, w, F, mode):
+    """The reference with its sums taken 256 terms at a time and those added
+    up pairwise, so that its own rounding stays below the float64 kernels'."""
+    k = w.double()[None, :] if w is not None and len(F) > 2 else None
+    for m, f in enumerate(F):
+        if m != mode:
+            k = f.double() if k is None else (k[:, None, :] * f.double()[None, :, :]).reshape(-1, f.shape[1])
+    u = torch.movedim(X.double(), mode, 0).reshape(X.shape[mode], -1)
+    return torch.stack([u[:, q : q + 256] @ k[q : q + 256] for q in range(0, u.shape[1], 256)], -1).sum(-1)
+
+
+@pytest.mark.parametrize("case", any_shape_cases.MTTKRP, ids=lambda c: "%s-%s-%d-%d" % (("f32", "f64")[c[0]],
+                         "x".join(map(str, c[1])), c[2], c[3]))
+def test_mttkrp_any_shape_tiles_per_wave(cuda, case):
+    """Two and more tiles per wave, with their remainders of rows, columns,
+    rank columns and chunks.  Up to 32,000 terms, in chains of at most a
+    hundredth of them and then of the partial sums': tolerance as above."""
+    import tensorly_amd as tla
+    f64, shape, rank, mode, weights, _ = case
+    dtype = torch.float64 if f64 else torch.float32
+    X, F, w = problem(cuda, shape, rank, dtype, rank + mode)
+    w = w if weights else None
+    out = tla.unfolding_dot_khatri_rao(X, (w, F), mode)
+    ref = reference_in_blocks(X, w, F, mode)
+    err = torch.linalg.vector_norm(out.double() - ref, dim=1) / torch.linalg.vector_norm(ref, dim=1)
+    assert float(torch.linalg.vector_norm(out.double() - ref) / torch.linalg.vector_norm(ref)) < TOL[dtype]
+    assert float(err.max()) < 10 * TOL[dtype]  # (and no row far off: the edges of tiles)
+
+
+@pytest.mark.parametrize("case", any_shape_cases.MODE_DOT, ids=lambda c: "%s-%s-%d" % (("f32", "f64")[c[0]],
+                         "x".join(map(str, c[1])), c[3]))
+def test_mode_dot_any_shape_tiles_per_wave(cuda, case):
+    """Wide tiles of columns and rows, alone and shared by a block's waves.
+    Sums of at most 37 terms: tolerance as above."""
+    import tensorly_amd as tla
+    f64, shape, mode, J, _, _ = case
+    dtype = torch.float64 if f64 else torch.float32
+    g = torch.Generator(device=cuda).manual_seed(J)
+    X = torch.randn(shape, generator=g, device=cuda, dtype=dtype)
+    U = torch.randn((J, shape[mode]), generator=g, device=cuda, dtype=dtype)
+    out = tla.mode_dot(X, U, mode)
+    ref = torch.movedim(torch.movedim(X.double(), mode, -1) @ U.double().T.contiguous(), -1, mode)
+    err = (out.double() - ref).abs()
+    assert float(torch.linalg.vector_norm(err) / torch.linalg.vector_norm(ref)) < TOL[dtype]
+    scale = torch.movedim(torch.movedim(X.double().abs(), mode, -1) @ U.double().abs().T.contiguous(), -1, mode)
+    assert float((err / scale).max()) < TOL[dtype]  # (every element: the edges of tiles)

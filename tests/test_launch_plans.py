@@ -176,3 +176,23 @@ def test_mttkrp_of_little_work_keeps_the_vector_kernel(any_plan):
     matrix += [(0, (149, 120, 90), 10, m, 1) for m in range(3)] + [(0, (14, 27, 5, 5), 64, 2, 1), (1, (40, 50, 60), 70, 0, 1)]
     assert all(p["vector"] for p in any_plan(vector))
     assert not any(p["vector"] for p in any_plan(matrix))
+
+
+def test_the_shapes_of_the_gpu_tests_reach_every_tile_count(any_plan, ttm_plan):
+    from any_shape_cases import MODE_DOT, MTTKRP
+    plans = any_plan([(f, s, R, m, w) for f, s, R, m, w, _ in MTTKRP])
+    reached = set()
+    for (f, s, R, m, w, TN), p in zip(MTTKRP, plans):
+        assert p["ok"] and not p["vector"], (s, R, m)
+        assert TN is None or p["TN"] == TN, (s, R, m, p["TN"])
+        reached.add((f, p["last"], p["TN"]))
+    assert {(f, 0, t) for f in (False, True) for t in (2, 3, 4)} <= reached
+    assert {(f, 1, t) for f in (False, True) for t in (2, 3)} <= reached
+    rows = []
+    for f, s, m, J, _, _ in MODE_DOT:
+        before, after = 1, 1
+        for i, v in enumerate(s):
+            before, after = (before * v if i < m else before), (after * v if i > m else after)
+        rows.append((f, before, s[m], after, J))
+    for (f, s, m, J, TN, split), p in zip(MODE_DOT, ttm_plan(rows)):
+        assert p["ok"] and not p["vector"] and p["TN"] == TN and p["split"] == split, (s, m, J, p)
