@@ -406,10 +406,10 @@ static void any_run_rows(int TN, unsigned grid, const AnyRowsArgs<T>& a, hipStre
 template <typename T, int RT>
 static void any_run_last(int TN, unsigned grid, const AnyLastArgs<T>& a, hipStream_t st) {
   // (a slab of ranks past 64 may have fewer rank tiles than the plan's)
-  if constexpr (RT == 1)
+  if constexpr (RT == 1) {
     if (TN == 3) any_last_kernel<T, 3, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
-  if constexpr (RT <= 2)
     if (TN == 2) any_last_kernel<T, 2, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
+  }
   if (TN == 1 && a.ga.R) any_last_kernel<T, 1, RT, true><<<grid, 64 * kAnyWaves, 0, st>>>(a);
   else if (TN == 1) any_last_kernel<T, 1, RT><<<grid, 64 * kAnyWaves, 0, st>>>(a);
 }

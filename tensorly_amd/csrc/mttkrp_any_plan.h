@@ -101,7 +101,7 @@ inline bool any_plan(bool f64, int ndim, const int64_t* shape, int R, int mode, 
     p->g_rows = p->A / p->J;
     if (p->A > kBig || p->g_rows > kBig / (R * sz) || p->K > kBig / (32 * sz)) return false;
     tiles = (p->K + 16 * V - 1) / (16 * V);
-    most = p->RT == 1 ? 3 : p->RT == 2 ? 2 : 1;
+    most = p->RT == 1 ? 3 : 1;  // (two tiles of two rank tiles halve the waves: never less)
   } else {
     p->Pb = p->Q / p->K;
     if (p->Q > kBig / (32 * sz) || p->Pb > kBig / (R * sz)) return false;
