@@ -290,10 +290,10 @@ static GramPlan gram_plan(bool f64, int64_t Pa, int64_t In, int64_t Pb) {
   constexpr int64_t kBig = 0x7fffff00;
   // Runs of 17 to 24 columns leave a second piece that is mostly padding (300 rows,
   // float32, 17 / 20 / 24 columns: 42 / 39 / 36 us, short 34 / 32 / 33; from 25 on,
-  // float64 from 22, the pieces win).  Float64 rows that begin off the 16-byte grid: past some 90 MB
+  // float64 from 22, and for 64 rows the pieces win).  Float64 rows that begin off the 16-byte grid: past some 90 MB
   // the pieces' loads fetch too many lines twice (3000 x 4001 / 3 x 3000 x 2049:
   // 1118 / 2222 us, short 996 / 1568; 2048 x 4001: 543, short 594).
-  const bool padded = Pb >= 17 && Pb <= (f64 ? 21 : 24);
+  const bool padded = In >= 200 && Pb >= 17 && Pb <= (f64 ? 21 : 24);
   const bool astray = f64 && Pb % 2 != 0 && tiles >= 2048 && Q > (int64_t(90) << 20) / 8 / In;
   if (Pb == 1 && In >= 2 && In <= kBig / 64 && tiles <= 65535) p.kind = GramPlan::Last;
   else if (!padded && !astray && Pb >= 14 && Pb <= kBig / (33 * 8) && tiles <= 65535) p.kind = GramPlan::Rows;
@@ -309,11 +309,14 @@ static GramPlan gram_plan(bool f64, int64_t Pa, int64_t In, int64_t Pb) {
   // that many.  About two per CU, as each adds a partial tile to write and
   // sum (1000 x 1000: 36 us, with eight per CU 46), but eight where that
   // leaves a block 64 pieces, for an even finish (256^3 123-133 -> 107-114 us,
-  // 512^3 1.9 -> 1.5 ms), or three (what float64 keeps in flight; 3 x 600 x 2049:
-  // 90 -> 66 us, float32 76 -> 62).  At most 128: their sum is a serial chain.
+  // 512^3 1.9 -> 1.5 ms), or three (what float64 keeps in flight) where it leaves
+  // 60 (3 x 600 x 2049: 90 -> 66 us, float32 76 -> 62; with 48, 120 x 512 x 26: 50 ->
+  // 56), but in the contiguous mode (157 x 60 x 514 float64: 80 -> 90).  At most
+  // 128: their sum is a serial chain.
   const int64_t pieces = p.kind == GramPlan::Last ? (Q + 15) / 16 : Pa * ((Pb + 15) / 16);
   const int64_t nt1 = std::max<int64_t>(tiles, 1);
-  const int64_t blocks = pieces / 64 >= 2048 / nt1 ? 2048 : pieces / 48 >= 768 / nt1 ? 768 : 576;
+  const int64_t blocks = pieces / 64 >= 2048 / nt1 ? 2048
+                         : p.kind == GramPlan::Rows && pieces / 60 >= 768 / nt1 ? 768 : 576;
   int64_t s = std::min<int64_t>({(pieces + 7) / 8, std::max<int64_t>(1, blocks / nt1), 128});
   if (s > 8) s = s / 8 * 8;
   p.splits = (int)std::max<int64_t>(1, s);
