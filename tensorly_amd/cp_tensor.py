@@ -217,7 +217,10 @@ def cp_lstsq_grad(cp_tensor, tensor, return_loss=False, mask=None):
     # in place of two passes (512^3, rank 32: 219 -> 141 us, the call 426 ->
     # 318).  The block moves less than a pass where shape[2] >= 4 rank, and
     # below 2^24 entries the launches decide (128^3, rank 16: 128 us apart, 137
-    # shared).
+    # shared).  Apart / shared from there on: 256^3, ranks 2 to 16: 122 / 120-125
+    # us, rank 32: 137 / 124, rank 64: 227 / 199; 320^3, rank 2 / 16 / 64: 156 / 120,
+    # 163 / 129, 343 / 276; 64 x 64 x 4096, rank 2 / 64: 343 / 323, 1134 / 794.  The
+    # exception found: few outputs over a long mode, 4096 x 64 x 64 at rank 2: 123 / 167.
     shared = None
     if (dt == torch.float32 and tensor.dim() == 3 and 4 * rank <= tensor.shape[2] and tensor.numel() >= 1 << 24
             and all(f.device == tensor.device and f.shape == (s, rank) for f, s in zip(factors, tensor.shape))

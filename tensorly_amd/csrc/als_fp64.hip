@@ -70,13 +70,6 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const double* __restr
   if (threadIdx.x == 0) *out = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// D = A B + C, A 16 x 4, B 4 x 16 (FP64 MFMA): lane l supplies A[l % 16][l / 16]
-// and B[l / 16][l % 16] and holds D[l / 16 + 4 e][l % 16], e < 4 (rows
-// interleaved by 4, unlike the FP32 16x16x4 form).
-__device__ __forceinline__ doublex4 mfma_f64(double a, double b, doublex4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-
 // ---------------------------------------------------------------------------
 // Gram G = A^T A in FP64: blocks of kSolveRows rows give partial R x R
 // matrices (a 16 x 16 matrix tile per wave and step), summed in block order

@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "mma_any.h"
 
 namespace tla {
 
@@ -32,14 +33,6 @@ constexpr int kEigWaves = kEigThreads / 64;
 constexpr int kJac = 64;           // n <= kJac: Jacobi with A and W in LDS
 constexpr int kJacLarge = 128;     // n <= kJacLarge: Jacobi with A in LDS, W in the workspace
 constexpr int kEigCapLarge = 128;  // larger subspace block
-
-typedef double doublex4 __attribute__((ext_vector_type(4)));
-
-// D = A B + C on FP64 MFMA (16 x 4 by 4 x 16): lane l supplies A[l % 16][l / 16]
-// and B[l / 16][l % 16] and holds D[l / 16 + 4 e][l % 16], e < 4.
-__device__ __forceinline__ doublex4 mfma_f64(double a, double b, doublex4 c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
 
 // C (M x N, ldc) = op(A) B over K, op(A)[m][k] = TA ? A[k * lda + m] : A[m * lda + k],
 // B[k][n] = B[k * ldb + n]; M, N multiples of 16, K a multiple of 8.  The

@@ -7,6 +7,13 @@ namespace tla {
 
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
+// D = A B + C on FP64 MFMA (16 x 4 by 4 x 16): lane l supplies A[l % 16][l / 16]
+// and B[l / 16][l % 16] and holds D[l / 16 + 4 e][l % 16], e < 4 (rows
+// interleaved by 4, unlike the FP32 16x16x4 form).
+__device__ __forceinline__ doublex4 mfma_f64(double a, double b, doublex4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
 // Vector types of the tensor's loads: 16 bytes, aligned to one element.
 template <typename T> struct AnyT;
 template <> struct AnyT<float> {
@@ -23,7 +30,7 @@ template <> struct AnyT<double> {
   static constexpr int V = 2;
   static __device__ __forceinline__ int row(int g, int e) { return g + 4 * e; }
   static __device__ __forceinline__ acc mma(double a, double b, acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    return mfma_f64(a, b, c);
   }
 };
 

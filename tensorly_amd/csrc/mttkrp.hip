@@ -24,8 +24,10 @@
 //  * mttkrp_any_*    (mttkrp_any.hip) shapes that are not aligned, ranks above
 //    64 and float64, on the FP32 / FP64 matrix instructions.
 //
-//  * mttkrp_generic  plain vector ALU: precision "valu", sizes past the index
-//    ranges of mttkrp_any, and callers that bring no scratch.
+//  * mttkrp_generic  plain vector ALU: precision "valu", calls of little work
+//    (any_vector_wins), a contiguous output mode of 2 or 3 entries (float64:
+//    1; a 16-byte load is wider than the row), sizes past the index ranges of
+//    mttkrp_any, and callers that bring no scratch.
 //
 // Precisions: FP32 (v_mfma_f32_16x16x4_f32), BF16 (v_mfma_f32_16x16x32_bf16:
 // the tensor RNE-rounded to bf16, or a bf16 copy of it, times the factor
@@ -1369,7 +1371,7 @@ static int make_plan(int x_dtype, int ndim, const int64_t* shape, int R, int kb,
   // Shapes the aligned kernels below do not take, ranks above 64 and
   // float64: the matrix-core kernels for any shape (float32 arithmetic in
   // float32, whatever the precision asks for).  The vector kernel is left
-  // for precision "valu" and for sizes past those kernels' index ranges.
+  // for what the head of this file lists.
   auto unaligned = [&]() -> int {
     p->path = Path::Generic;
     p->ws_bytes = 0;

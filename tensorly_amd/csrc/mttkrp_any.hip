@@ -1,4 +1,5 @@
-// MTTKRP of any mode sizes on the matrix cores, float32 and float64.
+// MTTKRP of any mode sizes on the matrix cores, float32 and float64 (but for a
+// contiguous output mode shorter than a 16-byte load).
 //
 // The tensor is viewed as X[a, i, q] (i = output mode) and the output is
 // out[i, r] = sum_{a, q} X[a, i, q] B[(a, q), r], where B holds the rows of

@@ -10,8 +10,10 @@
 //                  (16-byte loads of 4 consecutive b per lane, 256 bytes per
 //                  row per wave) and the m-range split over the 4 waves of a
 //                  block, reduced in LDS in a fixed order.
-// ttm_any.hip holds the float32 and float64 kernels (any sizes); a vector-ALU
-// kernel is left for precision "valu".
+// ttm_any.hip holds the float32 and float64 kernels; a vector-ALU kernel is
+// left for precision "valu", sizes that would be mostly padding there
+// (ttm_vector_wins), contiguous runs of 2 or 3 entries in float32 (a 16-byte
+// load is wider than the run) and sizes past their index ranges or a launch.
 #include <algorithm>
 
 #include "common.h"
@@ -732,8 +734,8 @@ extern "C" int tla_mode_dot(int dtype, const void* X, int ndim, const int64_t* s
     if (precision == TLA_PREC_BF16) return launch_ttm_cols<TLA_PREC_BF16>(a, st);
     return launch_ttm_cols<TLA_PREC_BF16X3>(a, st);
   }
-  // everything else in the tensor's own arithmetic; precision "valu" and the
-  // sizes that the matrix kernels do not index stay on the vector ALU
+  // everything else in the tensor's own arithmetic, on the matrix cores but for
+  // what the head of this file lists
   TtmPlan plan;
   if ((dtype == TLA_F64 || precision != TLA_PREC_VALU) && ttm_any_plan(dtype == TLA_F64, Pa, Im, Pb, J, &plan) &&
       !plan.vector)

@@ -1,4 +1,5 @@
-// n-mode product of any mode sizes on the matrix cores, float32 and float64:
+// n-mode product on the matrix cores, float32 and float64, any mode sizes but
+// contiguous runs shorter than a 16-byte load:
 // out[a, j, b] = sum_m U'(j, m) X[a, m, b], U'(j, m) = U[j ldj + m ldm].
 //
 //  * ttm_any_cols_kernel (b not empty): U' is the first operand and 16-byte

@@ -16,7 +16,7 @@ from . import _lib
 from ._lib import check, lib, ptr, shape_array, stream, workspace
 
 __all__ = ["svd_flip", "svd_checks", "truncated_svd", "svd_interface", "make_svd_non_negative", "gram_eigh",
-           "gram_left_singular", "qr",
+           "gram_eigh_batch", "gram_left_singular", "qr",
            "mode_gram", "SVD_FUNS"]
 
 SVD_FUNS = ["truncated_svd", "symeig_svd"]
@@ -54,7 +54,8 @@ def gram_eigh(G, k, warm=None, tol=1e-11, max_iter=300):
 def gram_eigh_batch(Gs, ks, warms=None, tol=1e-11, max_iter=300):
     """:func:`gram_eigh` of independent Grams side by side: one launch per
     solver kind, one workgroup per Gram (``tla_sym_eig_batch``).  Returns a
-    list of ``(evals, evecs)``."""
+    list of ``(evals, evecs)``.  (The SVD inits call
+    :func:`leading_left_singular_vectors_batch`, which adds the signs.)"""
     out = []
     for c0 in range(0, len(Gs), 8):
         chunk = list(range(c0, min(len(Gs), c0 + 8)))

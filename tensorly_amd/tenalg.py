@@ -12,7 +12,7 @@ Inputs are torch tensors on the GPU (what tensorly's pytorch backend hands
 over); outputs are new tensors of the input dtype.  The arithmetic of the
 tensor contractions is chosen with :func:`set_precision` /
 :func:`precision` ("fp32" default, "bf16", "bf16x3", "valu"); float64
-inputs always run in FP64 on the vector ALU.
+inputs always run in FP64.
 
 :func:`register` adds the functions to tensorly's tenalg dispatcher when
 tensorly is importable (``tenalg/base_tenalg.py:4-33``,
