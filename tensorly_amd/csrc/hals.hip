@@ -142,7 +142,8 @@ __global__ __launch_bounds__(kHalsThreads) void hals_nnls_kernel(HalsArgs a) {
 // of the lane's E columns, some 8 ns each (57 ns at rank 16, 155 at rank 64).
 // 256 rows, rank 16, 100 iterations take 92 us and 96 us with the decision and
 // the last launch (one launch per iteration, a thread per row and a dot
-// product per update: 1362 us); 512 rows, rank 64: 992 us (16.2 ms).
+// product per update: 1362 us); 512 rows, rank 64: 1011 us in two chunks
+// (16.2 ms).
 constexpr int kHalsRows = 16;     // rows per workgroup of one wave
 constexpr int kHalsChunk = 128;   // iterations per launch, at most
 constexpr int kHalsBlocks = 65536;  // workgroups, at most: more rows take turns
@@ -401,11 +402,13 @@ __global__ __launch_bounds__(8 * kHalsChunk) void hals_decide_kernel(HalsRun h, 
   h.state[3] = first + 1;
 }
 
-// Chunks grow from 16 iterations where one iteration of all rows takes more than
-// some 4 us (by R^2 and the rounds of workgroups on the GPU): there a rule that
-// fires early would leave most of a long chunk for nothing.  20000 rows, rank
-// 64, firing at the second of 100 iterations: 502 us so, 2263 with one chunk
-// (862 with a launch per iteration); never firing: 2227 and 2165.
+// The first chunk has 16 iterations where one iteration of all rows takes more
+// than some 4 us (by R^2 and the rounds of workgroups on the GPU): there a rule
+// that fires early would leave most of a long chunk for nothing.  100
+// iterations, a rule that fires at the second / never, one chunk before: 512
+// rows, rank 64: 1036 -> 234 / 986 -> 1011 us; 20000 rows, rank 64: 2270 ->
+// 508 / 2171 -> 2209; 1M rows, rank 16: 5835 -> 1013 / 5706 -> 4618.  (Chunks
+// of 16, 64 and 20 took 1048 us for the 512 rows.)
 template <typename T, int RT, bool FULL, bool LOOP>
 static void hals_run(HalsRun h, int n_iter_max, hipStream_t st) {
   const bool heavy = (int64_t)RT * RT * std::max<int64_t>(1024, (h.a.rows + kHalsRows - 1) / kHalsRows) > 1700000;
@@ -414,7 +417,7 @@ static void hals_run(HalsRun h, int n_iter_max, hipStream_t st) {
   h.only = n_iter_max == 1;
   for (h.begin = 0; h.begin < n_iter_max && !h.only; h.begin += h.iters, ++h.chunk) {
     h.iters = std::min(chunk, n_iter_max - h.begin);
-    chunk = std::min(4 * chunk, kHalsChunk);
+    chunk = kHalsChunk;
     hals_run_kernel<T, RT, FULL, LOOP><<<(unsigned)h.nblk, 64, 0, st>>>(h);
     if (sum) hals_sum_kernel<<<kHalsSums, kHalsChunk, 0, st>>>(h);
     hals_decide_kernel<<<1, 8 * kHalsChunk, 0, st>>>(h, sum ? h.sums : h.partial, sum ? kHalsSums : h.nblk);

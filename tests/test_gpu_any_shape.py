@@ -571,8 +571,8 @@ def test_hals_from_a_start_far_above_the_solution(cuda, rows, rank, n_iter, tol)
                                                   (110_000, 16, 30, 1e-8), (1_100_003, 3, 20, 1e-8), (1_100_003, 3, 100, 0.5),
                                                   (33, 7, 1, 1e-8), (1_050_000, 1, 1, 0.5)])
 def test_hals_growing_chunks_and_many_rows(cuda, rows, rank, n_iter, tol):
-    """Chunks that grow from 8 iterations (long ones, and many rows), rules
-    that fire in one of them, more rows than workgroups, and single
+    """A first chunk of 16 iterations (long ones, and many rows), rules
+    that fire in a chunk, more rows than workgroups, and single
     iterations, against the oracle in FP64; tolerance as above."""
     import numpy as np
     from oracle import tensorly_np as T
