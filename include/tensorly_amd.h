@@ -255,8 +255,9 @@ int tla_cp_lstsq_grad_mode(int dtype, const void* factor, const void* mttkrp, vo
  * updated in place, in FP64 arithmetic; iters_out (device int, nullable)
  * receives the iterations run.  With a workspace (nullable) and
  * n_iter_max <= 1000 the rows run up to 128 iterations per launch over the
- * whole GPU (float32 factors are rounded at the end, not in between);
- * otherwise one workgroup runs the loop.  Arguments otherwise as tla_nn_mu_update.
+ * whole GPU, 16 in the first where an iteration is long (float32 factors are
+ * rounded at the end, not in between); otherwise one workgroup runs the loop.
+ * Arguments otherwise as tla_nn_mu_update.
  * ------------------------------------------------------------------- */
 size_t tla_hals_nnls_workspace_size(int64_t rows, int rank);
 int tla_hals_nnls(int dtype, void* factor, const void* mttkrp, int64_t rows, int rank,
@@ -356,8 +357,9 @@ int tla_admm_update(int dtype, void* factor, double* x_split, double* dual, cons
  *   tla_mode_gram64: G = unfold(X, mode) unfold(X, mode)^T (I_mode^2 FP64),
  *                    without forming the unfolding.
  *   tla_sym_eig:     k leading eigenpairs (descending) of symmetric FP64 G
- *                    (n x n).  n <= 128: the whole matrix (a direct solver, any
- *                    k <= n); n > 128: subspace iteration with Rayleigh-Ritz,
+ *                    (n x n).  n <= 128: the whole matrix (a direct solver, QR
+ *                    steps for clustered eigenvalues, any k <= n);
+ *                    n > 128: subspace iteration with Rayleigh-Ritz,
  *                    block 48 / 64 / 128 for k <= 40 / 56 / 120 (larger k
  *                    returns TLA_ERR_UNSUPPORTED), optional warm start Q0
  *                    (n x k0, its first columns used), converged when every
