@@ -357,8 +357,8 @@ int tla_admm_update(int dtype, void* factor, double* x_split, double* dual, cons
  *   tla_mode_gram64: G = unfold(X, mode) unfold(X, mode)^T (I_mode^2 FP64),
  *                    without forming the unfolding.
  *   tla_sym_eig:     k leading eigenpairs (descending) of symmetric FP64 G
- *                    (n x n).  n <= 128: the whole matrix (a direct solver, QR
- *                    steps for clustered eigenvalues, any k <= n);
+ *                    (n x n).  n <= 128: the whole matrix (a direct solver, or
+ *                    Jacobi sweeps for clustered eigenvalues, any k <= n);
  *                    n > 128: subspace iteration with Rayleigh-Ritz,
  *                    block 48 / 64 / 128 for k <= 40 / 56 / 120 (larger k
  *                    returns TLA_ERR_UNSUPPORTED), optional warm start Q0

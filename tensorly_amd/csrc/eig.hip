@@ -6,9 +6,9 @@
 // of its eigenvalues.
 //
 //  * n <= 128: tridiagonalisation, Sturm counts and twisted factorisations
-//    (direct_eig), or QR steps where eigenvalues cluster (direct_qr); outside
-//    their range cyclic Jacobi on the whole matrix (round-robin pair ordering,
-//    all n/2 rotations of a round applied in parallel).
+//    (direct_eig); where eigenvalues cluster, cyclic Jacobi on the whole
+//    matrix (round-robin pair ordering, all n/2 rotations of a round applied
+//    in parallel).
 //  * n  > 128: block subspace iteration with Rayleigh-Ritz, block b = 48 for
 //    k <= 40, 64 for k <= 56 or 128 for k <= 120.  Each step: Z = G V, H = V^T Z on FP64
 //    MFMA, H = W diag(t) W^T (perturbation theory where the previous Ritz
@@ -623,13 +623,16 @@ __device__ void sort_desc(const double* A, int m, int* order) {
 //  4. Back transformation, eight lanes per column.
 //  5. One Newton step towards orthonormal columns, Z <- Z (3 I - Z^T Z) / 2.
 //
-// When a residual exceeds 1e-13 of the norm or the vectors before step 5 are
-// not orthogonal to 1e-8 (clusters of eigenvalues, where the vectors of one are
-// not determined by their own value) direct_qr takes steps 2 to 5's place, from
-// the same reflectors.  Returns false, with nothing but scratch written, for
-// NaN and norms outside [1e-200, 1e150]: the caller then takes the Jacobi
-// sweeps.  The FP64 instructions that one workgroup issues bound it, most
-// of all in 1 (1.1 us a step up to 64 rows, 1.7 above).  Measured, one call:
+// Returns false, with nothing but scratch written, when two eigenvalues after
+// step 2 are within 1e-14 of the norm, a residual exceeds 1e-13 of it or the
+// vectors before step 5 are not orthogonal to 1e-8 (clusters of eigenvalues,
+// where the vectors of one are not determined by their own value), for NaN and
+// for norms outside [1e-200, 1e150]: the caller then takes the Jacobi sweeps,
+// which need no separation.  (Implicit QR steps from the same tridiagonal form
+// took a sixth of the sweeps' time, but give another basis of a null space, which
+// factors of more columns than the rank then show.)  The FP64 instructions that
+// one workgroup issues bound it, most of all in 1 (1.1 us a step up to 64 rows,
+// 1.7 above).  Measured, one call:
 // n = 120, k = 10: 317 us against 9.4 ms of Jacobi sweeps; n = 128, k = 128:
 // 605 us against 11.0 ms; n = 48, k = 10: 90 us against 825; a 48 x 48 Ritz
 // matrix: 103 us against 94 per sweep.
@@ -726,115 +729,6 @@ __device__ __forceinline__ void descending(const double* d, int n, int* place) {
     place[tid] = rank;
   }
   __syncthreads();
-}
-
-// All eigenpairs of the tridiagonal matrix in L.d, L.e by implicit QR steps
-// with Wilkinson's shift (Golub and Van Loan, Matrix Computations, 8.3), for
-// clusters whose vectors the twisted factorisations cannot tell apart: they
-// need no separation.  Each of NB waves holds 64 components of every vector and
-// runs the scalar recurrence for itself, so nothing waits for anything; the
-// chain of one rotation after another bounds it.  Off-diagonal entries are
-// dropped below 1.1e-16 of the norm.  Takes the reflectors in Vh and overwrites
-// them; leaves the ne leading pairs in Z and theta, or returns false after 40 n
-// steps (or for NaN).  Clusters of four, n = 128 / 64 / 16, with the attempt
-// before it: 2530 / 602 / 77 us; Jacobi sweeps instead of both 15.5 ms / 1989 / 167.
-template <int NB>
-__device__ bool direct_qr(int n, int ne, double norm, double* Vh, double* Z, int ldZ, double* theta,
-                                       DirectLds<NB>& L) {
-  constexpr int N = 64 * NB;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const double sc = ldexp(1.0, -ilogb(norm)), tol = 1.1e-16;
-  // the product of the reflectors, transposed into Vh
-  for (int e = tid; e < n * n; e += kEigThreads) Z[(e / n) * ldZ + e % n] = e / n == e % n ? 1.0 : 0.0;
-  __syncthreads();
-  direct_back<NB>(Vh, Z, ldZ, n, n, L);
-  __syncthreads();
-  for (int e = tid; e < n * n; e += kEigThreads) Vh[(e / n) * N + e % n] = Z[(e % n) * ldZ + e / n];
-  if (tid == 0) L.ok = 1;
-  __syncthreads();
-  if (wave < NB) {
-    double* d = L.vbuf[wave];
-    double* e = L.wbuf[wave];
-    bool good = true;
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int i = lane + 64 * b;
-      d[i] = i < n ? L.d[i] * sc : 0.0;
-      e[i] = i + 1 < n ? L.e[i] * sc : 0.0;
-      good = good && isfinite(d[i]) && isfinite(e[i]);
-    }
-    good = __all(good);
-    const int row = 64 * wave + lane;
-    double* v = Vh + row;
-    int hi = n - 1, left = 40 * n;
-    while (good && hi > 0) {
-      // the last block [lo, hi] with no negligible entry inside
-      int lo = -1;
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const int i = lane + 64 * b;
-        const uint64_t small = __ballot(i < hi && fabs(e[i]) <= tol);
-        if (small) lo = 64 * b + 63 - __clzll((long long)small);
-      }
-      lo = __builtin_amdgcn_readfirstlane(lo) + 1;
-      if (lo == hi) {
-        --hi;
-        continue;
-      }
-      if (--left < 0) {
-        good = false;
-        break;
-      }
-      double a = d[lo], b = e[lo];
-      // the eigenvalue of the last 2 x 2 block nearer to its last entry
-      const double eh = e[hi - 1], dh = d[hi], half = 0.5 * (d[hi - 1] - dh);
-      const double mu = dh - eh * eh / (half + copysign(sqrt(fma(half, half, eh * eh)), half));
-      double x = a - mu, z = b;
-      double v0 = v[lo * N], v1 = v[(lo + 1) * N], f = d[lo + 1], en = e[lo + 1];
-      for (int k = lo; k < hi; ++k) {
-        // (the next entries, requested before this rotation's are written)
-        const int kn = min(k + 2, N - 1);
-        const double vn = v[kn * N], fn = d[kn], enn = e[kn];
-        const double r2 = fma(x, x, z * z);
-        double c = 1.0, s = 0.0, r = x;
-        if (r2 > 1e-290) {
-          const double inv = jac_rsqrt(r2);
-          c = x * inv;
-          s = z * inv;
-          r = r2 * inv;
-        }
-        if (k > lo) e[k - 1] = r;
-        const double w = fma(f - a, s, 2.0 * c * b), p = s * w;
-        d[k] = a + p;
-        a = f - p;
-        const double off = fma(c, w, -b);
-        v[k * N] = fma(c, v0, s * v1);
-        v0 = fma(c, v1, -s * v0);
-        x = off;
-        z = s * en;
-        b = k + 1 < hi ? c * en : off;
-        f = fn;
-        en = enn;
-        v1 = vn;
-      }
-      d[hi] = a;
-      e[hi - 1] = b;
-      v[hi * N] = v0;
-    }
-    if (!good && lane == 0) L.ok = 0;
-  }
-  __syncthreads();
-  if (!L.ok) return false;
-  const double* d = L.vbuf[0];
-  int* place = (int*)L.pbuf;
-  descending(d, n, place);
-  if (tid < n && place[tid] < ne) theta[place[tid]] = d[tid] / sc;
-  for (int q = tid; q < n * n; q += kEigThreads) {
-    const int i = q / n, row = q - i * n;
-    if (place[i] < ne) Z[row * ldZ + place[i]] = Vh[i * N + row];
-  }
-  __syncthreads();
-  return true;
 }
 
 // get(i, c): the matrix.  Vh: n x 64 NB (the reflectors, then the corrected
@@ -1076,6 +970,12 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
       __syncthreads();
     }
   }
+  // eigenvalues this close give one vector twice, orthogonal to 1e-2 at best:
+  // what follows would be in vain (n = 128, clusters of four: 0.39 ms before the
+  // sweeps' 15.4, 0.63 with the whole attempt; n = 16: 26 and 31 us before 192)
+  if (tid + 1 < ne && lo[tid] + hi[tid] - (lo[tid + 1] + hi[tid + 1]) < 2e-14 * tn) L.ok = 0;
+  __syncthreads();
+  if (!L.ok) return false;
   // twisted factorisations: thread r from the top, thread 256 + r from the bottom
   const int r = tid & 255;
   const bool down = tid < 256, on = r < ne;
@@ -1154,10 +1054,7 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
     Z[i * ldZ + c] = z;
   }
   __syncthreads();
-  if (!L.ok) {
-    __syncthreads();
-    return direct_qr<NB>(n, ne, tn, Vh, Z, ldZ, theta, L);
-  }
+  if (!L.ok) return false;
   direct_back<NB>(Vh, Z, ldZ, n, ne, L);
   __syncthreads();
   block_gemm_sym_f64(Z, ldZ, Z, ldZ, S, ldS, ne16, n16);
@@ -1170,10 +1067,7 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
   }
   if (!(worst <= 1e-8)) L.ok = 0;
   __syncthreads();
-  if (!L.ok) {
-    __syncthreads();
-    return direct_qr<NB>(n, ne, tn, Vh, Z, ldZ, theta, L);
-  }
+  if (!L.ok) return false;
   block_gemm_f64<false>(Z, ldZ, S, ldS, Vh, N, n16, ne16, ne16);
   for (int e = tid; e < n * ne; e += kEigThreads) {
     const int i = e / ne, c = e - i * ne;
@@ -1315,7 +1209,7 @@ __global__ __launch_bounds__(256) void eig_prep_kernel(EigBatch batch, int gtile
 }
 
 // The whole matrix, n <= CAP: the direct solver, and Jacobi sweeps where it
-// gives up (NaN, norms outside its range).  CAP 64 keeps everything in LDS; CAP 128 keeps the reflectors (or
+// gives up.  CAP 64 keeps everything in LDS; CAP 128 keeps the reflectors (or
 // the Jacobi's matrix) in LDS and the vectors in the workspace (a.W and a.Z,
 // ld 128).
 template <int CAP>

@@ -629,10 +629,9 @@ def _sym_eig(a, k, cuda):
 
 @pytest.mark.parametrize("kind", ["clusters", "low rank", "blocks", "projector", "wilkinson"])
 @pytest.mark.parametrize("n", [4, 8, 17, 33, 48, 63, 64, 65, 90, 127, 128])
-def test_sym_eig_clusters_need_no_sweeps(cuda, kind, n):
+def test_sym_eig_clusters(cuda, kind, n):
     """Clusters, where the vectors of the twisted factorisations cannot be told
-    apart, go through QR steps (one iteration; the sweeps report several).
-    Eigenvalues, residuals and orthonormality as above."""
+    apart.  Eigenvalues, residuals and orthonormality as above."""
     import numpy as np
     rng = np.random.default_rng(n)
     if kind in ("clusters", "low rank"):
@@ -648,9 +647,8 @@ def test_sym_eig_clusters_need_no_sweeps(cuda, kind, n):
     a = (a + a.T) / 2
     lam = np.linalg.eigvalsh(a)[::-1]
     for k in sorted({n // 2, n}):
-        w, v, it = _sym_eig(a, k, cuda)
+        w, v, _ = _sym_eig(a, k, cuda)
         tol = 1e-13 * n * np.abs(lam).max()
-        assert it <= 1  # (0: diagonal)
         assert np.max(np.abs(w - lam[:k])) < tol
         assert np.max(np.abs(a @ v - v * w)) < tol
         assert np.max(np.abs(v.T @ v - np.eye(k))) < 1e-13 * n
