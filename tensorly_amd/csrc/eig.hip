@@ -733,8 +733,11 @@ __device__ __forceinline__ void descending(const double* d, int n, int* place) {
 
 // get(i, c): the matrix.  Vh: n x 64 NB (the reflectors, then the corrected
 // vectors), S: ldS >= round16(ne), round16(n) rows; Z: likewise, the vectors
-// on return (columns in descending order of theta).  theta: ne.
-template <int NB, typename Get>
+// on return (columns in descending order of theta).  theta: ne.  WHOLE: a matrix
+// of the caller's; diagonal ones and clusters are seen early.  (A Ritz matrix is
+// next to diagonal as a rule, its null space in no order, and graded: vectors
+// of eigenvalues close to one another may hold all the same.)
+template <int NB, bool WHOLE, typename Get>
 __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ldS, double* Z, int ldZ, double* theta,
                            DirectLds<NB>& L) {
   constexpr int N = 64 * NB;
@@ -755,7 +758,7 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
   if (rowok && lk == 0) L.col[row] = x[0][0][0];
   // a matrix that is diagonal already, by the measure of the Jacobi sweeps, has
   // its entries and unit vectors (n = 128: 590 us -> 28)
-  {
+  if constexpr (WHOLE) {
     double off = 0.0, diag = 0.0;
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -774,10 +777,8 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
     off = dpp_wave_sum(off);
     diag = dpp_wave_sum(diag);
     if (lane == 0) L.wbuf[0][2 * wave] = off, L.wbuf[0][2 * wave + 1] = diag;
-  }
-  __syncthreads();
-  {
-    double off = 0.0, diag = 0.0;
+    __syncthreads();
+    off = 0.0, diag = 0.0;
     for (int w = 0; w < 4 * NB; ++w) off += L.wbuf[0][2 * w], diag += L.wbuf[0][2 * w + 1];
     if (off <= 1e-30 * (off + diag)) {  // (the same for every thread)
       int* place = (int*)L.pbuf;
@@ -973,9 +974,11 @@ __device__ bool direct_eig(Get get, int n, int ne, double* Vh, double* S, int ld
   // eigenvalues this close give one vector twice, orthogonal to 1e-2 at best:
   // what follows would be in vain (n = 128, clusters of four: 0.39 ms before the
   // sweeps' 15.4, 0.63 with the whole attempt; n = 16: 26 and 31 us before 192)
-  if (tid + 1 < ne && lo[tid] + hi[tid] - (lo[tid + 1] + hi[tid + 1]) < 2e-14 * tn) L.ok = 0;
-  __syncthreads();
-  if (!L.ok) return false;
+  if constexpr (WHOLE) {
+    if (tid + 1 < ne && lo[tid] + hi[tid] - (lo[tid + 1] + hi[tid + 1]) < 2e-14 * tn) L.ok = 0;
+    __syncthreads();
+    if (!L.ok) return false;
+  }
   // twisted factorisations: thread r from the top, thread 256 + r from the bottom
   const int r = tid & 255;
   const bool down = tid < 256, on = r < ne;
@@ -1231,7 +1234,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_small_kernel(EigBatch bat
   {
     const double* G = a.G;
     auto get = [=](int i, int c) { return 0.5 * (G[i * n + c] + G[c * n + i]); };
-    if (direct_eig<CAP / 64>(get, n, a.k, LOCAL ? Vl : A, LOCAL ? A : a.Z, LOCAL ? LDA : CAP, W, LDW, theta, dl)) {
+    if (direct_eig<CAP / 64, true>(get, n, a.k, LOCAL ? Vl : A, LOCAL ? A : a.Z, LOCAL ? LDA : CAP, W, LDW, theta, dl)) {
       eig_emit(a, W, LDW, nullptr, theta, sgn, 0);
       if (tid == 0 && a.iters) *a.iters = dl.ok == 2 ? 0 : 1;
       return;
@@ -1539,7 +1542,7 @@ __global__ __launch_bounds__(kEigThreads) void sym_eig_subspace_kernel(EigBatch 
       if constexpr (B == 48) {
         // (a separated leading block of few columns sweeps in less)
         if (pert == 0 && (!sep || k >= 24)) {
-          direct = direct_eig<1>([=](int i, int c) { return H[i * LDH + c]; }, B, B, stage, stage + B * 64, B, W, LDW,
+          direct = direct_eig<1, false>([=](int i, int c) { return H[i * LDH + c]; }, B, B, stage, stage + B * 64, B, W, LDW,
                                  theta, dl);
           if (!direct) {
             __syncthreads();
